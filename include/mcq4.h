@@ -144,11 +144,16 @@ int mcq4_matmul_q4_0_f16_grouped(const void *X, int64_t ldx, int count, const ui
  * MCQ4_DTYPE_BF16 / F32 follow the reference's path for those dtypes
  * (quantization.py:452-454): W dequantized to x_dtype (one rounding of the
  * exact product), Y = X @ W with fp32 accumulation, Y in x_dtype.  X and Y
- * aligned to x_dtype; no workspace is needed for them (may be NULL).
+ * aligned to x_dtype; the workspace is optional for them (NULL, or smaller than
+ * mcq4_matmul_q4_0_workspace_bytes: K is then not split over workgroups).
  */
 int mcq4_matmul_q4_0(const void *X, int x_dtype, int64_t ldx, const uint8_t *W, void *Y,
                      int64_t ldy, int64_t M, int64_t K, int64_t N, void *workspace,
                      size_t workspace_bytes, void *stream);
+
+/* Workspace bytes mcq4_matmul_q4_0 makes use of for this shape and x_dtype (for
+ * MCQ4_DTYPE_F16 mcq4_matmul_workspace_bytes); same conventions. */
+size_t mcq4_matmul_q4_0_workspace_bytes(int64_t M, int64_t K, int64_t N, int x_dtype);
 
 /*
  * Re-zeroes the counter area (the first 256 KiB) of a split-K workspace with a
@@ -265,7 +270,7 @@ size_t mcq4_matmul_int8_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t
 /* Y[M][ldy] = X[M][ldx] @ dequant(W), fp32 accumulation, X and Y in x_dtype.
  * fp16 activations with group_size % 16 == 0, K % 16 == 0 and N % 8 == 0 run
  * the MFMA GEMV (M <= 16); K and group_size % 32 == 0 with N % 128 == 0 the
- * MFMA GEMM; everything else the general fp32 kernel. */
+ * MFMA GEMM; everything else as in mcq4_matmul_int4. */
 int mcq4_matmul_int8(const void *X, int x_dtype, int64_t ldx, const int8_t *W, const void *scales,
                      const void *zeros, int sz_dtype, void *Y, int64_t ldy, int64_t M, int64_t K,
                      int64_t N, int64_t group_size, void *workspace, size_t workspace_bytes,

@@ -16,6 +16,7 @@
 
 #include "../../include/mcq4.h"
 #include "q4_prefill.h"
+#include "wx_common.h"
 
 namespace mcq4 {
 hipError_t launch_quantize(bool llama_rule, const float *W, int64_t ldw, int nb, int N,
@@ -45,8 +46,6 @@ hipError_t i4_gemv1_split_fallbacks(uint64_t *count, bool reset);
 hipError_t i4_gemm6_split_fallbacks(uint64_t *count, bool reset);
 hipError_t q4_gemv_span_split_fallbacks(uint64_t *count, bool reset);
 hipError_t q4_gemm8_split_fallbacks(uint64_t *count, bool reset);
-hipError_t launch_q4_xact(const void *X, int x_dt, int64_t ldx, const uint8_t *W, void *Y,
-                          int64_t ldy, int64_t M, int64_t K, int64_t N, hipStream_t s);
 bool gemv_dma_supported(const _Float16 *X, const uint8_t *W, int64_t K, int64_t N);
 hipError_t launch_gemv_dma_group(const _Float16 *X, const uint8_t *const *W, _Float16 *const *Y, int count,
                                  int K, int N, int *n_done, hipStream_t s);
@@ -260,6 +259,12 @@ size_t mcq4_matmul_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     return M <= 64 ? std::max(pre, mcq4::skinny_workspace_bytes(M, K, N)) : pre;
 }
 
+size_t mcq4_matmul_q4_0_workspace_bytes(int64_t M, int64_t K, int64_t N, int x_dtype) {
+    if (x_dtype == MCQ4_DTYPE_F16) return mcq4_matmul_workspace_bytes(M, K, N);
+    if (M <= 0 || K <= 0 || N <= 0 || K % 32) return 0;
+    return mcq4::wx_workspace_bytes(mcq4::WX_Q4, x_dtype, M, K, N);
+}
+
 int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, int64_t ldy,
                          int64_t M, int64_t K, int64_t N, void *workspace,
                          size_t workspace_bytes, void *stream) {
@@ -349,9 +354,9 @@ int mcq4_matmul_q4_0(const void *X, int x_dtype, int64_t ldx, const uint8_t *W, 
     if (!aligned(X, al) || !aligned(Y, al))
         return fail(MCQ4_ERR_ALIGNMENT, "X and Y must be aligned to their dtype");
     if (!aligned(W, 2)) return fail(MCQ4_ERR_ALIGNMENT, "W must be 2-byte aligned");
-    (void)workspace; (void)workspace_bytes;
-    return hip_status(mcq4::launch_q4_xact(X, x_dtype, ldx, W, Y, ldy, M, K, N, (hipStream_t)stream),
-                      "matmul launch");
+    if (workspace && !aligned(workspace, 16)) workspace = nullptr;   // optional here: K stays whole
+    const mcq4::WxCall c = {mcq4::WX_Q4, x_dtype, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32};
+    return hip_status(mcq4::launch_wx(c, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
 }
 
 int mcq4_reset_workspace(void *workspace, size_t workspace_bytes, void *stream) {

@@ -17,6 +17,7 @@
 
 #include "../../include/mcq4.h"
 #include "mcq4_options.h"
+#include "wx_common.h"
 
 namespace mcq4 {
 hipError_t launch_i4_quantize(const void *W, int w_dt, int64_t ldw, int64_t K, int64_t N,
@@ -112,6 +113,15 @@ size_t ws_bytes(int64_t M, int64_t K, int64_t N, int64_t gs, int x_dt, int wb = 
     return mcq4::i4_gemm_workspace_bytes(M, K, N);
 }
 
+// What the entry points make use of: the MFMA kernels' required workspace, or
+// the optional one of the kernels for other dtypes and shapes.
+size_t query_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t gs, int x_dt, int wb = 4) {
+    const size_t need = ws_bytes(M, K, N, gs, x_dt, wb);
+    if (M <= 0 || K <= 0 || N <= 0 || gs <= 0 || gs % 32) return need;
+    if (x_dt == MCQ4_DTYPE_F16 && N % 128 == 0 && K % 32 == 0) return need;
+    return std::max(need, mcq4::wx_workspace_bytes(wb == 4 ? mcq4::WX_I4 : mcq4::WX_I8, x_dt, M, K, N));
+}
+
 int matmul_common(int act, const void *X, int x_dtype, int64_t ldx, const uint8_t *packed,
                   const void *scales, const void *zeros, int sz_dtype, void *Y, int64_t ldy,
                   int64_t M, int64_t K, int64_t N, int64_t gs, void *workspace,
@@ -135,6 +145,12 @@ int matmul_common(int act, const void *X, int x_dtype, int64_t ldx, const uint8_
         return fail(MCQ4_ERR_ALIGNMENT, "scales and zeros must be aligned to their element size");
     I4Path path = i4_path(X, x_dtype, ldx, packed, scales, zeros, Y, ldy, M, K, N, gs, wb);
     if (path == I4Path::Gemm && (K % 32 || gs % 32)) path = I4Path::Generic;
+    const mcq4::WxCall wx = {wb == 4 ? mcq4::WX_I4 : mcq4::WX_I8, x_dtype, sz_dtype, act, X, ldx, packed, scales, zeros,
+                             Y, ldy, M, K, N, gs};
+    if (path == I4Path::Generic && !mcq4::opt_is("MCQ4_I4_PATH", 'g') && mcq4::wx_supported(wx)) {
+        if (workspace && !aligned(workspace, 16)) workspace = nullptr;   // optional here: K stays whole
+        return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, (hipStream_t)stream), "int4 matmul launch");
+    }
     const size_t need = path == I4Path::Generic ? 0 : ws_bytes(M, K, N, gs, x_dtype, wb);
     if (need && (!workspace || workspace_bytes < need))
         return fail(MCQ4_ERR_WORKSPACE, "workspace of %zu bytes required, %zu given", need,
@@ -200,7 +216,7 @@ int mcq4_quantize_to_int4(const float *W, int64_t ldw, int64_t K, int64_t N, int
 
 size_t mcq4_matmul_int8_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size,
                                         int x_dtype) {
-    return ws_bytes(M, K, N, group_size, x_dtype, 8);
+    return query_ws_bytes(M, K, N, group_size, x_dtype, 8);
 }
 
 int mcq4_matmul_int8(const void *X, int x_dtype, int64_t ldx, const int8_t *W, const void *scales,
@@ -231,7 +247,7 @@ int mcq4_dequantize_int4(const uint8_t *packed, const void *scales, const void *
 
 size_t mcq4_matmul_int4_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size,
                                         int x_dtype) {
-    return ws_bytes(M, K, N, group_size, x_dtype);
+    return query_ws_bytes(M, K, N, group_size, x_dtype);
 }
 
 int mcq4_matmul_int4(const void *X, int x_dtype, int64_t ldx, const uint8_t *packed,
@@ -267,7 +283,7 @@ int mcq4_matmul_int4_gelu(const void *X, int x_dtype, int64_t ldx, const uint8_t
 // activations and one zero-filled buffer keeps serving every entry point.
 constexpr size_t kCounterArea = (size_t)65536 * 4;
 static size_t norm_offset(int64_t M, int64_t K, int64_t N, int64_t gs) {
-    const size_t w = std::max(ws_bytes(M, K, N, gs, MCQ4_DTYPE_F16), kCounterArea);
+    const size_t w = std::max(query_ws_bytes(M, K, N, gs, MCQ4_DTYPE_F16), kCounterArea);
     return (w + 255) / 256 * 256;
 }
 

@@ -1,0 +1,291 @@
+// Shared parts of the any-activation matmul kernels (wx_gemm, wx_skinny):
+// quantized weights (block_q4_0, per-group INT4, per-group INT8) times fp16, bf16
+// or fp32 activations, any column count, any 2-byte (q4_0) or byte (INT4, INT8)
+// alignment of the weights.
+//
+// Semantics (quantization.py:207-239, :268-286, :452-454): the weight is
+// dequantized in fp32 and rounded once to the activations' dtype, then
+// Y = X @ W with fp32 sums and one rounding to the activations' dtype.
+//
+// Lane layout of a K step of 32 (MFMA 32x32): lane l supplies column (or row)
+// l % 32 and the 16 K elements 16 (l / 32) .. +15 of the step.  The MFMA K order
+// is a permutation of the real one, the same for both operands, so a lane's
+// weights are contiguous: 8 nibble bytes of a q4_0 block, 8 byte rows of INT4,
+// 16 of INT8.
+#pragma once
+
+#include "i4_common.h"
+
+namespace mcq4 {
+
+enum : int { WX_Q4 = 0, WX_I4 = 1, WX_I8 = 2 };
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
+
+struct WxArgs {
+    const void *X;
+    int64_t ldx;
+    const uint8_t *W;            // q4_0 blocks, packed INT4 or int8 rows
+    const void *scales, *zeros;  // INT4, INT8
+    int sz_dt;
+    void *Y;
+    int64_t ldy;
+    int M, K, N;
+    int spg;                     // K steps of 32 per group (INT4, INT8)
+    int act;                     // ACT_*
+    int S;                       // K splits (grid.z)
+    float *part;                 // [S][M][ldp] fp32 partials when S > 1
+    int ldp;
+    int tiles_m, tiles_n;
+};
+
+// Unaligned loads: gfx950 global loads need no alignment beyond the byte.
+template <typename T>
+__device__ __forceinline__ T load_u(const void *p) {
+    T v;
+    __builtin_memcpy(&v, p, sizeof(T));
+    return v;
+}
+
+__device__ __forceinline__ float ubyte_f32(uint32_t v, int b) { return (float)((v >> (8 * b)) & 0xFFu); }
+
+// Two fp32 values rounded (nearest even) to a pair of 16-bit activations' dtype.
+template <int XT>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+    if constexpr (XT == DT_BF16) {
+        return bitcast<uint32_t>(__builtin_convertvector((float2_t{a, b}), bf16x2_t));
+    } else {
+        return bitcast<uint32_t>(half2_t{(_Float16)a, (_Float16)b});
+    }
+}
+
+// What a lane loads of the weights for one K step and TN column tiles.
+template <int WT, int TN>
+struct WxRaw;
+template <int TN>
+struct WxRaw<WX_Q4, TN> {
+    uint32_t q[TN][2];
+    uint16_t d[TN];
+};
+template <int TN>
+struct WxRaw<WX_I4, TN> {
+    uint32_t q[8];               // byte rows, TN columns each
+    uint32_t s[TN], z[TN];       // raw scale and zero (16 or 32 bits)
+};
+template <int TN>
+struct WxRaw<WX_I8, TN> {
+    uint32_t q[16];
+    uint32_t s[TN], z[TN];
+};
+
+// The lane's place in the weights: its columns and the address of K step 0.
+// q4_0: tile j's column is n0 + 32 j + l % 32.  INT4 and INT8: n0 + TN (l % 32) + j, so one
+// load of a byte row serves every tile.  Lanes past N take the last columns
+// again (the same values; what they store there is identical).
+template <int WT, int TN>
+struct WxLane {
+    int n[TN];
+    int n0;                               // the workgroup-uniform column the offsets count from
+    uint32_t off[WT == WX_Q4 ? TN : 1];   // byte offset in the step's rows
+};
+template <int WT, int TN>
+__device__ __forceinline__ WxLane<WT, TN> wx_lane(const WxArgs &a, int n0, int lane) {
+    WxLane<WT, TN> L;
+    const int c = lane & 31, hi = lane >> 5;
+    if constexpr (WT == WX_Q4) {
+        L.n0 = min(n0, a.N - 1);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            L.n[j] = min(n0 + 32 * j + c, a.N - 1);
+            L.off[j] = (uint32_t)(L.n[j] - L.n0) * BLOCK_BYTES;
+        }
+    } else {
+        L.n0 = min(n0, a.N - TN);
+        const int nb = min(n0 + TN * c, a.N - TN);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) L.n[j] = nb + j;
+        L.off[0] = (uint32_t)hi * (WT == WX_I4 ? 8u : 16u) * (uint32_t)a.N + (uint32_t)(nb - L.n0);
+    }
+    return L;
+}
+
+template <int TN>
+__device__ __forceinline__ void wx_load_sz(const void *p, int64_t row, int dt, int n, uint32_t (&out)[TN]) {
+    if (dt == DT_F32) {
+        const float *q = (const float *)p + row;
+        if constexpr (TN == 2) {
+            const u32x2 v = load_u<u32x2>(q + n);
+            out[0] = v[0]; out[1] = v[1];
+        } else {
+            const uint4_t v = load_u<uint4_t>(q + n);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) out[j] = v[j];
+        }
+    } else {
+        const uint16_t *q = (const uint16_t *)p + row;
+        if constexpr (TN == 2) {
+            const uint32_t v = load_u<uint32_t>(q + n);
+            out[0] = v & 0xFFFFu; out[1] = v >> 16;
+        } else {
+            const u32x2 v = load_u<u32x2>(q + n);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) out[j] = (v[j / 2] >> (16 * (j & 1))) & 0xFFFFu;
+        }
+    }
+}
+
+// Loads K step `kb` (group `grp`).  TAIL: rows past K are clamped to the last
+// one (wx_dequant zeroes their weights).
+template <int WT, int TN, bool TAIL>
+__device__ __forceinline__ void wx_load(WxRaw<WT, TN> &r, const WxArgs &a, const WxLane<WT, TN> &L, int kb, int grp,
+                                        int lane) {
+    if constexpr (WT == WX_Q4) {
+        const uint8_t *base = a.W + ((int64_t)kb * a.N + L.n0) * BLOCK_BYTES;
+        const int hi = lane >> 5;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const uint8_t *p = base + L.off[j];
+            r.d[j] = load_u<uint16_t>(p);
+            const u32x2 v = load_u<u32x2>(p + 2 + 8 * hi);
+            r.q[j][0] = v[0]; r.q[j][1] = v[1];
+        }
+    } else {
+        constexpr int ROWS = WT == WX_I4 ? 8 : 16;
+        const uint8_t *base = a.W + (int64_t)kb * (2 * ROWS) * a.N + L.n0;
+        const int last = (WT == WX_I4 ? a.K / 2 : a.K) - 1 - kb * 2 * ROWS;   // last valid row of the step
+        const int hi = lane >> 5;
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            const uint8_t *p;
+            if constexpr (TAIL) p = base + (int64_t)min(hi * ROWS + i, last) * a.N + (L.off[0] - (uint32_t)hi * ROWS * (uint32_t)a.N);
+            else p = base + (int64_t)i * a.N + L.off[0];
+            if constexpr (TN == 2) r.q[i] = load_u<uint16_t>(p);
+            else r.q[i] = load_u<uint32_t>(p);
+        }
+        const int64_t row = (int64_t)grp * a.N;
+        wx_load_sz<TN>(a.scales, row, a.sz_dt, L.n[0], r.s);
+        wx_load_sz<TN>(a.zeros, row, a.sz_dt, L.n[0], r.z);
+    }
+}
+
+__device__ __forceinline__ float wx_sz_f32(uint32_t v, int dt) {
+    if (dt == DT_F32) return __uint_as_float(v);
+    if (dt == DT_F16) return (float)bitcast<_Float16>((uint16_t)v);
+    return bf16_bits_to_f32((uint16_t)v);
+}
+
+// The lane's 16 weights of tile j in fp32, in K order.
+// q4_0: v_perm_b32 puts a nibble byte into bytes 0 and 2 and v_and_or_b32 makes
+// it the fp16 pair {1024 + q0, 64 + q1}; minus {1032, 72} gives q - 8, and one
+// mixed-precision multiply each (q - 8) d, exact in fp32 (d has 11 significant
+// bits).  INT4 and INT8: (q - z) s in the reference's two fp32 roundings.
+// TAIL: weights of rows past K are zero (`valid` = rows of the lane's 16 below K).
+template <int WT, int XT, int TN, bool TAIL>
+__device__ __forceinline__ void wx_values(const WxRaw<WT, TN> &r, int j, int sz_dt, int valid, float (&w)[16]) {
+    if constexpr (WT == WX_Q4) {
+        const uint32_t nib_mask = opaque_sgpr(0x00F0000Fu), exp_bits = opaque_vgpr(0x54006400u);
+        const float d = (float)bitcast<_Float16>(r.d[j]);
+        const half2_t off = {(_Float16)1032.0f, (_Float16)72.0f};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const half2_t p = bitcast<half2_t>(and_or(__builtin_amdgcn_perm(0u, r.q[j][h], (uint32_t)b * 0x00010001u + 0x0C000C00u),
+                                                          nib_mask, exp_bits)) - off;
+                w[8 * h + 2 * b] = __builtin_fmaf((float)p[0], d, 0.0f);
+                w[8 * h + 2 * b + 1] = __builtin_fmaf((float)p[1], d, 0.0f);
+            }
+        }
+    } else {
+        const float s = wx_sz_f32(r.s[j], sz_dt), z = wx_sz_f32(r.z[j], sz_dt);
+        auto val = [&](float q) {
+#pragma clang fp contract(off)
+            return (q - z) * s;
+        };
+        if constexpr (WT == WX_I4) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                w[2 * i] = val(ubyte_f32(r.q[i] & 0x0F0F0F0Fu, j));
+                w[2 * i + 1] = val(ubyte_f32((r.q[i] >> 4) & 0x0F0F0F0Fu, j));
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) w[i] = val(ubyte_f32(r.q[i] ^ 0x80808080u, j) - 128.0f);
+        }
+        if constexpr (TAIL) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) w[i] = i < valid ? w[i] : 0.f;
+        }
+    }
+}
+
+// The B operands of tile j for 16-bit activations: ops[ks] = K elements
+// 8 ks .. +7 of the lane's 16.
+template <int WT, int XT, int TN, bool TAIL>
+__device__ __forceinline__ void wx_operands(const WxRaw<WT, TN> &r, int j, int sz_dt, int valid, uint4_t (&ops)[2]) {
+    if constexpr (WT == WX_Q4 && XT == DT_F16) {
+        const uint32_t dd = r.d[j];
+        const half2_t d2 = bitcast<half2_t>(dd | (dd << 16));
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) ops[ks] = bitcast<uint4_t>(dequant8_nat(r.q[j][ks], d2));
+    } else {
+        float w[16];
+        wx_values<WT, XT, TN, TAIL>(r, j, sz_dt, valid, w);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) ops[ks][u] = pack2<XT>(w[8 * ks + 2 * u], w[8 * ks + 2 * u + 1]);
+    }
+}
+
+template <int XT>
+__device__ __forceinline__ float16_t wx_mfma(uint4_t a, uint4_t b, float16_t c) {
+    if constexpr (XT == DT_BF16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(bitcast<bf16x8_t>(a), bitcast<bf16x8_t>(b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(bitcast<half8_t>(a), bitcast<half8_t>(b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ float wx_activate(float y, int act) {
+    if (act == ACT_SILU) return activate<ACT_SILU>(y);
+    if (act == ACT_GELU) return activate<ACT_GELU>(y);
+    return y;
+}
+
+// 16 bytes of activations (K elements k .. k + 16/ES - 1 of a row), any element
+// alignment, zero past K.
+template <int XT>
+__device__ __forceinline__ uint4_t wx_load_x_any(const uint8_t *row, int k, int K) {
+    uint4_t v = {0u, 0u, 0u, 0u};
+    if constexpr (XT == DT_F32) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (k + e < K) v[e] = ((const uint32_t *)row)[k + e];
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (k + e < K) v[e / 2] |= (uint32_t)((const uint16_t *)row)[k + e] << (16 * (e & 1));
+    }
+    return v;
+}
+
+// ---- host ------------------------------------------------------------------
+struct WxCall {
+    int wt, x_dt, sz_dt, act;
+    const void *X;
+    int64_t ldx;
+    const uint8_t *W;
+    const void *scales, *zeros;
+    void *Y;
+    int64_t ldy;
+    int64_t M, K, N, gs;
+};
+// Whether wx_gemm / wx_skinny take the call (any workspace, or none).
+bool wx_supported(const WxCall &c);
+size_t wx_workspace_bytes(int wt, int x_dt, int64_t M, int64_t K, int64_t N);
+// ws may be null or too small: the plan then keeps K whole.
+hipError_t launch_wx(const WxCall &c, void *ws, size_t ws_bytes, hipStream_t s);
+
+}  // namespace mcq4

@@ -1,0 +1,215 @@
+// Any-activation decode and small-batch matmul, M <= 64 (wx_common.h): one
+// 8-wave workgroup owns 32 TN columns; its waves split K, each a contiguous
+// range of K steps, and sum through LDS in wave order.
+//
+//   * Weights and activations go from global memory straight into MFMA operand
+//     registers, PF K steps ahead: no barrier until the end, any alignment.
+//     Each weight is read and dequantized once.
+//   * 32 TM activation rows (rows past M repeat the last one, their outputs are
+//     not stored): the weights' bytes bound the kernel, not its MFMAs.
+//   * Split K over workgroups (grid.z) where the columns alone leave CUs idle:
+//     fp32 partial rows summed in split order by wx_reduce_kernel.
+//
+// Measured: q4_0 x bf16 M = 4 4096x11008 13.0 us, was 199 (one thread per column,
+// 2-byte weight loads); INT4 x fp32 M = 32 4096x4096 26 us, was 811.
+#include <algorithm>
+
+#include "wx_common.h"
+
+namespace mcq4 {
+
+constexpr int WS_NW = 8;
+
+template <int WT, int XT, int TM, int TN, bool ANY>
+__global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
+    constexpr int ES = XT == DT_F32 ? 4 : 2;
+    constexpr int XV = XT == DT_F32 ? 4 : 2;     // 16-byte activation loads per row tile and step
+    constexpr int PF = TM == 1 && XT != DT_F32 && WT == WX_Q4 ? 4 : 2;
+    extern __shared__ __attribute__((aligned(16))) float red[];   // [waves][TM TN][16][64]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lrow = lane & 31, lhi = lane >> 5;
+    const int n0 = blockIdx.x * (32 * TN), z = blockIdx.z;
+    const int nks = (a.K + 31) / 32;
+    const int ws = z * WS_NW + wave, wt = a.S * WS_NW;
+    const int k_lo = (int)((int64_t)nks * ws / wt), nk = (int)((int64_t)nks * (ws + 1) / wt) - k_lo;
+
+    const WxLane<WT, TN> L = wx_lane<WT, TN>(a, n0, lane);
+    const uint8_t *xrow[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) xrow[i] = (const uint8_t *)a.X + (int64_t)min(32 * i + lrow, a.M - 1) * a.ldx * ES;
+
+    struct Step {
+        WxRaw<WT, TN> r;
+        uint4_t x[TM][XV];
+    } ring[PF];
+    int kld = 0, grp = WT == WX_Q4 ? 0 : k_lo / a.spg, gcnt = WT == WX_Q4 ? 0 : k_lo % a.spg;
+    auto load = [&](Step &p) {
+        const int kb = k_lo + kld;
+        wx_load<WT, TN, ANY && WT != WX_Q4>(p.r, a, L, kb, grp, lane);
+        const int k = kb * 32 + 16 * lhi;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int v = 0; v < XV; ++v) {
+                if constexpr (ANY) p.x[i][v] = wx_load_x_any<XT>(xrow[i], k + v * (16 / ES), a.K);
+                else p.x[i][v] = *(const uint4_t *)(xrow[i] + (int64_t)(k + v * (16 / ES)) * ES);
+            }
+        if (kld + 1 < nk) {
+            ++kld;
+            if (WT != WX_Q4 && ++gcnt == a.spg) { gcnt = 0; ++grp; }
+        }
+    };
+
+    float16_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+    auto step = [&](Step &p, int kk) {
+        const int valid = a.K - (k_lo + kk) * 32 - 16 * lhi;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            if constexpr (XT == DT_F32) {
+                float w[16];
+                wx_values<WT, XT, TN, ANY>(p.r, j, a.sz_dt, valid, w);
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(p.x[i][e / 4][e % 4]), w[e], acc[i][j], 0, 0, 0);
+            } else {
+                uint4_t B[2];
+                wx_operands<WT, XT, TN, ANY>(p.r, j, a.sz_dt, valid, B);
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) acc[i][j] = wx_mfma<XT>(p.x[i][ks], B[ks], acc[i][j]);
+            }
+        }
+    };
+
+    if (nk > 0) {
+#pragma unroll
+        for (int p = 0; p < PF; ++p) load(ring[p]);
+        for (int k0 = 0; k0 < nk; k0 += PF) {
+#pragma unroll
+            for (int p = 0; p < PF; ++p) {
+                if (k0 + p >= nk) break;
+                step(ring[p], k0 + p);
+                load(ring[p]);
+            }
+        }
+    }
+
+    // Wave sums: lane l holds rows 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of each tile.
+    constexpr int T = TM * TN;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (32 * i + 8 * (r >> 2) < a.M) red[((wave * T + i * TN + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+    __syncthreads();
+#pragma unroll 1
+    for (int v = tid; v < T * 1024; v += WS_NW * 64) {
+        const int t = v >> 10, r = (v >> 6) & 15, i = t / TN, j = t % TN;
+        const int m = 32 * i + 8 * (r >> 2) + 4 * lhi + (r & 3);
+        const int c0 = n0 + (WT == WX_Q4 ? 32 * j + lrow : TN * lrow);
+        if (m >= a.M || c0 >= a.N) continue;
+        const int n = WT == WX_Q4 ? c0 : min(c0, a.N - TN) + j;
+        float sum = red[v];
+#pragma unroll
+        for (int w = 1; w < WS_NW; ++w) sum += red[w * T * 1024 + v];
+        if (a.S > 1) a.part[((int64_t)z * a.M + m) * a.ldp + n] = sum;
+        else store_dt(a.Y, (int64_t)m * a.ldy + n, wx_activate(sum, a.act), XT);
+    }
+}
+
+hipError_t launch_wx_reduce(const WxArgs &a, int x_dt, hipStream_t s);
+hipError_t launch_wx_gemm(WxArgs a, int wt, int x_dt, bool any, hipStream_t s);
+int wx_gemm_splits(int64_t M, int64_t K, int64_t N);
+
+template <int WT, int XT, int TM, int TN, bool ANY>
+static hipError_t launch_wx_skinny_k(const WxArgs &a, hipStream_t s) {
+    const size_t lds = (size_t)WS_NW * TM * TN * 1024 * sizeof(float);
+    const dim3 grid((a.N + 32 * TN - 1) / (32 * TN), 1, a.S);
+    if (lds > 64 * 1024)
+        if (hipError_t e = hipFuncSetAttribute((const void *)wx_skinny_kernel<WT, XT, TM, TN, ANY>,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
+            return e;
+    hipLaunchKernelGGL((wx_skinny_kernel<WT, XT, TM, TN, ANY>), grid, dim3(WS_NW * 64), lds, s, a);
+    return hipGetLastError();
+}
+template <int WT, int XT>
+static hipError_t launch_wx_skinny_t(const WxArgs &a, bool any, hipStream_t s) {
+    constexpr int TN = 2;
+    if (a.M <= 32) return any ? launch_wx_skinny_k<WT, XT, 1, TN, true>(a, s) : launch_wx_skinny_k<WT, XT, 1, TN, false>(a, s);
+    return any ? launch_wx_skinny_k<WT, XT, 2, TN, true>(a, s) : launch_wx_skinny_k<WT, XT, 2, TN, false>(a, s);
+}
+template <int WT>
+static hipError_t launch_wx_skinny_w(const WxArgs &a, int x_dt, bool any, hipStream_t s) {
+    if (x_dt == DT_F16) return launch_wx_skinny_t<WT, DT_F16>(a, any, s);
+    if (x_dt == DT_BF16) return launch_wx_skinny_t<WT, DT_BF16>(a, any, s);
+    return launch_wx_skinny_t<WT, DT_F32>(a, any, s);
+}
+
+// K splits: one workgroup per CU, every wave at least 2 K steps.
+static int wx_skinny_splits(int64_t K, int64_t N) {
+    const int64_t t = (N + 63) / 64, nks = (K + 31) / 32;
+    int S = 1;
+    while (t * S * 2 <= 256 && nks / (S * 2 * WS_NW) >= 2 && S < 16) S *= 2;
+    return S;
+}
+
+static int64_t wx_ldp(int64_t N) { return (N + 3) / 4 * 4; }
+
+// Partials stay within 16 MiB, what the allocation-free entry point holds.
+static int wx_splits(int64_t M, int64_t K, int64_t N) {
+    int S = M <= 64 ? wx_skinny_splits(K, N) : wx_gemm_splits(M, K, N);
+    while (S > 1 && (int64_t)S * M * wx_ldp(N) * 4 > ((int64_t)16 << 20)) S /= 2;
+    return S;
+}
+
+size_t wx_workspace_bytes(int wt, int x_dt, int64_t M, int64_t K, int64_t N) {
+    (void)wt; (void)x_dt;
+    const int S = wx_splits(M, K, N);
+    // Partials follow the counter area, which other kernels rely on staying zero.
+    return S == 1 ? 0 : COUNTER_BYTES + (size_t)S * M * wx_ldp(N) * sizeof(float);
+}
+
+// Every q4_0 call; INT4 and INT8 with groups of whole K steps, at least one pair
+// of columns (a lane loads two at a time) and 16 rows within a 32-bit offset.  The fused
+// activations exist for INT4 x fp16 only.
+bool wx_supported(const WxCall &c) {
+    if (c.wt != WX_Q4 && (c.gs % 32 != 0 || c.N < 2 || c.N > (1 << 27))) return false;
+    if (c.act != ACT_NONE && (c.wt != WX_I4 || c.x_dt != DT_F16)) return false;
+    return true;
+}
+
+hipError_t launch_wx(const WxCall &c, void *ws, size_t ws_bytes, hipStream_t s) {
+    WxArgs a;
+    a.X = c.X; a.ldx = c.ldx; a.W = c.W; a.scales = c.scales; a.zeros = c.zeros; a.sz_dt = c.sz_dt;
+    a.Y = c.Y; a.ldy = c.ldy; a.M = (int)c.M; a.K = (int)c.K; a.N = (int)c.N;
+    a.spg = c.wt == WX_Q4 ? 1 : (int)std::min<int64_t>(c.gs / 32, 1 << 26);
+    a.act = c.act;
+    a.S = wx_splits(c.M, c.K, c.N);
+    if (a.S > 1 && (!ws || ws_bytes < wx_workspace_bytes(c.wt, c.x_dt, c.M, c.K, c.N))) a.S = 1;
+    a.ldp = (int)wx_ldp(c.N);
+    a.part = a.S > 1 ? (float *)((char *)ws + COUNTER_BYTES) : nullptr;
+    a.tiles_m = a.tiles_n = 0;
+    const int es = c.x_dt == DT_F32 ? 4 : 2;
+    const bool any = (uintptr_t)c.X % 16 != 0 || (c.ldx * es) % 16 != 0 || c.K % 32 != 0;
+    if (c.M > 64) return launch_wx_gemm(a, c.wt, c.x_dt, any, s);
+    const hipError_t e = c.wt == WX_Q4   ? launch_wx_skinny_w<WX_Q4>(a, c.x_dt, any, s)
+                         : c.wt == WX_I4 ? launch_wx_skinny_w<WX_I4>(a, c.x_dt, any, s)
+                                         : launch_wx_skinny_w<WX_I8>(a, c.x_dt, any, s);
+    if (e != hipSuccess || a.S == 1) return e;
+    return launch_wx_reduce(a, c.x_dt, s);
+}
+
+}  // namespace mcq4

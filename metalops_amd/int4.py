@@ -248,9 +248,10 @@ def matmul_int4(
     fp32 accumulation; the result has ``X``'s dtype.  fp16 activations run the
     MFMA kernels (decode GEMV for M <= 16 rows, and up to 32 rows when N is a
     multiple of 128; prefill GEMM above); fp32 and
-    bf16 activations run the general fp32 kernel with the weight rounded to
-    ``X``'s dtype first, as the reference builds ``W`` in ``X.dtype``
-    (quantization.py:220-239).
+    bf16 activations, and fp16 ones at other shapes, use the weight rounded to
+    ``X``'s dtype, as the reference builds ``W`` in ``X.dtype``
+    (quantization.py:220-239), on the matrix cores of that dtype; group sizes
+    that are no multiple of 32 run the general fp32 kernel.
     """
     return _matmul(X, W_packed, scales, zeros, group_size, 0)
 
@@ -322,8 +323,8 @@ def matmul_int8(
 
     ``W[k, n] = (q - zero) * scale`` per group of ``group_size`` rows; fp32
     accumulation, result in ``X``'s dtype.  fp16 activations run the MFMA
-    kernels, other dtypes the general kernel (weights rounded to ``X``'s dtype
-    as the reference's fallback builds ``W`` in ``X.dtype``).
+    kernels; other dtypes use weights rounded to ``X``'s dtype, as the
+    reference's fallback builds ``W`` in ``X.dtype``.
     """
     _require_device(X, W_packed, scales, zeros)
     if X.dim() != 2:

@@ -212,10 +212,15 @@ def matmul_ggml_q4_0(X: torch.Tensor, W_blocks: torch.Tensor) -> torch.Tensor:
     stream = _stream(X.device)
     if X.dtype != torch.float16:
         x = X if (X.stride(1) == 1 and X.stride(0) >= K) else X.contiguous()
+        code = _DTYPE_CODES[x.dtype]
+        need = int(_lib.lib.mcq4_matmul_q4_0_workspace_bytes(M, K, N, code))
+        ws_ptr, ws_bytes = None, 0
+        if need:
+            ws = _workspace.get(x.device, stream, need)
+            ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
         with torch.cuda.device(x.device):
-            _lib.check(_lib.lib.mcq4_matmul_q4_0(x.data_ptr(), _DTYPE_CODES[x.dtype], x.stride(0),
-                                                 w.data_ptr(), Y.data_ptr(), N, M, K, N, None, 0,
-                                                 stream),
+            _lib.check(_lib.lib.mcq4_matmul_q4_0(x.data_ptr(), code, x.stride(0), w.data_ptr(), Y.data_ptr(), N, M, K,
+                                                 N, ws_ptr, ws_bytes, stream),
                        "mcq4_matmul_q4_0")
         return Y
     x = X
