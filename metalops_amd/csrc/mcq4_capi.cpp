@@ -38,7 +38,7 @@ hipError_t launch_zero_counters(void *ws, hipStream_t s);
 size_t gemm7_workspace_bytes(int64_t M, int64_t K, int64_t N);
 bool gemm7_supported(const _Float16 *X, int64_t ldx, const uint8_t *W, int64_t M, int64_t K, int64_t N);
 hipError_t launch_gemm7(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
-                        int64_t ldy, int M, int K, int N, void *ws, hipStream_t s);
+                        int64_t ldy, int M, int K, int N, int x_dt, void *ws, hipStream_t s);
 hipError_t q4_gemvm_split_fallbacks(uint64_t *count, bool reset);
 hipError_t q4_gemm6_split_fallbacks(uint64_t *count, bool reset);
 hipError_t i4_gemv_split_fallbacks(uint64_t *count, bool reset);
@@ -73,15 +73,14 @@ constexpr int64_t kMaxDim = (int64_t)1 << 30;  // keeps 32-bit lane offsets safe
 
 bool aligned(const void *p, uintptr_t a) { return ((uintptr_t)p % a) == 0; }
 
-// Prefill kernel choice (M > 64).  When N % 128 == 0 and the pointers are
-// 16-byte aligned: the few-tile GEMM (q4_gemm8) when its plan is one round of
-// workgroups, the 256 x 256-tile GEMM (q4_gemm7) on grids that nearly fill the
-// CUs, else the 128 x 256-tile LDS-staged GEMM with two waves per SIMD
-// (q4_gemm6).  Otherwise the async-copy GEMM (q4_gemm2) when its alignment
-// needs hold and the output has at least 128 tiles of 128x256; otherwise the
-// register-staged split-K kernel.  MCQ4_GEMM_PATH=sync|async|6|7|8 forces one
-// kernel (tests).
-enum class Prefill { Sync, Async2, Staged6, Wide7, Few8 };
+// Prefill kernel choice (M > 64).  When N % 8 == 0 and the pointers are
+// 16-byte aligned: the few-tile GEMM (q4_gemm8, N % 128 == 0) when its plan is
+// one round of workgroups, the 256 x 256-tile GEMM (q4_gemm7) on grids that
+// nearly fill the CUs, else the 128 x 256-tile LDS-staged GEMM with two waves per
+// SIMD (q4_gemm6).  Otherwise the kernel without alignment needs (wx_gemm).
+// MCQ4_GEMM_PATH=sync|async|6|7|8 forces one kernel (tests; sync and async are
+// the fp16 kernels q4_gemm and q4_gemm2).
+enum class Prefill { Sync, Async2, Staged6, Wide7, Few8, Any };
 Prefill prefill_kernel(const _Float16 *X, int64_t ldx, const uint8_t *W, int64_t M, int64_t K,
                        int64_t N) {
     const bool ok2 = mcq4::gemm2_supported(X, ldx, W, K, N);
@@ -117,8 +116,13 @@ Prefill prefill_kernel(const _Float16 *X, int64_t ldx, const uint8_t *W, int64_t
         if (t7 >= 160 || (t7 >= 96 && K >= 8192)) return Prefill::Wide7;
     }
     if (ok6) return Prefill::Staged6;
-    if (ok2 && ((M + 127) / 128) * ((N + 255) / 256) >= 128) return Prefill::Async2;
-    return Prefill::Sync;
+    return Prefill::Any;
+}
+
+// The most any of the aligned prefill kernels asks for.
+size_t prefill_ws_bytes(int64_t M, int64_t K, int64_t N) {
+    return std::max({mcq4::gemm6_workspace_bytes(M, K, N), mcq4::gemm7_workspace_bytes(M, K, N),
+                     mcq4::gemm8_workspace_bytes(M, K, N)});
 }
 
 int check_kn(int64_t K, int64_t N) {
@@ -249,20 +253,27 @@ int mcq4_dequantize_q4_0(const uint8_t *blocks, int64_t K, int64_t N, void *out,
                       "dequantize launch");
 }
 
-size_t mcq4_matmul_workspace_bytes(int64_t M, int64_t K, int64_t N) {
+// What mcq4_matmul_q4_0_f16 cannot do without.
+static size_t required_ws_bytes(int64_t M, int64_t K, int64_t N) {
     if (M <= 0 || K <= 0 || N <= 0 || K % 32) return 0;
     if (M <= 32) return mcq4::skinny_workspace_bytes(M, K, N);
     // The largest of the split-K kernels' needs: an upper bound for any prefill kernel.
-    const size_t pre = std::max({mcq4::gemm_workspace_bytes(M, K, N), mcq4::gemm6_workspace_bytes(M, K, N),
-                                 mcq4::gemm7_workspace_bytes(M, K, N), mcq4::gemm8_workspace_bytes(M, K, N)});
+    const size_t pre = std::max(mcq4::gemm_workspace_bytes(M, K, N), prefill_ws_bytes(M, K, N));
     // 33..64 rows run either family, depending on the pointers' alignment.
     return M <= 64 ? std::max(pre, mcq4::skinny_workspace_bytes(M, K, N)) : pre;
+}
+
+size_t mcq4_matmul_workspace_bytes(int64_t M, int64_t K, int64_t N) {
+    const size_t need = required_ws_bytes(M, K, N);
+    // wx splits K only where the workspace covers it.
+    return M > 32 && K > 0 && N > 0 && K % 32 == 0 ? std::max(need, mcq4::wx_workspace_bytes(mcq4::WX_Q4, mcq4::DT_F16, M, K, N)) : need;
 }
 
 size_t mcq4_matmul_q4_0_workspace_bytes(int64_t M, int64_t K, int64_t N, int x_dtype) {
     if (x_dtype == MCQ4_DTYPE_F16) return mcq4_matmul_workspace_bytes(M, K, N);
     if (M <= 0 || K <= 0 || N <= 0 || K % 32) return 0;
-    return mcq4::wx_workspace_bytes(mcq4::WX_Q4, x_dtype, M, K, N);
+    const size_t any = mcq4::wx_workspace_bytes(mcq4::WX_Q4, x_dtype, M, K, N);
+    return x_dtype == MCQ4_DTYPE_BF16 && M > 64 ? std::max(any, prefill_ws_bytes(M, K, N)) : any;
 }
 
 int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, int64_t ldy,
@@ -279,7 +290,7 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
         return fail(MCQ4_ERR_ALIGNMENT, "X must be 16-byte aligned with ldx %% 8 == 0");
     if (!aligned(W, 2)) return fail(MCQ4_ERR_ALIGNMENT, "W must be 2-byte aligned");
     if (!aligned(Y, 2)) return fail(MCQ4_ERR_ALIGNMENT, "Y must be 2-byte aligned");
-    const size_t need = mcq4_matmul_workspace_bytes(M, K, N);
+    const size_t need = required_ws_bytes(M, K, N);
     if (need && (!workspace || workspace_bytes < need))
         return fail(MCQ4_ERR_WORKSPACE, "workspace of %zu bytes required, %zu given", need,
                     workspace ? workspace_bytes : (size_t)0);
@@ -297,10 +308,11 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
         _Float16 *y = (_Float16 *)Y;
         hipStream_t st = (hipStream_t)stream;
         switch (prefill_kernel(x, ldx, W, M, K, N)) {
-            case Prefill::Staged6: e = mcq4::launch_gemm6(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, workspace, st); break;
-            case Prefill::Wide7: e = mcq4::launch_gemm7(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, workspace, st); break;
-            case Prefill::Few8: e = mcq4::launch_gemm8(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, workspace, st); break;
+            case Prefill::Staged6: e = mcq4::launch_gemm6(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, mcq4::DT_F16, workspace, st); break;
+            case Prefill::Wide7: e = mcq4::launch_gemm7(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, mcq4::DT_F16, workspace, st); break;
+            case Prefill::Few8: e = mcq4::launch_gemm8(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, mcq4::DT_F16, workspace, st); break;
             case Prefill::Async2: e = mcq4::launch_gemm2(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, st); break;
+            case Prefill::Any: e = mcq4::launch_wx({mcq4::WX_Q4, mcq4::DT_F16, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32}, workspace, workspace_bytes, st); break;
             default: e = mcq4::launch_gemm(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, workspace, st); break;
         }
     }
@@ -355,6 +367,22 @@ int mcq4_matmul_q4_0(const void *X, int x_dtype, int64_t ldx, const uint8_t *W, 
         return fail(MCQ4_ERR_ALIGNMENT, "X and Y must be aligned to their dtype");
     if (!aligned(W, 2)) return fail(MCQ4_ERR_ALIGNMENT, "W must be 2-byte aligned");
     if (workspace && !aligned(workspace, 16)) workspace = nullptr;   // optional here: K stays whole
+    if (x_dtype == MCQ4_DTYPE_BF16 && M > 64 && aligned(X, 16) && ldx % 8 == 0) {
+        // The aligned prefill kernels, where the workspace covers their plans.
+        const size_t need = prefill_ws_bytes(M, K, N);
+        if (!need || (workspace && workspace_bytes >= need)) {
+            const _Float16 *x = (const _Float16 *)X;
+            _Float16 *y = (_Float16 *)Y;
+            hipStream_t st = (hipStream_t)stream;
+            const int m = (int)M, k = (int)K, n = (int)N, dt = mcq4::DT_BF16;
+            switch (prefill_kernel(x, ldx, W, M, K, N)) {
+                case Prefill::Staged6: return hip_status(mcq4::launch_gemm6(x, ldx, W, y, ldy, m, k, n, dt, workspace, st), "matmul launch");
+                case Prefill::Wide7: return hip_status(mcq4::launch_gemm7(x, ldx, W, y, ldy, m, k, n, dt, workspace, st), "matmul launch");
+                case Prefill::Few8: return hip_status(mcq4::launch_gemm8(x, ldx, W, y, ldy, m, k, n, dt, workspace, st), "matmul launch");
+                default: break;
+            }
+        }
+    }
     const mcq4::WxCall c = {mcq4::WX_Q4, x_dtype, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32};
     return hip_status(mcq4::launch_wx(c, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
 }
@@ -388,7 +416,7 @@ int mcq4_matmul_q4_0_f16_noalloc(const void *X, int64_t ldx, const uint8_t *W, v
                                  int64_t M, int64_t K, int64_t N, void *stream) {
     g_err[0] = 0;
     if (M > 0 && K > 0 && N > 0 && K % 32 == 0) {
-        const size_t need = mcq4_matmul_workspace_bytes(M, K, N);
+        const size_t need = required_ws_bytes(M, K, N);
         if (need > kNoAllocScratchBytes)
             return fail(MCQ4_ERR_WORKSPACE,
                         "shape M=%lld K=%lld N=%lld needs a %zu-byte workspace; the allocation-free entry "

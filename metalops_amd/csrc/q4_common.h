@@ -110,8 +110,9 @@ __host__ __device__ __forceinline__ uint32_t xcd_ticket_local_mask(uint64_t tota
     }
 
 // One output of the q4_0 product over K blocks [kb0, kb1): sum of x[k] times
-// the fp16 weight (q - 8)*d, in fp32 -- the split-K recompute path of the
+// the fp16 (BF16: bf16, x too) weight (q - 8)*d, in fp32 -- the split-K recompute path of the
 // exchange above (slow, taken only when a split ran on another XCD).
+template <bool BF16 = false>
 __device__ __forceinline__ float q4_dot_range(const _Float16 *xrow, const uint8_t *W, int N, int n,
                                                   int kb0, int kb1) {
     float acc = 0.f;
@@ -121,8 +122,10 @@ __device__ __forceinline__ float q4_dot_range(const _Float16 *xrow, const uint8_
         for (int i = 0; i < 8; ++i) {
             const uint32_t w = b[1 + i];
             for (int e = 0; e < 4; ++e) {
-                const _Float16 wv = (_Float16)((float)((int)((w >> (4 * e)) & 0xF) - 8) * d);
-                acc += (float)xrow[kb * QK + 4 * i + e] * (float)wv;
+                const float wv = (float)((int)((w >> (4 * e)) & 0xF) - 8) * d;
+                const _Float16 x = xrow[kb * QK + 4 * i + e];
+                if constexpr (BF16) acc += (float)__builtin_bit_cast(__bf16, x) * (float)(__bf16)wv;
+                else acc += (float)x * (float)(_Float16)wv;
             }
         }
     }

@@ -43,6 +43,7 @@ constexpr size_t G6_LDS = (size_t)G6_NS * (128 * WGM) * G6_ROWB + (size_t)(4 * W
 static_assert(2 * G6_LDS <= 160 * 1024, "LDS budget: two workgroups per CU");
 static_assert(G6_RAW_SLOT >= 1024 + 64 * 4 && G6_RAW_SLOT >= G6_RAW_W + 16, "raw slot covers the remainder copy and the read overhang");
 
+template <int XT>
 __global__ void __launch_bounds__(256, 2)
 q4_gemm6_kernel(Gemm6Args a) {
     constexpr int BM = 128 * WGM, NWAVES = 4 * WGM;
@@ -100,7 +101,10 @@ q4_gemm6_kernel(Gemm6Args a) {
     const __amdgpu_buffer_rsrc_t w_rs =
         __builtin_amdgcn_make_buffer_rsrc((void *)a.W, (short)0, (int)0x7fffffff, 0x00020000);
     const uint32_t w_so0 = (uint32_t)k_lo * row_bytes + (wcols ? (uint32_t)(n0 + wn * WN) * BLOCK_BYTES : 0u);
-    const uint32_t w_vo16 = 16 * lane, w_vo4 = 4 * min(lane, 31);
+    // Columns past N (N % 8 == 0): the lane re-reads the row's last bytes, whose
+    // outputs are not stored, so nothing past the row is read.
+    const uint32_t w_valid = wcols ? (uint32_t)min(WN, a.N - (n0 + wn * WN)) * BLOCK_BYTES : G6_RAW_W;
+    const uint32_t w_vo16 = min(16u * lane, w_valid - 16), w_vo4 = min(1024u + 4u * min(lane, 31), w_valid - 4);
 
     // Copy ci (0 .. GROUP-1) of stage s_dst: A copies, then per step t the raw
     // bytes 0..1023 (16 per lane) and 1024..1151 (4 per lane for lanes 0..31;
@@ -127,7 +131,7 @@ q4_gemm6_kernel(Gemm6Args a) {
                                                      so, 0, 0);
         else
             __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rs, (__attribute__((address_space(3))) void *)(dst + 1024), 4,
-                                                     w_vo4, so + 1024, 0, 0);
+                                                     w_vo4, so, 0, 0);
     };
     auto issue_stage = [&](int s_dst) {
 #pragma unroll
@@ -164,8 +168,6 @@ q4_gemm6_kernel(Gemm6Args a) {
     for (int u = 0; u < 4; ++u) bsel[u] = (uint32_t)(q_b + u) * 0x00010001u + 0x0C000C00u;
     const uint32_t nib_mask = opaque_sgpr(0x00F0000Fu), exp_bits = opaque_vgpr(0x54006400u);
     auto load_b = [&](int k, half8_t (&bv)[2][TN]) {
-#pragma clang fp contract(off)
-        const half2_t off = {(_Float16)1032.0f, (_Float16)72.0f};
         const lds_u8 *Rs = lds_ptr(lds_addr(ring + (k % G6_RAW_N) * G6_RAW_SLOT));
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
@@ -174,15 +176,15 @@ q4_gemm6_kernel(Gemm6Args a) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) qd[t] = qp[t];
             const uint32_t dd = *(const lds_u16 *)(Rs + d_off + j * 32 * 18);
-            const half2_t d2 = bitcast<half2_t>(__builtin_amdgcn_perm(dd, dd, 0x01000100u));
+            Q4Scale<XT> sc;
+            sc.set(dd);
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
                 uint4_t r;
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    const half2_t h = bitcast<half2_t>(
+                    r[u] = sc.weights(
                         and_or(__builtin_amdgcn_perm(qd[2 * ks + 1], qd[2 * ks], bsel[u]), nib_mask, exp_bits));
-                    r[u] = bitcast<uint32_t>((h - off) * d2);
                 }
                 bv[ks][j] = bitcast<half8_t>(r);
             }
@@ -208,7 +210,6 @@ q4_gemm6_kernel(Gemm6Args a) {
     half8_t A[2][TM];
     auto step = [&](auto with_copies, int cs, const half8_t (&B)[2][TN], int k_next,
                     half8_t (&Bn)[2][TN], int a_s, int a_t) {
-#pragma clang fp contract(off)
         const lds_u8 *Rs = lds_ptr(lds_addr(ring + (k_next % G6_RAW_N) * G6_RAW_SLOT));
         uint32_t qd[TN][4], dd[TN];
 #pragma unroll
@@ -218,25 +219,24 @@ q4_gemm6_kernel(Gemm6Args a) {
             for (int t = 0; t < 4; ++t) qd[j][t] = qp[t];
             dd[j] = *(const lds_u16 *)(Rs + d_off + j * 32 * 18);
         }
-        const half2_t off = {(_Float16)1032.0f, (_Float16)72.0f};
-        half2_t d2[TN];
+        Q4Scale<XT> sc[TN];
         uint32_t xw[NMF];
         uint4_t bb[2 * TN];
         auto first = [&](int d) {
             const int unit = d >> 2, u = d & 3, uj = unit >> 1, uk = unit & 1;
-            if (u == 0 && uk == 0) d2[uj] = bitcast<half2_t>(__builtin_amdgcn_perm(dd[uj], dd[uj], 0x01000100u));
+            if (u == 0 && uk == 0) sc[uj].set(dd[uj]);
             xw[d] = and_or(__builtin_amdgcn_perm(qd[uj][2 * uk + 1], qd[uj][2 * uk], bsel[u]), nib_mask, exp_bits);
         };
         auto second = [&](int d) {
             const int unit = d >> 2, u = d & 3, uj = unit >> 1, uk = unit & 1;
-            bb[unit][u] = bitcast<uint32_t>((bitcast<half2_t>(xw[d]) - off) * d2[uj]);
+            bb[unit][u] = sc[uj].weights(xw[d]);
             if (u == 3) Bn[uk][uj] = bitcast<half8_t>(bb[unit]);
         };
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int idx = 0; idx < NMF; ++idx) {
             const int ks = idx / (TM * TN), i = (idx / TN) % TM, j = idx % TN;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[ks][i], B[ks][j], acc[i][j], 0, 0, 0);
+            acc[i][j] = mfma32<XT>(A[ks][i], B[ks][j], acc[i][j]);
             if (j == TN - 1) A[ks][i] = read_a1(a_s, a_t, ks, i);
             if constexpr (decltype(with_copies)::value) {
                 if ((idx & 1) == 1 && (idx >> 1) < GROUP) issue_one(cs, idx >> 1);
@@ -279,7 +279,7 @@ q4_gemm6_kernel(Gemm6Args a) {
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[ks][i], B0[ks][j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = mfma32<XT>(A[ks][i], B0[ks][j], acc[i][j]);
     }
     wait_vmcnt<0>();
 
@@ -293,7 +293,7 @@ q4_gemm6_kernel(Gemm6Args a) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int m = m0 + wm * WM + i * 32 + 8 * (r >> 2) + rsub + (r & 3);
-                    if (m < a.M && n < a.N) a.Y[(int64_t)m * a.ldy + n] = (_Float16)acc[i][j][r];
+                    if (m < a.M && n < a.N) a.Y[(int64_t)m * a.ldy + n] = out16<XT>(acc[i][j][r]);
                 }
             }
         return;
@@ -346,7 +346,7 @@ q4_gemm6_kernel(Gemm6Args a) {
 #pragma unroll 1
         for (int v = tid; v < BM * G6_BN; v += 256) {
             const int m = min(m0 + v / G6_BN, a.M - 1), n = min(n0 + v % G6_BN, a.N - 1);
-            other[v] = q4_dot_range(a.X + (int64_t)m * a.ldx, a.W, a.N, n, o_lo, o_hi);
+            other[v] = q4_dot_range<XT == DT_BF16>(a.X + (int64_t)m * a.ldx, a.W, a.N, n, o_lo, o_hi);
         }
         wait_vmcnt<0>();
         __syncthreads();
@@ -367,18 +367,18 @@ q4_gemm6_kernel(Gemm6Args a) {
                 const int m = m0 + wm * WM + i * 32 + 8 * (r >> 2) + rsub + (r & 3), n = n0 + nl;
                 // p0 + p1 in split order
                 const float v = z == 0 ? acc[i][j][r] + o[r] : o[r] + acc[i][j][r];
-                if (m < a.M && n < a.N) a.Y[(int64_t)m * a.ldy + n] = (_Float16)v;
+                if (m < a.M && n < a.N) a.Y[(int64_t)m * a.ldy + n] = out16<XT>(v);
             }
         }
 }
 
 // Sums the S fp32 partial tiles of every output tile in split order
-// (deterministic) and stores fp16.  Thread t of block b owns float4 v = 256 b +
+// (deterministic) and stores fp16 or bf16.  Thread t of block b owns float4 v = 256 b +
 // t + 256 u of the [tiles][128 x 256] output for u < G6_RV; with S a template
 // argument every split's loads of all its float4 go out before the first add
 // (SC == 0: S read at run time, one split's loads at a time).
 constexpr int G6_RV = 2;
-template <int SC>
+template <int SC, int XT>
 __global__ void __launch_bounds__(256)
 q4_gemm6_reduce_kernel(Gemm6Args a) {
     constexpr int TILE = G6_BM * G6_BN;
@@ -427,12 +427,12 @@ q4_gemm6_reduce_kernel(Gemm6Args a) {
         if (m >= a.M) continue;
         _Float16 *y = a.Y + (int64_t)m * a.ldy + n;
         if (n + 3 < a.N && ((uintptr_t)y & 7) == 0) {
-            const half4_t h = {(_Float16)sum[u][0], (_Float16)sum[u][1], (_Float16)sum[u][2], (_Float16)sum[u][3]};
+            const half4_t h = {out16<XT>(sum[u][0]), out16<XT>(sum[u][1]), out16<XT>(sum[u][2]), out16<XT>(sum[u][3])};
             *(half4_t *)y = h;
         } else {
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                if (n + c < a.N) y[c] = (_Float16)sum[u][c];
+                if (n + c < a.N) y[c] = out16<XT>(sum[u][c]);
         }
     }
 }
@@ -458,7 +458,7 @@ static int gemm6_splits(int64_t M, int64_t K, int64_t N) {
 
 bool gemm6_supported(const _Float16 *X, int64_t ldx, const uint8_t *W, int64_t M, int64_t K, int64_t N) {
     // Buffer loads: activations below 2^31 bytes, W below 2^31 bytes.
-    return N % 128 == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)X % 16) == 0 && ldx % 8 == 0 &&
+    return N % 8 == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)X % 16) == 0 && ldx % 8 == 0 &&
            K >= QK && M * ldx < ((int64_t)1 << 30) && (K / QK) * N * BLOCK_BYTES < ((int64_t)1 << 31);
 }
 
@@ -469,7 +469,8 @@ size_t gemm6_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     return COUNTER_BYTES + (size_t)t * S * G6_BM * G6_BN * sizeof(float);
 }
 
-hipError_t launch_gemm6(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
+template <int XT>
+static hipError_t launch_gemm6_t(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
                         int64_t ldy, int M, int K, int N, void *ws, hipStream_t s) {
     Gemm6Args a;
     a.X = X; a.ldx = ldx; a.W = W; a.Y = Y; a.ldy = ldy;
@@ -493,25 +494,31 @@ hipError_t launch_gemm6(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float
     if (e != hipSuccess) return e;
     const uint64_t bit = 1ull << (dev & 63);
     if (!(done.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void *)q4_gemm6_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+        e = hipFuncSetAttribute((const void *)q4_gemm6_kernel<XT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)G6_LDS);
         if (e != hipSuccess) return e;
         done.fetch_or(bit, std::memory_order_acq_rel);
     }
     const int ntiles = a.tiles_m * a.tiles_n;
     const int gx = a.tickets ? (ntiles + 7) / 8 * 8 : ntiles;
-    hipLaunchKernelGGL(q4_gemm6_kernel, dim3(gx, 1, a.S), dim3(256), G6_LDS, s, a);
+    hipLaunchKernelGGL(q4_gemm6_kernel<XT>, dim3(gx, 1, a.S), dim3(256), G6_LDS, s, a);
     if (a.S > 1 && !a.tickets) {
         const int64_t n4 = (int64_t)ntiles * (G6_BM * G6_BN / 4);
         const dim3 grid((unsigned)((n4 + 256 * G6_RV - 1) / (256 * G6_RV)));
         switch (a.S) {
-            case 2: hipLaunchKernelGGL(q4_gemm6_reduce_kernel<2>, grid, dim3(256), 0, s, a); break;
-            case 4: hipLaunchKernelGGL(q4_gemm6_reduce_kernel<4>, grid, dim3(256), 0, s, a); break;
-            case 8: hipLaunchKernelGGL(q4_gemm6_reduce_kernel<8>, grid, dim3(256), 0, s, a); break;
-            default: hipLaunchKernelGGL(q4_gemm6_reduce_kernel<0>, grid, dim3(256), 0, s, a); break;
+            case 2: hipLaunchKernelGGL((q4_gemm6_reduce_kernel<2, XT>), grid, dim3(256), 0, s, a); break;
+            case 4: hipLaunchKernelGGL((q4_gemm6_reduce_kernel<4, XT>), grid, dim3(256), 0, s, a); break;
+            case 8: hipLaunchKernelGGL((q4_gemm6_reduce_kernel<8, XT>), grid, dim3(256), 0, s, a); break;
+            default: hipLaunchKernelGGL((q4_gemm6_reduce_kernel<0, XT>), grid, dim3(256), 0, s, a); break;
         }
     }
     return hipGetLastError();
+}
+
+hipError_t launch_gemm6(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
+                        int64_t ldy, int M, int K, int N, int x_dt, void *ws, hipStream_t s) {
+    return x_dt == DT_BF16 ? launch_gemm6_t<DT_BF16>(X, ldx, W, Y, ldy, M, K, N, ws, s)
+                           : launch_gemm6_t<DT_F16>(X, ldx, W, Y, ldy, M, K, N, ws, s);
 }
 
 }  // namespace mcq4

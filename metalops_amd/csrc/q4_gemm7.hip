@@ -58,6 +58,15 @@ struct Gemm7Args {
     float *partials;     // [tiles][S][256*256] when S > 1
 };
 
+// A plain function: with these lines inside the kernel template, the host pass
+// drops the kernel's stub.
+__device__ __forceinline__ void g7_copy_a(const uint8_t *base, int off, int bytes, uint8_t *dst, int vo) {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(base + off), (short)0, max(0, bytes - off), 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16, vo, 0, 0, 0);
+}
+
+template <int XT>
 __global__ void __launch_bounds__(256, 1)
 q4_gemm7_kernel(Gemm7Args a) {
     constexpr int TM = G7_BM / 32, TN = G7_WN / 32;   // 8 x 2
@@ -102,13 +111,13 @@ q4_gemm7_kernel(Gemm7Args a) {
     const int vo_a1 = (64 * wave + (lane >> 3)) * x_row + 16 * (a_c1 & 3) + 64 * (a_c1 >> 2);
 
     const int row_bytes = a.N * BLOCK_BYTES;
-    const int w_off = k_lo * row_bytes + (n0 + wave * G7_WN) * BLOCK_BYTES;
+    const int w_off = k_lo * row_bytes + min(n0 + wave * G7_WN, a.N - 8) * BLOCK_BYTES;
     const uint8_t *w_base = a.W + w_off;
     const int w_bytes = a.nb * row_bytes - w_off;                                       // readable from w_base
-    const int vo_w0 = 16 * lane, vo_w1 = 1024 + 4 * min(lane, 31);
-    auto rsrc = [](const uint8_t *base, int off, int bytes) {
-        return __builtin_amdgcn_make_buffer_rsrc((void *)(base + off), (short)0, max(0, bytes - off), 0x00020000);
-    };
+    // Columns past N (N % 8 == 0): the lane re-reads the row's last bytes, whose
+    // outputs are not stored (a wave wholly past N: any bytes in range).
+    const int w_valid = max(16, min(G7_WN, a.N - (n0 + wave * G7_WN)) * BLOCK_BYTES);
+    const int vo_w0 = min(16 * lane, w_valid - 16), vo_w1 = min(1024 + 4 * min(lane, 31), w_valid - 4);
 
     // Copies of a stage: A copies ci = 0..7 of stage s_a, then the raw copies
     // ci = 8..11 of stage s_r: per step t the raw bytes 0..1023 (16 per lane)
@@ -125,14 +134,12 @@ q4_gemm7_kernel(Gemm7Args a) {
     // per lane still fill 4 bytes per lane).  Stages past the end re-copy the
     // last stage, so every stage issues the same number of copies and the vmcnt
     // waits are exact.
-    const __amdgpu_buffer_rsrc_t w_rs = rsrc(w_base, 0, w_bytes);
+    const __amdgpu_buffer_rsrc_t w_rs = __builtin_amdgcn_make_buffer_rsrc((void *)w_base, (short)0, max(0, w_bytes), 0x00020000);
     auto issue_one = [&](int s_a, int as_, int s_r, int ci) {
         if (ci < A_LD) {
             const int s_src = min(s_a, nst - 1);
             uint8_t *dst = sA + as_ * G7_A_SLOT + G7_ROWB * (64 * wave + 8 * ci);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(x_base, 128 * s_src, x_bytes),
-                                                     (__attribute__((address_space(3))) void *)dst, 16,
-                                                     ((ci & 1) ? vo_a1 : vo_a0) + 8 * ci * x_row, 0, 0, 0);
+            g7_copy_a(x_base, 128 * s_src, x_bytes, dst, ((ci & 1) ? vo_a1 : vo_a0) + 8 * ci * x_row);
             return;
         }
         const int s_src = min(s_r, nst - 1);
@@ -196,22 +203,18 @@ q4_gemm7_kernel(Gemm7Args a) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) bsel[u] = (uint32_t)(q_b + u) * 0x00010001u + 0x0C000C00u;
     const uint32_t nib_mask = opaque_sgpr(0x00F0000Fu), exp_bits = opaque_vgpr(0x54006400u);
-    auto dq2 = [&](uint32_t hi_w, uint32_t lo_w, int u, half2_t d2) {
-#pragma clang fp contract(off)
-        const half2_t off = {(_Float16)1032.0f, (_Float16)72.0f};
-        const uint32_t x = __builtin_amdgcn_perm(hi_w, lo_w, bsel[u]);
-        const half2_t h = bitcast<half2_t>(and_or(x, nib_mask, exp_bits));
-        return bitcast<uint32_t>((h - off) * d2);
-    };
     auto build_b = [&](const Raw &rw, half8_t (&bv)[2][TN]) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const half2_t d2 = bitcast<half2_t>(__builtin_amdgcn_perm(rw.dd[j], rw.dd[j], 0x01000100u));
+            Q4Scale<XT> sc;
+            sc.set(rw.dd[j]);
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
                 uint4_t r;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) r[u] = dq2(rw.qd[j][2 * ks + 1], rw.qd[j][2 * ks], u, d2);
+                for (int u = 0; u < 4; ++u)
+                    r[u] = sc.weights(and_or(__builtin_amdgcn_perm(rw.qd[j][2 * ks + 1], rw.qd[j][2 * ks], bsel[u]),
+                                             nib_mask, exp_bits));
                 bv[ks][j] = bitcast<half8_t>(r);
             }
         }
@@ -238,25 +241,23 @@ q4_gemm7_kernel(Gemm7Args a) {
     auto step = [&](auto with_copies, int s_a, int as_, int s_r, const half8_t (&A)[2][TM],
                     half8_t (&An)[2][TM], const half8_t (&B)[2][TN], half8_t (&Bn)[2][TN], const Raw &rc,
                     Raw &rn, int k_read, int a_slot, int a_t) {
-#pragma clang fp contract(off)
-        const half2_t off = {(_Float16)1032.0f, (_Float16)72.0f};
-        half2_t d2[TN];
+        Q4Scale<XT> sc[TN];
         uint32_t xw[16];
         uint4_t bb[2 * TN];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int idx = 0; idx < NMF; ++idx) {
             const int ks = idx / (TM * TN), i = (idx / TN) % TM, j = idx % TN;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[ks][i], B[ks][j], acc[i][j], 0, 0, 0);
+            acc[i][j] = mfma32<XT>(A[ks][i], B[ks][j], acc[i][j]);
             {
                 const int d = idx >> 1, unit = d >> 2, u = d & 3, uj = unit >> 1, uk = unit & 1;
                 if ((idx & 1) == 0) {
                     if ((idx & 15) == 0)
-                        d2[uj] = bitcast<half2_t>(__builtin_amdgcn_perm(rc.dd[uj], rc.dd[uj], 0x01000100u));
+                        sc[uj].set(rc.dd[uj]);
                     xw[d] = and_or(__builtin_amdgcn_perm(rc.qd[uj][2 * uk + 1], rc.qd[uj][2 * uk], bsel[u]),
                                    nib_mask, exp_bits);
                 } else {
-                    bb[unit][u] = bitcast<uint32_t>((bitcast<half2_t>(xw[d]) - off) * d2[uj]);
+                    bb[unit][u] = sc[uj].weights(xw[d]);
                     if (u == 3) Bn[uk][uj] = bitcast<half8_t>(bb[unit]);
                 }
             }
@@ -323,7 +324,7 @@ q4_gemm7_kernel(Gemm7Args a) {
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A0[ks][i], B0[ks][j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = mfma32<XT>(A0[ks][i], B0[ks][j], acc[i][j]);
     }
     wait_vmcnt<0>();
 
@@ -337,7 +338,7 @@ q4_gemm7_kernel(Gemm7Args a) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int m = m0 + i * 32 + 8 * (r >> 2) + rsub + (r & 3);
-                    if (m < a.M && n < a.N) a.Y[(int64_t)m * a.ldy + n] = (_Float16)acc[i][j][r];
+                    if (m < a.M && n < a.N) a.Y[(int64_t)m * a.ldy + n] = out16<XT>(acc[i][j][r]);
                 }
             }
         return;
@@ -361,6 +362,7 @@ q4_gemm7_kernel(Gemm7Args a) {
 // spaced a workgroup apart (all loads issued before the sums), non-temporal:
 // the partials are read once.
 constexpr int G7_RV = 4;
+template <int XT>
 __global__ void __launch_bounds__(256)
 q4_gemm7_reduce_kernel(Gemm7Args a) {
     constexpr int TILE = G7_BM * G7_BN;
@@ -396,12 +398,12 @@ q4_gemm7_reduce_kernel(Gemm7Args a) {
         if (n + 3 < a.N && (a.ldy & 3) == 0 && ((uintptr_t)a.Y & 7) == 0) {
             half4_t h;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) h[c] = (_Float16)sum[u][c];
+            for (int c = 0; c < 4; ++c) h[c] = out16<XT>(sum[u][c]);
             *(half4_t *)(a.Y + (int64_t)m * a.ldy + n) = h;
         } else {
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                if (n + c < a.N) a.Y[(int64_t)m * a.ldy + n + c] = (_Float16)sum[u][c];
+                if (n + c < a.N) a.Y[(int64_t)m * a.ldy + n + c] = out16<XT>(sum[u][c]);
         }
     }
 }
@@ -432,7 +434,8 @@ bool gemm7_supported(const _Float16 *X, int64_t ldx, const uint8_t *W, int64_t M
            (K / QK) * N * BLOCK_BYTES < ((int64_t)1 << 31);
 }
 
-hipError_t launch_gemm7(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
+template <int XT>
+static hipError_t launch_gemm7_t(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
                         int64_t ldy, int M, int K, int N, void *ws, hipStream_t s) {
     Gemm7Args a;
     a.X = X; a.ldx = ldx; a.W = W; a.Y = Y; a.ldy = ldy;
@@ -451,19 +454,25 @@ hipError_t launch_gemm7(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float
     if (e != hipSuccess) return e;
     const uint64_t bit = 1ull << (dev & 63);
     if (!(done.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void *)q4_gemm7_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+        e = hipFuncSetAttribute((const void *)q4_gemm7_kernel<XT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)G7_LDS);
         if (e != hipSuccess) return e;
         done.fetch_or(bit, std::memory_order_acq_rel);
     }
     const int ntiles = a.tiles_m * a.tiles_n;
-    hipLaunchKernelGGL(q4_gemm7_kernel, dim3(ntiles, 1, a.S), dim3(256), G7_LDS, s, a);
+    hipLaunchKernelGGL(q4_gemm7_kernel<XT>, dim3(ntiles, 1, a.S), dim3(256), G7_LDS, s, a);
     if (a.S > 1) {
         const int64_t n4 = (int64_t)ntiles * (G7_BM * G7_BN / 4);
-        hipLaunchKernelGGL(q4_gemm7_reduce_kernel, dim3((unsigned)((n4 + 256 * G7_RV - 1) / (256 * G7_RV))),
+        hipLaunchKernelGGL(q4_gemm7_reduce_kernel<XT>, dim3((unsigned)((n4 + 256 * G7_RV - 1) / (256 * G7_RV))),
                            dim3(256), 0, s, a);
     }
     return hipGetLastError();
+}
+
+hipError_t launch_gemm7(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
+                        int64_t ldy, int M, int K, int N, int x_dt, void *ws, hipStream_t s) {
+    return x_dt == DT_BF16 ? launch_gemm7_t<DT_BF16>(X, ldx, W, Y, ldy, M, K, N, ws, s)
+                           : launch_gemm7_t<DT_F16>(X, ldx, W, Y, ldy, M, K, N, ws, s);
 }
 
 }  // namespace mcq4

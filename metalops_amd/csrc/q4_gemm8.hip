@@ -72,6 +72,7 @@ constexpr size_t g8_lds(int cw) {
 }
 static_assert(g8_lds(1) <= 160 * 1024 && g8_lds(2) <= 160 * 1024, "LDS budget: one workgroup per CU");
 
+template <int XT>
 __global__ void __launch_bounds__(64 * G8_PH * G8_CW, 1)
 q4_gemm8_kernel(Gemm6Args a) {
     constexpr int CW = G8_CW;
@@ -200,12 +201,6 @@ q4_gemm8_kernel(Gemm6Args a) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) bsel[u] = (uint32_t)(q_b + u) * 0x00010001u + 0x0C000C00u;
     const uint32_t nib_mask = opaque_sgpr(0x00F0000Fu), exp_bits = opaque_vgpr(0x54006400u);
-    auto dq2 = [&](uint32_t hi_w, uint32_t lo_w, int u, half2_t d2) {
-#pragma clang fp contract(off)
-        const half2_t off = {(_Float16)1032.0f, (_Float16)72.0f};
-        const half2_t h = bitcast<half2_t>(and_or(__builtin_amdgcn_perm(hi_w, lo_w, bsel[u]), nib_mask, exp_bits));
-        return bitcast<uint32_t>((h - off) * d2);
-    };
     auto load_b = [&](int s, half8_t (&bv)[2][TN]) {
         const lds_u8 *Rs = lds_ptr(lds_addr(ring + (s % G8_RAW_N) * RAW_SLOT));
 #pragma unroll
@@ -215,12 +210,14 @@ q4_gemm8_kernel(Gemm6Args a) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) qd[t] = qp[t];
             const uint32_t dd = *(const lds_u16 *)(Rs + d_off + j * 32 * 18);
-            const half2_t d2 = bitcast<half2_t>(__builtin_amdgcn_perm(dd, dd, 0x01000100u));
+            Q4Scale<XT> sc;
+            sc.set(dd);
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
                 uint4_t r;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) r[u] = dq2(qd[2 * ks + 1], qd[2 * ks], u, d2);
+                for (int u = 0; u < 4; ++u)
+                    r[u] = sc.weights(and_or(__builtin_amdgcn_perm(qd[2 * ks + 1], qd[2 * ks], bsel[u]), nib_mask, exp_bits));
                 bv[ks][j] = bitcast<half8_t>(r);
             }
         }
@@ -244,7 +241,6 @@ q4_gemm8_kernel(Gemm6Args a) {
     static_assert(NMF == 8 * TN, "one B dword per MFMA");
     half8_t A[2][TM];
     auto stage = [&](int cs, const half8_t (&B)[2][TN], int s_next, half8_t (&Bn)[2][TN]) {
-#pragma clang fp contract(off)
         const lds_u8 *Rs = lds_ptr(lds_addr(ring + (s_next % G8_RAW_N) * RAW_SLOT));
         uint32_t qd[TN][4], dd[TN];
 #pragma unroll
@@ -254,25 +250,24 @@ q4_gemm8_kernel(Gemm6Args a) {
             for (int t = 0; t < 4; ++t) qd[j][t] = qp[t];
             dd[j] = *(const lds_u16 *)(Rs + d_off + j * 32 * 18);
         }
-        const half2_t off = {(_Float16)1032.0f, (_Float16)72.0f};
-        half2_t d2[TN];
+        Q4Scale<XT> sc[TN];
         uint32_t xw[NMF];
         uint4_t bb[2 * TN];
         auto first = [&](int d) {
             const int unit = d >> 2, u = d & 3, uj = unit >> 1, uk = unit & 1;
-            if (u == 0 && uk == 0) d2[uj] = bitcast<half2_t>(__builtin_amdgcn_perm(dd[uj], dd[uj], 0x01000100u));
+            if (u == 0 && uk == 0) sc[uj].set(dd[uj]);
             xw[d] = and_or(__builtin_amdgcn_perm(qd[uj][2 * uk + 1], qd[uj][2 * uk], bsel[u]), nib_mask, exp_bits);
         };
         auto second = [&](int d) {
             const int unit = d >> 2, u = d & 3, uj = unit >> 1, uk = unit & 1;
-            bb[unit][u] = bitcast<uint32_t>((bitcast<half2_t>(xw[d]) - off) * d2[uj]);
+            bb[unit][u] = sc[uj].weights(xw[d]);
             if (u == 3) Bn[uk][uj] = bitcast<half8_t>(bb[unit]);
         };
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int idx = 0; idx < NMF; ++idx) {
             const int ks = idx / (TM * TN), i = (idx / TN) % TM, j = idx % TN;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[ks][i], B[ks][j], acc[i][j], 0, 0, 0);
+            acc[i][j] = mfma32<XT>(A[ks][i], B[ks][j], acc[i][j]);
             if (j == TN - 1) A[ks][i] = read_a1(s_next, ks, i);
             if ((idx & 1) == 1 && (idx >> 1) < GROUP) issue_one(cs, idx >> 1);
             if (idx >= 2) second(idx - 2);
@@ -331,7 +326,7 @@ q4_gemm8_kernel(Gemm6Args a) {
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[ks][i], B0[ks][j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = mfma32<XT>(A[ks][i], B0[ks][j], acc[i][j]);
     }
     wait_vmcnt<0>();
     lds_barrier();                                // every copy landed; LDS free for the phase sum
@@ -394,7 +389,7 @@ q4_gemm8_kernel(Gemm6Args a) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = m0 + rsub + 8 * (r >> 2) + (r & 3);
-                if (m < a.M) a.Y[(int64_t)m * a.ldy + n] = (_Float16)fin[j][r];
+                if (m < a.M) a.Y[(int64_t)m * a.ldy + n] = out16<XT>(fin[j][r]);
             }
         }
         return;
@@ -436,7 +431,7 @@ q4_gemm8_kernel(Gemm6Args a) {
 #pragma unroll 1
         for (int v = tid; v < TILE; v += 64 * NW) {
             const int m = min(m0 + v / G8_BN, a.M - 1), n = n0 + v % G8_BN;
-            other[v] = q4_dot_range(a.X + (int64_t)m * a.ldx, a.W, a.N, n, o_lo, o_hi);
+            other[v] = q4_dot_range<XT == DT_BF16>(a.X + (int64_t)m * a.ldx, a.W, a.N, n, o_lo, o_hi);
         }
         wait_vmcnt<0>();
         __syncthreads();
@@ -451,7 +446,7 @@ q4_gemm8_kernel(Gemm6Args a) {
         for (int r = 0; r < 16; ++r) {
             const int m = m0 + rsub + 8 * (r >> 2) + (r & 3), n = n0 + nl;
             const float v = z == 0 ? fin[j][r] + o[r] : o[r] + fin[j][r];   // p0 + p1 in split order
-            if (m < a.M) a.Y[(int64_t)m * a.ldy + n] = (_Float16)v;
+            if (m < a.M) a.Y[(int64_t)m * a.ldy + n] = out16<XT>(v);
         }
     }
 }
@@ -492,7 +487,8 @@ size_t gemm8_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     return COUNTER_BYTES + (size_t)t * 2 * G8_BM * G8_BN * sizeof(float);
 }
 
-hipError_t launch_gemm8(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
+template <int XT>
+static hipError_t launch_gemm8_t(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
                         int64_t ldy, int M, int K, int N, void *ws, hipStream_t s) {
     if (!gemm8_supported(X, ldx, W, M, K, N)) return hipErrorInvalidValue;
     Gemm6Args a;
@@ -514,15 +510,21 @@ hipError_t launch_gemm8(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float
     if (e != hipSuccess) return e;
     const uint64_t bit = 1ull << (dev & 63);
     if (!(done.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void *)q4_gemm8_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+        e = hipFuncSetAttribute((const void *)q4_gemm8_kernel<XT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)g8_lds(G8_CW));
         if (e != hipSuccess) return e;
         done.fetch_or(bit, std::memory_order_acq_rel);
     }
     const int ntiles = a.tiles_m * a.tiles_n;
     const int gx = a.S == 2 ? (ntiles + 7) / 8 * 8 : ntiles;
-    hipLaunchKernelGGL(q4_gemm8_kernel, dim3(gx, 1, a.S), dim3(64 * G8_PH * G8_CW), g8_lds(G8_CW), s, a);
+    hipLaunchKernelGGL(q4_gemm8_kernel<XT>, dim3(gx, 1, a.S), dim3(64 * G8_PH * G8_CW), g8_lds(G8_CW), s, a);
     return hipGetLastError();
+}
+
+hipError_t launch_gemm8(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
+                        int64_t ldy, int M, int K, int N, int x_dt, void *ws, hipStream_t s) {
+    return x_dt == DT_BF16 ? launch_gemm8_t<DT_BF16>(X, ldx, W, Y, ldy, M, K, N, ws, s)
+                           : launch_gemm8_t<DT_F16>(X, ldx, W, Y, ldy, M, K, N, ws, s);
 }
 
 }  // namespace mcq4

@@ -14,15 +14,11 @@
 // 16 of INT8.
 #pragma once
 
-#include "i4_common.h"
+#include "q4_prefill.h"
 
 namespace mcq4 {
 
 enum : int { WX_Q4 = 0, WX_I4 = 1, WX_I8 = 2 };
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float float2_t __attribute__((ext_vector_type(2)));
 
 struct WxArgs {
     const void *X;
@@ -242,10 +238,7 @@ __device__ __forceinline__ void wx_operands(const WxRaw<WT, TN> &r, int j, int s
 
 template <int XT>
 __device__ __forceinline__ float16_t wx_mfma(uint4_t a, uint4_t b, float16_t c) {
-    if constexpr (XT == DT_BF16)
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(bitcast<bf16x8_t>(a), bitcast<bf16x8_t>(b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(bitcast<half8_t>(a), bitcast<half8_t>(b), c, 0, 0, 0);
+    return mfma32<XT>(bitcast<half8_t>(a), bitcast<half8_t>(b), c);
 }
 
 __device__ __forceinline__ float wx_activate(float y, int act) {

@@ -214,11 +214,11 @@ def matmul_ggml_q4_0(X: torch.Tensor, W_blocks: torch.Tensor) -> torch.Tensor:
         x = X if (X.stride(1) == 1 and X.stride(0) >= K) else X.contiguous()
         code = _DTYPE_CODES[x.dtype]
         need = int(_lib.lib.mcq4_matmul_q4_0_workspace_bytes(M, K, N, code))
-        ws_ptr, ws_bytes = None, 0
+        ws, ws_ptr, ws_bytes = None, None, 0
         if need:
             ws = _workspace.get(x.device, stream, need)
             ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
-        with torch.cuda.device(x.device):
+        with torch.cuda.device(x.device), _workspace.guard(ws, stream):
             _lib.check(_lib.lib.mcq4_matmul_q4_0(x.data_ptr(), code, x.stride(0), w.data_ptr(), Y.data_ptr(), N, M, K,
                                                  N, ws_ptr, ws_bytes, stream),
                        "mcq4_matmul_q4_0")
