@@ -44,6 +44,9 @@ hipError_t q4_gemm6_split_fallbacks(uint64_t *count, bool reset);
 hipError_t i4_gemv_split_fallbacks(uint64_t *count, bool reset);
 hipError_t i4_gemv1_split_fallbacks(uint64_t *count, bool reset);
 hipError_t i4_gemm6_split_fallbacks(uint64_t *count, bool reset);
+size_t gemv_span_bf16_workspace_bytes(int64_t M, int64_t K, int64_t N);
+hipError_t launch_gemv_span_bf16(const void *X, int64_t ldx, const uint8_t *W, void *Y, int64_t ldy, int64_t M, int64_t K,
+                                 int64_t N, void *ws, size_t ws_bytes, bool *done, hipStream_t s);
 hipError_t q4_gemv_span_split_fallbacks(uint64_t *count, bool reset);
 hipError_t q4_gemm8_split_fallbacks(uint64_t *count, bool reset);
 bool gemv_dma_supported(const _Float16 *X, const uint8_t *W, int64_t K, int64_t N);
@@ -273,7 +276,8 @@ size_t mcq4_matmul_q4_0_workspace_bytes(int64_t M, int64_t K, int64_t N, int x_d
     if (x_dtype == MCQ4_DTYPE_F16) return mcq4_matmul_workspace_bytes(M, K, N);
     if (M <= 0 || K <= 0 || N <= 0 || K % 32) return 0;
     const size_t any = mcq4::wx_workspace_bytes(mcq4::WX_Q4, x_dtype, M, K, N);
-    return x_dtype == MCQ4_DTYPE_BF16 && M > 64 ? std::max(any, prefill_ws_bytes(M, K, N)) : any;
+    if (x_dtype != MCQ4_DTYPE_BF16) return any;
+    return std::max(any, M > 64 ? prefill_ws_bytes(M, K, N) : mcq4::gemv_span_bf16_workspace_bytes(M, K, N));
 }
 
 int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, int64_t ldy,
@@ -382,6 +386,11 @@ int mcq4_matmul_q4_0(const void *X, int x_dtype, int64_t ldx, const uint8_t *W, 
                 default: break;
             }
         }
+    }
+    if (x_dtype == MCQ4_DTYPE_BF16 && M <= 16) {
+        bool done = false;
+        const hipError_t e = mcq4::launch_gemv_span_bf16(X, ldx, W, Y, ldy, M, K, N, workspace, workspace_bytes, &done, (hipStream_t)stream);
+        if (done || e != hipSuccess) return hip_status(e, "matmul launch");
     }
     const mcq4::WxCall c = {mcq4::WX_Q4, x_dtype, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32};
     return hip_status(mcq4::launch_wx(c, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");

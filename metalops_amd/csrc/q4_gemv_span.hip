@@ -46,7 +46,7 @@
 #include <atomic>
 #include <type_traits>
 
-#include "q4_common.h"
+#include "q4_prefill.h"
 
 namespace mcq4 {
 
@@ -102,13 +102,18 @@ struct GemvSpanArgs {
     uint32_t foreign = 0;                    // splits treated as run on another XCD (test switch)
 };
 
-template <int GR, bool SPLIT>
+// XT = DT_BF16: bf16 activations (X and Y addressed as _Float16).  Their weights are
+// rounded to bf16 before the product, so the scale goes into the B operand
+// (exact products in fp32, one packed conversion: about two VALU instructions per
+// weight against 0.75) and the MFMA accumulates over the rows.
+template <int GR, bool SPLIT, int XT = DT_F16>
 __global__ void __launch_bounds__(GS_NW * 64)
 q4_gemv_span_kernel(GemvSpanArgs a) {
     static_assert(GR == 1 || GR == 4 || GR == 8 || GR == 16, "row groups");
     constexpr int NA = GR <= 4 ? 1 : GR / 4;     // accumulators per group
     constexpr int IS = GR == 1 ? 0 : 16 / GR;    // accumulator i is MFMA result element i * IS
-    constexpr bool HOIST = GR == 1;              // -S for all 8 rows up front (else per row pair)
+    constexpr bool BF = XT == DT_BF16;
+    constexpr bool HOIST = GR == 1 && !BF;       // -S for all 8 rows up front (else per row pair)
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int nb = a.nb, ngt = a.groups, M = a.M;
     const uint32_t grow = a.grow;
@@ -151,7 +156,8 @@ q4_gemv_span_kernel(GemvSpanArgs a) {
         // grid is fixed, groups <= 1024, so wg * groups fits 32 bits).
         const int wg = ((int)blockIdx.x & 7) * (GS_GRID / 8) + ((int)blockIdx.x >> 3);
         g0 = (wg * ngt) >> 8;
-        ng = (((wg + 1) * ngt) >> 8) - g0;                         // 1..GS_NGMAX
+        ng = (((wg + 1) * ngt) >> 8) - g0;                         // 1..GS_NGMAX (0 with fewer groups than workgroups)
+        if (BF && ng == 0) return;
         static_assert(GS_GRID == 256, "span bounds by a shift of 8");
     }
     const int row0 = kb0 + wave * GS_B;
@@ -167,7 +173,7 @@ q4_gemv_span_kernel(GemvSpanArgs a) {
     // for an odd one (whose first word is the nibble bytes exactly) -- and the scale
     // comes from the two words instead of a read of its own.  The B operand is
     // unchanged: the second word only feeds byte 3 of w8, which the masks drop.
-    const uint32_t q1off = GR == 1 && g == 0 && (c & 1) ? doff - 2 : qal + 4;
+    const uint32_t q1off = GR == 1 && !BF && g == 0 && (c & 1) ? doff - 2 : qal + 4;
     const uint32_t dsel = (c & 1) ? 0x0C0C0706u : 0x0C0C0100u;     // scale bytes of (q1, q0)
     const uint32_t e1024 = opaque_vgpr(0x64006400u), e64 = opaque_vgpr(0x54005400u);
     const uint32_t mlo = opaque_sgpr(0x000F000Fu), mhi = opaque_sgpr(0x00F000F0u);
@@ -180,6 +186,9 @@ q4_gemv_span_kernel(GemvSpanArgs a) {
     for (int grp = 0; grp < GS_NGMAX; ++grp)
 #pragma unroll
         for (int i = 0; i < NA; ++i) acc[grp][i] = 0.f;
+    float4_t accm[BF ? GS_NGMAX : 1];            // bf16: the MFMA accumulators
+#pragma unroll
+    for (int grp = 0; grp < (BF ? GS_NGMAX : 1); ++grp) accm[grp] = z;
     // One templated body per span width ng (the copy addresses divide by the
     // constant 18 ng, and the waits count its copies).
     auto item = [&](auto NGc) {
@@ -252,11 +261,51 @@ q4_gemv_span_kernel(GemvSpanArgs a) {
                     const uint32_t ro = (R0 + v) * rowb + grp * 288;
                     q0[v][grp] = *(const lds_u32 *)(lds_ptr(vq0) + ro);
                     q1[v][grp] = *(const lds_u32 *)(lds_ptr(vq1) + ro);
-                    if constexpr (GR == 1)
+                    if constexpr (GR == 1 && !BF)
                         dh[v][grp] = bitcast<_Float16>((uint16_t)__builtin_amdgcn_perm(q1[v][grp], q0[v][grp], dsel));
                     else
                         dh[v][grp] = bitcast<_Float16>(*(const lds_u16 *)(lds_ptr(vd) + ro));
                 }
+            if constexpr (BF) {
+                // (1024 + q) d - 1032 d and (64 + q) d - 72 d, one mixed-precision fma
+                // each, exact in fp32 for a finite d; otherwise q - 8 first, so an
+                // infinite d gives the signed infinities of (q - 8) d.
+                auto rows_bf = [&](auto fin) {
+#pragma unroll
+                    for (int v = 0; v < NR; ++v) {
+                        if (R0 + v >= rows) break;
+#pragma unroll
+                        for (int grp = 0; grp < NG; ++grp) {
+                            const uint32_t w = __builtin_amdgcn_alignbit(q1[v][grp], q0[v][grp], qsh);
+                            const uint32_t w8 = __builtin_amdgcn_alignbit(q1[v][grp], q0[v][grp], qsh + 8);
+                            const uint4_t bq = {and_or(w, mlo, e1024), and_or(w, mhi, e64), and_or(w8, mlo, e1024),
+                                                and_or(w8, mhi, e64)};
+                            const float d = (float)dh[v][grp];
+                            const float cc[2] = {-1032.0f * d, -72.0f * d};
+                            uint4_t b;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                half2_t p = bitcast<half2_t>(bq[i]);
+                                if constexpr (!decltype(fin)::value)
+                                    p -= (i & 1) ? half2_t{(_Float16)72.0f, (_Float16)72.0f} : half2_t{(_Float16)1032.0f, (_Float16)1032.0f};
+                                const float add = decltype(fin)::value ? cc[i & 1] : 0.0f;
+                                const float2_t f = {__builtin_fmaf((float)p[0], d, add), __builtin_fmaf((float)p[1], d, add)};
+                                b[i] = bitcast<uint32_t>(__builtin_convertvector(f, bf16x2_t));
+                            }
+                            accm[grp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8_t>(xq[R0 + v]), bitcast<bf16x8_t>(b),
+                                                                               accm[grp], 0, 0, 0);
+                        }
+                    }
+                };
+                float chk = 0.f;                 // NaN once a scale is not finite
+#pragma unroll
+                for (int v = 0; v < NR; ++v)
+#pragma unroll
+                    for (int grp = 0; grp < NG; ++grp) chk = __builtin_fmaf((float)dh[v][grp], 0.0f, chk);
+                if (__builtin_expect(__any(chk != chk), 0)) rows_bf(std::false_type{});
+                else rows_bf(std::true_type{});
+                return;
+            }
             float4_t ns[NR];
 #pragma unroll
             for (int v = 0; v < NR; ++v) {
@@ -309,6 +358,12 @@ q4_gemv_span_kernel(GemvSpanArgs a) {
         // Every LDS read of the slot has returned before it holds the partials.
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
+    if constexpr (BF) {
+#pragma unroll
+        for (int grp = 0; grp < GS_NGMAX; ++grp)
+#pragma unroll
+            for (int i = 0; i < NA; ++i) acc[grp][i] = accm[grp][i * IS];
+    }
     // Partials into this wave's slot: [output row][64 columns] floats.  Accumulator
     // i of lane (c, g) is output row g GR/4 + i (row 0 for every lane at M == 1).
     float *mine = (float *)slot;
@@ -329,7 +384,7 @@ q4_gemv_span_kernel(GemvSpanArgs a) {
         const float *p = (const float *)(smem + XS) + row * 64 + col;
 #pragma unroll
         for (int w = 0; w < GS_NW; ++w) s += p[w * (GS_SLOT / 4)];
-        if constexpr (!SPLIT) Y[(int64_t)row * ldy + n] = (_Float16)s;
+        if constexpr (!SPLIT) Y[(int64_t)row * ldy + n] = out16<XT>(s);
     }
     if constexpr (SPLIT) {
         // Split 0 sums the S partials in split order: its own from registers, the
@@ -384,10 +439,10 @@ q4_gemv_span_kernel(GemvSpanArgs a) {
             float pv;
             if (q == sp && ((local >> q) & 1)) pv = s;
             else if ((local >> q) & 1) pv = load_l2_f32(a.part, (int)((((int64_t)q * M + row) * N + n) * 4));
-            else pv = q4_dot_range(X + (int64_t)row * ldx, W, N, n, min(q * a.bps, nb), min((q + 1) * a.bps, nb));
+            else pv = q4_dot_range<BF>(X + (int64_t)row * ldx, W, N, n, min(q * a.bps, nb), min((q + 1) * a.bps, nb));
             tot += pv;
         }
-        Y[(int64_t)row * ldy + n] = (_Float16)tot;
+        Y[(int64_t)row * ldy + n] = out16<XT>(tot);
     }
 }
 
@@ -403,7 +458,7 @@ bool gemv_span_supported(const _Float16 *X, int64_t ldx, const uint8_t *W, int64
            (M == 1 || ldx % 8 == 0) && N * 18 * 8 < ((int64_t)1 << 31);
 }
 
-template <int GR, bool SPLIT>
+template <int GR, bool SPLIT, int XT = DT_F16>
 static hipError_t launch_span_gr(const GemvSpanArgs &a, dim3 grid, hipStream_t s) {
     const size_t lds = (GR == 1 ? GS_XS : 0) + (size_t)GS_NW * GS_SLOT + GS_PAD;
     static std::atomic<uint64_t> done{0};
@@ -412,12 +467,12 @@ static hipError_t launch_span_gr(const GemvSpanArgs &a, dim3 grid, hipStream_t s
     if (e != hipSuccess) return e;
     const uint64_t bit = 1ull << (dev & 63);
     if (!(done.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void *)q4_gemv_span_kernel<GR, SPLIT>,
+        e = hipFuncSetAttribute((const void *)q4_gemv_span_kernel<GR, SPLIT, XT>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return e;
         done.fetch_or(bit, std::memory_order_acq_rel);
     }
-    hipLaunchKernelGGL((q4_gemv_span_kernel<GR, SPLIT>), grid, dim3(GS_NW * 64), lds, s, a);
+    hipLaunchKernelGGL((q4_gemv_span_kernel<GR, SPLIT, XT>), grid, dim3(GS_NW * 64), lds, s, a);
     return hipGetLastError();
 }
 
@@ -501,6 +556,60 @@ hipError_t launch_gemv_span_split(const _Float16 *X, int64_t ldx, const uint8_t 
     // 11.3-11.8 against 10.8-11.0 us, same box; equal at M = 2).
     if (M <= 8) return launch_span_gr<8, true>(a, grid, s);
     return launch_span_gr<16, true>(a, grid, s);
+}
+
+// bf16 activations, 1 <= M <= 16: the span form for any N % 16 == 0 up to 16384 at
+// K <= 4096 (below 4096 columns one 16-column group per workgroup, the rest idle),
+// the split form where it keeps its waves busy.
+static bool span_bf16_fits(const void *X, int64_t ldx, const uint8_t *W, int64_t M, int64_t K, int64_t N) {
+    return M >= 1 && M <= 16 && N % 16 == 0 && N / 16 <= GS_GRID * GS_NGMAX && K >= QK && K <= GS_NW * GS_B * QK &&
+           ((uintptr_t)W % 16) == 0 && ((uintptr_t)X % 16) == 0 && (M == 1 || ldx % 8 == 0);
+}
+static bool span_split_bf16_shape(int64_t M, int64_t K, int64_t N) {
+    if (M < 1 || M > 16 || N % 64 || N < 64 || N > 4096 || K <= GS_NW * GS_B * QK) return false;
+    const SpanSplitPlan p = span_split_plan(K, N);
+    return p.S >= 2 && p.bps <= GS_NW * GS_B && K / QK >= (int64_t)64 * p.S;
+}
+
+size_t gemv_span_bf16_workspace_bytes(int64_t M, int64_t K, int64_t N) {
+    if (!span_split_bf16_shape(M, K, N)) return 0;
+    const SpanSplitPlan p = span_split_plan(K, N);
+    return COUNTER_BYTES + (size_t)p.S * M * N * sizeof(float) + (size_t)(N / 64) * p.S * sizeof(uint32_t);
+}
+
+// *done = false: neither form takes the call (or the split form has no workspace).
+hipError_t launch_gemv_span_bf16(const void *X, int64_t ldx, const uint8_t *W, void *Y, int64_t ldy, int64_t M, int64_t K,
+                                 int64_t N, void *ws, size_t ws_bytes, bool *done, hipStream_t s) {
+    GemvSpanArgs a;
+    a.X = (const _Float16 *)X; a.W = W; a.Y = (_Float16 *)Y;
+    a.ldx = ldx; a.ldy = ldy;
+    a.M = (int)M;
+    a.nb = (int)(K / QK);
+    a.groups = (int)(N / 16);
+    a.grow = (uint32_t)N * BLOCK_BYTES;
+    *done = true;
+    if (span_bf16_fits(X, ldx, W, M, K, N)) {
+        const dim3 grid(GS_GRID);
+        if (M == 1) return launch_span_gr<1, false, DT_BF16>(a, grid, s);
+        if (M <= 4) return launch_span_gr<4, false, DT_BF16>(a, grid, s);
+        if (M <= 8) return launch_span_gr<8, false, DT_BF16>(a, grid, s);
+        return launch_span_gr<16, false, DT_BF16>(a, grid, s);
+    }
+    if (span_split_bf16_shape(M, K, N) && ((uintptr_t)W % 16) == 0 && ((uintptr_t)X % 16) == 0 && ldx % 8 == 0 &&
+        !opt_is("MCQ4_XCD_LOCAL", '0') && ws && ws_bytes >= gemv_span_bf16_workspace_bytes(M, K, N)) {
+        const SpanSplitPlan p = span_split_plan(K, N);
+        a.S = p.S;
+        a.bps = p.bps;
+        a.part = (float *)((char *)ws + COUNTER_BYTES);
+        a.flags = (uint32_t *)(a.part + (int64_t)p.S * M * N);
+        a.spin = split_spin();
+        a.foreign = split_foreign_mask();
+        const dim3 grid(p.gx, p.S);
+        if (M <= 8) return launch_span_gr<8, true, DT_BF16>(a, grid, s);
+        return launch_span_gr<16, true, DT_BF16>(a, grid, s);
+    }
+    *done = false;
+    return hipSuccess;
 }
 
 }  // namespace mcq4

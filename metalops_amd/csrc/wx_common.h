@@ -14,6 +14,8 @@
 // 16 of INT8.
 #pragma once
 
+#include <type_traits>
+
 #include "q4_prefill.h"
 
 namespace mcq4 {
@@ -29,7 +31,9 @@ struct WxArgs {
     void *Y;
     int64_t ldy;
     int M, K, N;
-    int spg;                     // K steps of 32 per group (INT4, INT8)
+    // Group of K step k = mulhi(k, spg_mul) + (k & spg_one): spg_mul = ceil(2^32 / K
+    // steps per group), or 0 with one group or one step per group (spg_one = ~0).
+    uint32_t spg_mul, spg_one;
     int act;                     // ACT_*
     int S;                       // K splits (grid.z)
     float *part;                 // [S][M][ldp] fp32 partials when S > 1
@@ -107,9 +111,9 @@ __device__ __forceinline__ WxLane<WT, TN> wx_lane(const WxArgs &a, int n0, int l
     return L;
 }
 
-template <int TN>
-__device__ __forceinline__ void wx_load_sz(const void *p, int64_t row, int dt, int n, uint32_t (&out)[TN]) {
-    if (dt == DT_F32) {
+template <int TN, bool SZ32>
+__device__ __forceinline__ void wx_load_sz(const void *p, int64_t row, int n, uint32_t (&out)[TN]) {
+    if constexpr (SZ32) {
         const float *q = (const float *)p + row;
         if constexpr (TN == 2) {
             const u32x2 v = load_u<u32x2>(q + n);
@@ -132,11 +136,15 @@ __device__ __forceinline__ void wx_load_sz(const void *p, int64_t row, int dt, i
     }
 }
 
-// Loads K step `kb` (group `grp`).  TAIL: rows past K are clamped to the last
+// Group of K step k: exact for k and steps per group below 2^16 (wx_supported).
+__device__ __forceinline__ int wx_group(const WxArgs &a, int k) {
+    return (int)(__umulhi((uint32_t)k, a.spg_mul) + ((uint32_t)k & a.spg_one));
+}
+
+// Loads K step `kb`.  TAIL: rows past K are clamped to the last
 // one (wx_dequant zeroes their weights).
-template <int WT, int TN, bool TAIL>
-__device__ __forceinline__ void wx_load(WxRaw<WT, TN> &r, const WxArgs &a, const WxLane<WT, TN> &L, int kb, int grp,
-                                        int lane) {
+template <int WT, int TN, bool SZ32, bool TAIL>
+__device__ __forceinline__ void wx_load(WxRaw<WT, TN> &r, const WxArgs &a, const WxLane<WT, TN> &L, int kb, int lane) {
     if constexpr (WT == WX_Q4) {
         const uint8_t *base = a.W + ((int64_t)kb * a.N + L.n0) * BLOCK_BYTES;
         const int hi = lane >> 5;
@@ -160,42 +168,76 @@ __device__ __forceinline__ void wx_load(WxRaw<WT, TN> &r, const WxArgs &a, const
             if constexpr (TN == 2) r.q[i] = load_u<uint16_t>(p);
             else r.q[i] = load_u<uint32_t>(p);
         }
-        const int64_t row = (int64_t)grp * a.N;
-        wx_load_sz<TN>(a.scales, row, a.sz_dt, L.n[0], r.s);
-        wx_load_sz<TN>(a.zeros, row, a.sz_dt, L.n[0], r.z);
+        const int64_t row = (int64_t)wx_group(a, kb) * a.N;
+        wx_load_sz<TN, SZ32>(a.scales, row, L.n[0], r.s);
+        wx_load_sz<TN, SZ32>(a.zeros, row, L.n[0], r.z);
     }
 }
 
+// Both 16-bit readings and a select: a branch here would end the block that the
+// loads and MFMAs around it are scheduled in.
+template <bool SZ32>
 __device__ __forceinline__ float wx_sz_f32(uint32_t v, int dt) {
-    if (dt == DT_F32) return __uint_as_float(v);
-    if (dt == DT_F16) return (float)bitcast<_Float16>((uint16_t)v);
-    return bf16_bits_to_f32((uint16_t)v);
+    if constexpr (SZ32) return __uint_as_float(v);
+    const float h = (float)bitcast<_Float16>((uint16_t)v), b = __uint_as_float(v << 16);
+    return dt == DT_F16 ? h : b;
 }
 
-// The lane's 16 weights of tile j in fp32, in K order.
-// q4_0: v_perm_b32 puts a nibble byte into bytes 0 and 2 and v_and_or_b32 makes
-// it the fp16 pair {1024 + q0, 64 + q1}; minus {1032, 72} gives q - 8, and one
-// mixed-precision multiply each (q - 8) d, exact in fp32 (d has 11 significant
-// bits).  INT4 and INT8: (q - z) s in the reference's two fp32 roundings.
+// q4_0 weights come out of a dword of nibbles (elements e0..e7) in the pair order
+// [e0, e4, e1, e5, e2, e6, e3, e7]: two masks on the dword and on the dword
+// shifted by 8, no byte moves.  wx_order puts 16-bit activations in that order
+// (INT4 and INT8 keep the natural one); wx_slot is the element of slot s.
+template <int WT>
+__device__ __forceinline__ uint4_t wx_order(uint4_t x) {
+    if constexpr (WT == WX_Q4)
+        return uint4_t{__builtin_amdgcn_perm(x[2], x[0], 0x05040100u), __builtin_amdgcn_perm(x[2], x[0], 0x07060302u),
+                       __builtin_amdgcn_perm(x[3], x[1], 0x05040100u), __builtin_amdgcn_perm(x[3], x[1], 0x07060302u)};
+    else
+        return x;
+}
+template <int WT>
+constexpr int wx_slot(int s) {
+    return WT == WX_Q4 ? (s & ~7) + ((s & 7) >> 1) + 4 * (s & 1) : s;
+}
+
+// The fp16 pairs {1024 + e0, 1024 + e4}, {64 + e1, 64 + e5}, ... of a nibble dword, exact.
+__device__ __forceinline__ void q4_pairs(uint32_t w, uint32_t (&p)[4]) {
+    const uint32_t mlo = opaque_sgpr(0x000F000Fu), mhi = opaque_sgpr(0x00F000F0u);
+    const uint32_t e1024 = opaque_vgpr(0x64006400u), e64 = opaque_vgpr(0x54005400u);
+    p[0] = and_or(w, mlo, e1024);
+    p[1] = and_or(w, mhi, e64);
+    p[2] = and_or(w >> 8, mlo, e1024);
+    p[3] = and_or(w >> 8, mhi, e64);
+}
+
+// Whether a lane's block scale is infinite or NaN.
+__device__ __forceinline__ bool q4_scale_odd(uint16_t d) { return (d & 0x7C00u) == 0x7C00u; }
+
+// The lane's 16 weights of tile j in fp32, in slot order.
+// q4_0, FIN (every scale finite): (1024 + q) d - 1032 d and (64 + q) d - 72 d, one
+// mixed-precision fma each, exact in fp32 (d has 11 significant bits).  Without
+// FIN q - 8 first, so an infinite d gives the signed infinities of (q - 8) d.
+// INT4 and INT8: (q - z) s in the reference's two fp32 roundings.
 // TAIL: weights of rows past K are zero (`valid` = rows of the lane's 16 below K).
-template <int WT, int XT, int TN, bool TAIL>
+template <int WT, int XT, int TN, bool SZ32, bool TAIL, bool FIN>
 __device__ __forceinline__ void wx_values(const WxRaw<WT, TN> &r, int j, int sz_dt, int valid, float (&w)[16]) {
     if constexpr (WT == WX_Q4) {
-        const uint32_t nib_mask = opaque_sgpr(0x00F0000Fu), exp_bits = opaque_vgpr(0x54006400u);
         const float d = (float)bitcast<_Float16>(r.d[j]);
-        const half2_t off = {(_Float16)1032.0f, (_Float16)72.0f};
+        const float c[2] = {-1032.0f * d, -72.0f * d};
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
+            uint32_t p[4];
+            q4_pairs(r.q[j][h], p);
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const half2_t p = bitcast<half2_t>(and_or(__builtin_amdgcn_perm(0u, r.q[j][h], (uint32_t)b * 0x00010001u + 0x0C000C00u),
-                                                          nib_mask, exp_bits)) - off;
-                w[8 * h + 2 * b] = __builtin_fmaf((float)p[0], d, 0.0f);
-                w[8 * h + 2 * b + 1] = __builtin_fmaf((float)p[1], d, 0.0f);
+            for (int i = 0; i < 4; ++i) {
+                half2_t v = bitcast<half2_t>(p[i]);
+                if constexpr (!FIN) v -= (i & 1) ? half2_t{(_Float16)72.0f, (_Float16)72.0f} : half2_t{(_Float16)1032.0f, (_Float16)1032.0f};
+                w[8 * h + 2 * i] = __builtin_fmaf((float)v[0], d, FIN ? c[i & 1] : 0.0f);
+                w[8 * h + 2 * i + 1] = __builtin_fmaf((float)v[1], d, FIN ? c[i & 1] : 0.0f);
             }
         }
     } else {
-        const float s = wx_sz_f32(r.s[j], sz_dt), z = wx_sz_f32(r.z[j], sz_dt);
+        const float s = wx_sz_f32<SZ32>(r.s[j], sz_dt), z = wx_sz_f32<SZ32>(r.z[j], sz_dt);
         auto val = [&](float q) {
 #pragma clang fp contract(off)
             return (q - z) * s;
@@ -217,22 +259,45 @@ __device__ __forceinline__ void wx_values(const WxRaw<WT, TN> &r, int j, int sz_
     }
 }
 
-// The B operands of tile j for 16-bit activations: ops[ks] = K elements
-// 8 ks .. +7 of the lane's 16.
-template <int WT, int XT, int TN, bool TAIL>
+// The B operands of tile j for 16-bit activations: ops[ks] = slots 8 ks .. +7 of
+// the lane's 16.
+template <int WT, int XT, int TN, bool SZ32, bool TAIL, bool FIN>
 __device__ __forceinline__ void wx_operands(const WxRaw<WT, TN> &r, int j, int sz_dt, int valid, uint4_t (&ops)[2]) {
     if constexpr (WT == WX_Q4 && XT == DT_F16) {
+#pragma clang fp contract(off)
         const uint32_t dd = r.d[j];
         const half2_t d2 = bitcast<half2_t>(dd | (dd << 16));
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) ops[ks] = bitcast<uint4_t>(dequant8_nat(r.q[j][ks], d2));
+        for (int ks = 0; ks < 2; ++ks) {
+            uint32_t p[4];
+            q4_pairs(r.q[j][ks], p);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const half2_t off = (i & 1) ? half2_t{(_Float16)72.0f, (_Float16)72.0f} : half2_t{(_Float16)1032.0f, (_Float16)1032.0f};
+                ops[ks][i] = bitcast<uint32_t>((bitcast<half2_t>(p[i]) - off) * d2);
+            }
+        }
     } else {
         float w[16];
-        wx_values<WT, XT, TN, TAIL>(r, j, sz_dt, valid, w);
+        wx_values<WT, XT, TN, SZ32, TAIL, FIN>(r, j, sz_dt, valid, w);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int u = 0; u < 4; ++u) ops[ks][u] = pack2<XT>(w[8 * ks + 2 * u], w[8 * ks + 2 * u + 1]);
+    }
+}
+
+// body(FIN) with FIN = every lane's scales are finite (q4_0; always, otherwise).
+template <int WT, int XT, int TN, typename F>
+__device__ __forceinline__ void wx_if_finite(const uint16_t *d, F body) {
+    if constexpr (WT == WX_Q4 && XT != DT_F16) {
+        bool odd = false;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) odd |= q4_scale_odd(d[j]);
+        if (__builtin_expect(__any(odd), 0)) body(std::false_type{});
+        else body(std::true_type{});
+    } else {
+        body(std::true_type{});
     }
 }
 

@@ -18,13 +18,21 @@
 
 namespace mcq4 {
 
+#ifndef WS_NW_SET
 constexpr int WS_NW = 8;
+#else
+constexpr int WS_NW = WS_NW_SET;
+#endif
+#ifndef WS_TN_SET
+#define WS_TN_SET 2
+#endif
 
-template <int WT, int XT, int TM, int TN, bool ANY>
+template <int WT, int XT, int TM, int TN, bool SZ32, bool ANY>
 __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
     constexpr int ES = XT == DT_F32 ? 4 : 2;
     constexpr int XV = XT == DT_F32 ? 4 : 2;     // 16-byte activation loads per row tile and step
-    constexpr int PF = TM == 1 && XT != DT_F32 && WT == WX_Q4 ? 4 : 2;
+    // Ring slots: R - 1 K steps in flight beside the one in work.
+    constexpr int R = TM == 2 && (WT == WX_I8 || XT == DT_F32) ? 2 : 4;
     extern __shared__ __attribute__((aligned(16))) float red[];   // [waves][TM TN][16][64]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -42,11 +50,10 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
     struct Step {
         WxRaw<WT, TN> r;
         uint4_t x[TM][XV];
-    } ring[PF];
-    int kld = 0, grp = WT == WX_Q4 ? 0 : k_lo / a.spg, gcnt = WT == WX_Q4 ? 0 : k_lo % a.spg;
-    auto load = [&](Step &p) {
-        const int kb = k_lo + kld;
-        wx_load<WT, TN, ANY && WT != WX_Q4>(p.r, a, L, kb, grp, lane);
+    } ring[R];
+    auto load = [&](Step &p, int kk) {
+        const int kb = k_lo + min(kk, nk - 1);
+        wx_load<WT, TN, SZ32, ANY && WT != WX_Q4>(p.r, a, L, kb, lane);
         const int k = kb * 32 + 16 * lhi;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -55,10 +62,6 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
                 if constexpr (ANY) p.x[i][v] = wx_load_x_any<XT>(xrow[i], k + v * (16 / ES), a.K);
                 else p.x[i][v] = *(const uint4_t *)(xrow[i] + (int64_t)(k + v * (16 / ES)) * ES);
             }
-        if (kld + 1 < nk) {
-            ++kld;
-            if (WT != WX_Q4 && ++gcnt == a.spg) { gcnt = 0; ++grp; }
-        }
     };
 
     float16_t acc[TM][TN];
@@ -71,36 +74,52 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
 
     auto step = [&](Step &p, int kk) {
         const int valid = a.K - (k_lo + kk) * 32 - 16 * lhi;
+        if constexpr (XT != DT_F32) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            if constexpr (XT == DT_F32) {
-                float w[16];
-                wx_values<WT, XT, TN, ANY>(p.r, j, a.sz_dt, valid, w);
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int e = 0; e < 16; ++e)
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(p.x[i][e / 4][e % 4]), w[e], acc[i][j], 0, 0, 0);
-            } else {
-                uint4_t B[2];
-                wx_operands<WT, XT, TN, ANY>(p.r, j, a.sz_dt, valid, B);
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) acc[i][j] = wx_mfma<XT>(p.x[i][ks], B[ks], acc[i][j]);
-            }
+                for (int ks = 0; ks < 2; ++ks) p.x[i][ks] = wx_order<WT>(p.x[i][ks]);
         }
+        const uint16_t *d = nullptr;
+        if constexpr (WT == WX_Q4) d = p.r.d;
+        wx_if_finite<WT, XT, TN>(d, [&](auto fin) {
+            constexpr bool FIN = decltype(fin)::value;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                if constexpr (XT == DT_F32) {
+                    float w[16];
+                    wx_values<WT, XT, TN, SZ32, ANY, FIN>(p.r, j, a.sz_dt, valid, w);
+#pragma unroll
+                    for (int s = 0; s < 16; ++s) {
+                        const int e = wx_slot<WT>(s);
+#pragma unroll
+                        for (int i = 0; i < TM; ++i)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(p.x[i][e / 4][e % 4]), w[s], acc[i][j], 0, 0, 0);
+                    }
+                } else {
+                    uint4_t B[2];
+                    wx_operands<WT, XT, TN, SZ32, ANY, FIN>(p.r, j, a.sz_dt, valid, B);
+#pragma unroll
+                    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                        for (int i = 0; i < TM; ++i) acc[i][j] = wx_mfma<XT>(p.x[i][ks], B[ks], acc[i][j]);
+                }
+            }
+        });
     };
 
     if (nk > 0) {
+        // The load of step k + R - 1 goes into the slot that step k - 1 has left, so no
+        // value in flight is ever moved.
 #pragma unroll
-        for (int p = 0; p < PF; ++p) load(ring[p]);
-        for (int k0 = 0; k0 < nk; k0 += PF) {
+        for (int p = 0; p < R - 1; ++p) load(ring[p], p);
+        for (int k0 = 0; k0 < nk; k0 += R) {
 #pragma unroll
-            for (int p = 0; p < PF; ++p) {
+            for (int p = 0; p < R; ++p) {
                 if (k0 + p >= nk) break;
+                load(ring[(p + R - 1) % R], k0 + p + R - 1);
+                __builtin_amdgcn_sched_barrier(0);
                 step(ring[p], k0 + p);
-                load(ring[p]);
             }
         }
     }
@@ -131,36 +150,44 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
 }
 
 hipError_t launch_wx_reduce(const WxArgs &a, int x_dt, hipStream_t s);
+hipError_t launch_wx_gemv(const WxArgs &a, int x_dt, bool any, hipStream_t s);
 hipError_t launch_wx_gemm(WxArgs a, int wt, int x_dt, bool any, hipStream_t s);
 int wx_gemm_splits(int64_t M, int64_t K, int64_t N);
 
-template <int WT, int XT, int TM, int TN, bool ANY>
+template <int WT, int XT, int TM, int TN, bool SZ32, bool ANY>
 static hipError_t launch_wx_skinny_k(const WxArgs &a, hipStream_t s) {
     const size_t lds = (size_t)WS_NW * TM * TN * 1024 * sizeof(float);
     const dim3 grid((a.N + 32 * TN - 1) / (32 * TN), 1, a.S);
     if (lds > 64 * 1024)
-        if (hipError_t e = hipFuncSetAttribute((const void *)wx_skinny_kernel<WT, XT, TM, TN, ANY>,
+        if (hipError_t e = hipFuncSetAttribute((const void *)wx_skinny_kernel<WT, XT, TM, TN, SZ32, ANY>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
             return e;
-    hipLaunchKernelGGL((wx_skinny_kernel<WT, XT, TM, TN, ANY>), grid, dim3(WS_NW * 64), lds, s, a);
+    hipLaunchKernelGGL((wx_skinny_kernel<WT, XT, TM, TN, SZ32, ANY>), grid, dim3(WS_NW * 64), lds, s, a);
     return hipGetLastError();
 }
-template <int WT, int XT>
+template <int WT, int XT, bool SZ32>
 static hipError_t launch_wx_skinny_t(const WxArgs &a, bool any, hipStream_t s) {
-    constexpr int TN = 2;
-    if (a.M <= 32) return any ? launch_wx_skinny_k<WT, XT, 1, TN, true>(a, s) : launch_wx_skinny_k<WT, XT, 1, TN, false>(a, s);
-    return any ? launch_wx_skinny_k<WT, XT, 2, TN, true>(a, s) : launch_wx_skinny_k<WT, XT, 2, TN, false>(a, s);
+    constexpr int TN = WS_TN_SET;
+    if (a.M <= 32)
+        return any ? launch_wx_skinny_k<WT, XT, 1, TN, SZ32, true>(a, s) : launch_wx_skinny_k<WT, XT, 1, TN, SZ32, false>(a, s);
+    return any ? launch_wx_skinny_k<WT, XT, 2, TN, SZ32, true>(a, s) : launch_wx_skinny_k<WT, XT, 2, TN, SZ32, false>(a, s);
+}
+template <int WT, bool SZ32>
+static hipError_t launch_wx_skinny_s(const WxArgs &a, int x_dt, bool any, hipStream_t s) {
+    if (x_dt == DT_F16) return launch_wx_skinny_t<WT, DT_F16, SZ32>(a, any, s);
+    if (x_dt == DT_BF16) return launch_wx_skinny_t<WT, DT_BF16, SZ32>(a, any, s);
+    return launch_wx_skinny_t<WT, DT_F32, SZ32>(a, any, s);
 }
 template <int WT>
 static hipError_t launch_wx_skinny_w(const WxArgs &a, int x_dt, bool any, hipStream_t s) {
-    if (x_dt == DT_F16) return launch_wx_skinny_t<WT, DT_F16>(a, any, s);
-    if (x_dt == DT_BF16) return launch_wx_skinny_t<WT, DT_BF16>(a, any, s);
-    return launch_wx_skinny_t<WT, DT_F32>(a, any, s);
+    if constexpr (WT != WX_Q4)
+        if (a.sz_dt == DT_F32) return launch_wx_skinny_s<WT, true>(a, x_dt, any, s);
+    return launch_wx_skinny_s<WT, false>(a, x_dt, any, s);
 }
 
 // K splits: one workgroup per CU, every wave at least 2 K steps.
 static int wx_skinny_splits(int64_t K, int64_t N) {
-    const int64_t t = (N + 63) / 64, nks = (K + 31) / 32;
+    const int64_t t = (N + 32 * WS_TN_SET - 1) / (32 * WS_TN_SET), nks = (K + 31) / 32;
     int S = 1;
     while (t * S * 2 <= 256 && nks / (S * 2 * WS_NW) >= 2 && S < 16) S *= 2;
     return S;
@@ -168,25 +195,27 @@ static int wx_skinny_splits(int64_t K, int64_t N) {
 
 static int64_t wx_ldp(int64_t N) { return (N + 3) / 4 * 4; }
 
-// Partials stay within 16 MiB, what the allocation-free entry point holds.
-static int wx_splits(int64_t M, int64_t K, int64_t N) {
+// Partials of q4_0 x fp16 stay within 16 MiB, what the allocation-free entry point holds.
+static int wx_splits(int wt, int x_dt, int64_t M, int64_t K, int64_t N) {
+    if (wt == WX_Q4 && M <= 16) return 1;         // wx_gemv
     int S = M <= 64 ? wx_skinny_splits(K, N) : wx_gemm_splits(M, K, N);
-    while (S > 1 && (int64_t)S * M * wx_ldp(N) * 4 > ((int64_t)16 << 20)) S /= 2;
+    if (wt == WX_Q4 && x_dt == DT_F16)
+        while (S > 1 && (int64_t)S * M * wx_ldp(N) * 4 > ((int64_t)16 << 20)) S /= 2;
     return S;
 }
 
 size_t wx_workspace_bytes(int wt, int x_dt, int64_t M, int64_t K, int64_t N) {
-    (void)wt; (void)x_dt;
-    const int S = wx_splits(M, K, N);
+    const int S = wx_splits(wt, x_dt, M, K, N);
     // Partials follow the counter area, which other kernels rely on staying zero.
     return S == 1 ? 0 : COUNTER_BYTES + (size_t)S * M * wx_ldp(N) * sizeof(float);
 }
 
 // Every q4_0 call; INT4 and INT8 with groups of whole K steps, at least one pair
-// of columns (a lane loads two at a time) and 16 rows within a 32-bit offset.  The fused
+// of columns (a lane loads two at a time), 16 rows within a 32-bit offset and a
+// K that keeps the group's multiply-high exact.  The fused
 // activations exist for INT4 x fp16 only.
 bool wx_supported(const WxCall &c) {
-    if (c.wt != WX_Q4 && (c.gs % 32 != 0 || c.N < 2 || c.N > (1 << 27))) return false;
+    if (c.wt != WX_Q4 && (c.gs % 32 != 0 || c.N < 2 || c.N > (1 << 27) || c.K > 65535 * 32)) return false;
     if (c.act != ACT_NONE && (c.wt != WX_I4 || c.x_dt != DT_F16)) return false;
     return true;
 }
@@ -195,15 +224,19 @@ hipError_t launch_wx(const WxCall &c, void *ws, size_t ws_bytes, hipStream_t s) 
     WxArgs a;
     a.X = c.X; a.ldx = c.ldx; a.W = c.W; a.scales = c.scales; a.zeros = c.zeros; a.sz_dt = c.sz_dt;
     a.Y = c.Y; a.ldy = c.ldy; a.M = (int)c.M; a.K = (int)c.K; a.N = (int)c.N;
-    a.spg = c.wt == WX_Q4 ? 1 : (int)std::min<int64_t>(c.gs / 32, 1 << 26);
+    const int64_t spg = c.wt == WX_Q4 ? 1 : c.gs / 32;
+    a.spg_mul = spg * 32 >= c.K ? 0u : (uint32_t)((((uint64_t)1 << 32) + spg - 1) / spg);
+    a.spg_one = 0u;
+    if (spg == 1) { a.spg_mul = 0u; a.spg_one = ~0u; }   // 2^32 itself does not fit
     a.act = c.act;
-    a.S = wx_splits(c.M, c.K, c.N);
+    a.S = wx_splits(c.wt, c.x_dt, c.M, c.K, c.N);
     if (a.S > 1 && (!ws || ws_bytes < wx_workspace_bytes(c.wt, c.x_dt, c.M, c.K, c.N))) a.S = 1;
     a.ldp = (int)wx_ldp(c.N);
     a.part = a.S > 1 ? (float *)((char *)ws + COUNTER_BYTES) : nullptr;
     a.tiles_m = a.tiles_n = 0;
     const int es = c.x_dt == DT_F32 ? 4 : 2;
     const bool any = (uintptr_t)c.X % 16 != 0 || (c.ldx * es) % 16 != 0 || c.K % 32 != 0;
+    if (c.wt == WX_Q4 && c.M <= 16) return launch_wx_gemv(a, c.x_dt, any, s);
     if (c.M > 64) return launch_wx_gemm(a, c.wt, c.x_dt, any, s);
     const hipError_t e = c.wt == WX_Q4   ? launch_wx_skinny_w<WX_Q4>(a, c.x_dt, any, s)
                          : c.wt == WX_I4 ? launch_wx_skinny_w<WX_I4>(a, c.x_dt, any, s)

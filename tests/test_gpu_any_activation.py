@@ -38,7 +38,9 @@ def _check(Y, X, W, xdt, act=None):
 # Rows: the smallest, around 32 and 64 (row tiles, the decode / prefill line), around
 # 128 (row tile of the prefill kernel).  Columns: 1, around 64 and 256 (column tiles),
 # odd.  K: one block, an odd number of blocks, splits over workgroups.
-SHAPES = [(1, 32, 1), (1, 4096, 257), (3, 96, 63), (16, 2080, 64), (31, 1024, 65), (32, 4096, 128), (33, 64, 130),
+# Spans of 0..4 column groups (N = 48, 4096, 8208, 16384 at K <= 4096) and their K split
+# (N <= 4096, long K).
+SHAPES = [(1, 4096, 48), (4, 2080, 4096), (9, 1024, 8208), (8, 288, 16384), (1, 8224, 4096), (13, 14336, 1024), (1, 32, 1), (1, 4096, 257), (3, 96, 63), (16, 2080, 64), (31, 1024, 65), (32, 4096, 128), (33, 64, 130),
           (64, 4128, 100), (65, 32, 255), (65, 1056, 257), (127, 992, 256), (129, 2080, 513), (300, 4096, 40)]
 
 
