@@ -49,6 +49,8 @@ hipError_t launch_gemv_span_bf16(const void *X, int64_t ldx, const uint8_t *W, v
                                  int64_t N, void *ws, size_t ws_bytes, bool *done, hipStream_t s);
 hipError_t q4_gemv_span_split_fallbacks(uint64_t *count, bool reset);
 hipError_t q4_gemm8_split_fallbacks(uint64_t *count, bool reset);
+hipError_t wx_mid_split_fallbacks(uint64_t *count, bool reset);
+bool wx_mid_supported(const WxCall &c);
 bool gemv_dma_supported(const _Float16 *X, const uint8_t *W, int64_t K, int64_t N);
 hipError_t launch_gemv_dma_group(const _Float16 *X, const uint8_t *const *W, _Float16 *const *Y, int count,
                                  int K, int N, int *n_done, hipStream_t s);
@@ -269,7 +271,7 @@ static size_t required_ws_bytes(int64_t M, int64_t K, int64_t N) {
 size_t mcq4_matmul_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     const size_t need = required_ws_bytes(M, K, N);
     // wx splits K only where the workspace covers it.
-    return M > 32 && K > 0 && N > 0 && K % 32 == 0 ? std::max(need, mcq4::wx_workspace_bytes(mcq4::WX_Q4, mcq4::DT_F16, M, K, N)) : need;
+    return M > 16 && K > 0 && N > 0 && K % 32 == 0 ? std::max(need, mcq4::wx_workspace_bytes(mcq4::WX_Q4, mcq4::DT_F16, M, K, N)) : need;
 }
 
 size_t mcq4_matmul_q4_0_workspace_bytes(int64_t M, int64_t K, int64_t N, int x_dtype) {
@@ -303,6 +305,12 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
     hipError_t e;
     // 33..64 rows: q4_gemm6 (flat ~31 us for any M <= 128 on 4096x14336) beats the
     // register-load decode kernel (40-77 us) wherever its alignment rules hold.
+    // 17..64 rows: the kernel between the decode and the prefill ones.  MCQ4_GEMVM_SPLIT,
+    // MCQ4_GEMV_PATH, MCQ4_DECODE_PATH (tests) leave these rows to the decode kernels.
+    const mcq4::WxCall mid = {mcq4::WX_Q4, mcq4::DT_F16, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32};
+    if (M > 16 && M <= 64 && mcq4::wx_mid_supported(mid) && !mcq4::opt("MCQ4_GEMVM_SPLIT") && !mcq4::opt("MCQ4_GEMV_PATH") &&
+        !mcq4::opt("MCQ4_DECODE_PATH"))
+        return hip_status(mcq4::launch_wx(mid, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
     const bool skinny = M <= 32 || (M <= 64 && !mcq4::gemm6_supported((const _Float16 *)X, ldx, W, M, K, N));
     if (skinny)
         e = mcq4::launch_skinny((const _Float16 *)X, ldx, W, (_Float16 *)Y, ldy, (int)M, (int)K,
@@ -413,7 +421,7 @@ int mcq4_split_fallback_count(uint64_t *count, int reset) {
     hipError_t (*const readers[])(uint64_t *, bool) = {
         mcq4::q4_gemvm_split_fallbacks, mcq4::q4_gemm6_split_fallbacks, mcq4::i4_gemv_split_fallbacks,
         mcq4::i4_gemv1_split_fallbacks, mcq4::i4_gemm6_split_fallbacks, mcq4::q4_gemv_span_split_fallbacks,
-        mcq4::q4_gemm8_split_fallbacks};
+        mcq4::q4_gemm8_split_fallbacks, mcq4::wx_mid_split_fallbacks};
     for (auto rd : readers)
         if (int st = hip_status(rd(count, reset != 0), "split fallback counter")) return st;
     return MCQ4_OK;

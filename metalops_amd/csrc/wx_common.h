@@ -39,6 +39,10 @@ struct WxArgs {
     float *part;                 // [S][M][ldp] fp32 partials when S > 1
     int ldp;
     int tiles_m, tiles_n;
+    // wx_mid with S > 1: [column tiles][S] flag words behind the partials (null: the
+    // reduction kernel sums), polls of a flag, splits treated as run on another XCD.
+    uint32_t *flags = nullptr;
+    uint32_t spin = 0, foreign = 0;
 };
 
 // Unaligned loads: gfx950 global loads need no alignment beyond the byte.
@@ -213,29 +217,56 @@ __device__ __forceinline__ void q4_pairs(uint32_t w, uint32_t (&p)[4]) {
 // Whether a lane's block scale is infinite or NaN.
 __device__ __forceinline__ bool q4_scale_odd(uint16_t d) { return (d & 0x7C00u) == 0x7C00u; }
 
-// The lane's 16 weights of tile j in fp32, in slot order.
-// q4_0, FIN (every scale finite): (1024 + q) d - 1032 d and (64 + q) d - 72 d, one
-// mixed-precision fma each, exact in fp32 (d has 11 significant bits).  Without
-// FIN q - 8 first, so an infinite d gives the signed infinities of (q - 8) d.
-// INT4 and INT8: (q - z) s in the reference's two fp32 roundings.
+// The eight weights of a nibble dword in fp32, in slot order.  FIN (d finite):
+// (1024 + q) d - 1032 d and (64 + q) d - 72 d, one mixed-precision fma each, exact
+// in fp32 (d has 11 significant bits).  Otherwise q - 8 first, so an infinite d
+// gives the signed infinities of (q - 8) d.
+template <bool FIN>
+__device__ __forceinline__ void q4_values8(uint32_t q, float d, float *w) {
+    const float c[2] = {-1032.0f * d, -72.0f * d};
+    uint32_t p[4];
+    q4_pairs(q, p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        half2_t v = bitcast<half2_t>(p[i]);
+        if constexpr (!FIN) v -= (i & 1) ? half2_t{(_Float16)72.0f, (_Float16)72.0f} : half2_t{(_Float16)1032.0f, (_Float16)1032.0f};
+        w[2 * i] = __builtin_fmaf((float)v[0], d, FIN ? c[i & 1] : 0.0f);
+        w[2 * i + 1] = __builtin_fmaf((float)v[1], d, FIN ? c[i & 1] : 0.0f);
+    }
+}
+// The same eight as a B operand of 16-bit activations (fp16: one packed multiply,
+// the single rounding of the exact product).
+template <int XT, bool FIN>
+__device__ __forceinline__ uint4_t q4_operand8(uint32_t q, uint16_t d) {
+    uint4_t r;
+    if constexpr (XT == DT_F16) {
+#pragma clang fp contract(off)
+        const uint32_t dd = d;
+        const half2_t d2 = bitcast<half2_t>(dd | (dd << 16));
+        uint32_t p[4];
+        q4_pairs(q, p);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const half2_t off = (i & 1) ? half2_t{(_Float16)72.0f, (_Float16)72.0f} : half2_t{(_Float16)1032.0f, (_Float16)1032.0f};
+            r[i] = bitcast<uint32_t>((bitcast<half2_t>(p[i]) - off) * d2);
+        }
+    } else {
+        float w[8];
+        q4_values8<FIN>(q, (float)bitcast<_Float16>(d), w);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = pack2<XT>(w[2 * i], w[2 * i + 1]);
+    }
+    return r;
+}
+
+// The lane's 16 weights of tile j in fp32, in slot order.  INT4 and INT8:
+// (q - z) s in the reference's two fp32 roundings.
 // TAIL: weights of rows past K are zero (`valid` = rows of the lane's 16 below K).
 template <int WT, int XT, int TN, bool SZ32, bool TAIL, bool FIN>
 __device__ __forceinline__ void wx_values(const WxRaw<WT, TN> &r, int j, int sz_dt, int valid, float (&w)[16]) {
     if constexpr (WT == WX_Q4) {
-        const float d = (float)bitcast<_Float16>(r.d[j]);
-        const float c[2] = {-1032.0f * d, -72.0f * d};
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            uint32_t p[4];
-            q4_pairs(r.q[j][h], p);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                half2_t v = bitcast<half2_t>(p[i]);
-                if constexpr (!FIN) v -= (i & 1) ? half2_t{(_Float16)72.0f, (_Float16)72.0f} : half2_t{(_Float16)1032.0f, (_Float16)1032.0f};
-                w[8 * h + 2 * i] = __builtin_fmaf((float)v[0], d, FIN ? c[i & 1] : 0.0f);
-                w[8 * h + 2 * i + 1] = __builtin_fmaf((float)v[1], d, FIN ? c[i & 1] : 0.0f);
-            }
-        }
+        for (int h = 0; h < 2; ++h) q4_values8<FIN>(r.q[j][h], (float)bitcast<_Float16>(r.d[j]), w + 8 * h);
     } else {
         const float s = wx_sz_f32<SZ32>(r.s[j], sz_dt), z = wx_sz_f32<SZ32>(r.z[j], sz_dt);
         auto val = [&](float q) {
@@ -263,20 +294,9 @@ __device__ __forceinline__ void wx_values(const WxRaw<WT, TN> &r, int j, int sz_
 // the lane's 16.
 template <int WT, int XT, int TN, bool SZ32, bool TAIL, bool FIN>
 __device__ __forceinline__ void wx_operands(const WxRaw<WT, TN> &r, int j, int sz_dt, int valid, uint4_t (&ops)[2]) {
-    if constexpr (WT == WX_Q4 && XT == DT_F16) {
-#pragma clang fp contract(off)
-        const uint32_t dd = r.d[j];
-        const half2_t d2 = bitcast<half2_t>(dd | (dd << 16));
+    if constexpr (WT == WX_Q4) {
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            uint32_t p[4];
-            q4_pairs(r.q[j][ks], p);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const half2_t off = (i & 1) ? half2_t{(_Float16)72.0f, (_Float16)72.0f} : half2_t{(_Float16)1032.0f, (_Float16)1032.0f};
-                ops[ks][i] = bitcast<uint32_t>((bitcast<half2_t>(p[i]) - off) * d2);
-            }
-        }
+        for (int ks = 0; ks < 2; ++ks) ops[ks] = q4_operand8<XT, FIN>(r.q[j][ks], r.d[j]);
     } else {
         float w[16];
         wx_values<WT, XT, TN, SZ32, TAIL, FIN>(r, j, sz_dt, valid, w);
@@ -301,6 +321,13 @@ __device__ __forceinline__ void wx_if_finite(const uint16_t *d, F body) {
     }
 }
 
+template <int XT>
+__device__ __forceinline__ float4_t wx_mfma16(uint4_t a, uint4_t b, float4_t c) {
+    if constexpr (XT == DT_BF16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8_t>(a), bitcast<bf16x8_t>(b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(bitcast<half8_t>(a), bitcast<half8_t>(b), c, 0, 0, 0);
+}
 template <int XT>
 __device__ __forceinline__ float16_t wx_mfma(uint4_t a, uint4_t b, float16_t c) {
     return mfma32<XT>(bitcast<half8_t>(a), bitcast<half8_t>(b), c);

@@ -93,12 +93,7 @@ __global__ void __launch_bounds__(NW * 64) wx_gemv_kernel(WxArgs a) {
                         uint4_t B[2];
                         wx_operands<WX_Q4, XT, 1, false, false, FIN>(r, 0, 0, 16, B);
 #pragma unroll
-                        for (int ks = 0; ks < 2; ++ks) {
-                            if constexpr (XT == DT_BF16)
-                                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8_t>(p.x[2 * h + ks]), bitcast<bf16x8_t>(B[ks]), acc[j], 0, 0, 0);
-                            else
-                                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bitcast<half8_t>(p.x[2 * h + ks]), bitcast<half8_t>(B[ks]), acc[j], 0, 0, 0);
-                        }
+                        for (int ks = 0; ks < 2; ++ks) acc[j] = wx_mfma16<XT>(p.x[2 * h + ks], B[ks], acc[j]);
                     }
                 }
             }

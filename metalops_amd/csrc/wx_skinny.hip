@@ -151,6 +151,11 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
 
 hipError_t launch_wx_reduce(const WxArgs &a, int x_dt, hipStream_t s);
 hipError_t launch_wx_gemv(const WxArgs &a, int x_dt, bool any, hipStream_t s);
+bool wx_mid_shape(int wt, int x_dt, int64_t M, int64_t N);
+bool wx_mid_supported(const WxCall &c);
+int wx_mid_splits(int64_t K, int64_t N);
+size_t wx_mid_flag_bytes(int64_t N, int S);
+hipError_t launch_wx_mid(WxArgs a, int x_dt, bool *reduce, hipStream_t s);
 hipError_t launch_wx_gemm(WxArgs a, int wt, int x_dt, bool any, hipStream_t s);
 int wx_gemm_splits(int64_t M, int64_t K, int64_t N);
 
@@ -198,7 +203,8 @@ static int64_t wx_ldp(int64_t N) { return (N + 3) / 4 * 4; }
 // Partials of q4_0 x fp16 stay within 16 MiB, what the allocation-free entry point holds.
 static int wx_splits(int wt, int x_dt, int64_t M, int64_t K, int64_t N) {
     if (wt == WX_Q4 && M <= 16) return 1;         // wx_gemv
-    int S = M <= 64 ? wx_skinny_splits(K, N) : wx_gemm_splits(M, K, N);
+    // One plan for a shape, whatever the alignment: wx_mid and wx_skinny share it.
+    int S = wx_mid_shape(wt, x_dt, M, N) ? wx_mid_splits(K, N) : M <= 64 ? wx_skinny_splits(K, N) : wx_gemm_splits(M, K, N);
     if (wt == WX_Q4 && x_dt == DT_F16)
         while (S > 1 && (int64_t)S * M * wx_ldp(N) * 4 > ((int64_t)16 << 20)) S /= 2;
     return S;
@@ -207,7 +213,9 @@ static int wx_splits(int wt, int x_dt, int64_t M, int64_t K, int64_t N) {
 size_t wx_workspace_bytes(int wt, int x_dt, int64_t M, int64_t K, int64_t N) {
     const int S = wx_splits(wt, x_dt, M, K, N);
     // Partials follow the counter area, which other kernels rely on staying zero.
-    return S == 1 ? 0 : COUNTER_BYTES + (size_t)S * M * wx_ldp(N) * sizeof(float);
+    if (S == 1) return 0;
+    return COUNTER_BYTES + (size_t)S * M * wx_ldp(N) * sizeof(float) +
+           (wx_mid_shape(wt, x_dt, M, N) ? wx_mid_flag_bytes(N, S) : 0);
 }
 
 // Every q4_0 call; INT4 and INT8 with groups of whole K steps, at least one pair
@@ -238,10 +246,12 @@ hipError_t launch_wx(const WxCall &c, void *ws, size_t ws_bytes, hipStream_t s) 
     const bool any = (uintptr_t)c.X % 16 != 0 || (c.ldx * es) % 16 != 0 || c.K % 32 != 0;
     if (c.wt == WX_Q4 && c.M <= 16) return launch_wx_gemv(a, c.x_dt, any, s);
     if (c.M > 64) return launch_wx_gemm(a, c.wt, c.x_dt, any, s);
-    const hipError_t e = c.wt == WX_Q4   ? launch_wx_skinny_w<WX_Q4>(a, c.x_dt, any, s)
+    bool reduce = a.S > 1;
+    const hipError_t e = wx_mid_supported(c) ? launch_wx_mid(a, c.x_dt, &reduce, s)
+                         : c.wt == WX_Q4   ? launch_wx_skinny_w<WX_Q4>(a, c.x_dt, any, s)
                          : c.wt == WX_I4 ? launch_wx_skinny_w<WX_I4>(a, c.x_dt, any, s)
                                          : launch_wx_skinny_w<WX_I8>(a, c.x_dt, any, s);
-    if (e != hipSuccess || a.S == 1) return e;
+    if (e != hipSuccess || !reduce) return e;
     return launch_wx_reduce(a, c.x_dt, s);
 }
 
