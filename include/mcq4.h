@@ -79,6 +79,11 @@ int mcq4_quantize_q4_0_llama(const float *W, int64_t ldw, int64_t K, int64_t N,
 int mcq4_dequantize_q4_0(const uint8_t *blocks, int64_t K, int64_t N, void *out,
                          int64_t ldo, int out_dtype, void *stream);
 
+/* The same for a bf16 out: the exact product rounded once to nearest-even bf16
+ * (dequantize_ggml_q4_0(blocks, torch.bfloat16)). */
+int mcq4_dequantize_q4_0_bf16(const uint8_t *blocks, int64_t K, int64_t N, void *out, int64_t ldo,
+                              void *stream);
+
 /*
  * Workspace bytes mcq4_matmul_q4_0_f16 needs for this shape (0 = none).  The
  * workspace starts with a fixed 256 KiB area of per-tile arrival counters,

@@ -31,6 +31,7 @@ SIGNATURES = {
     "mcq4_quantize_q4_0_typed": (_int, [_p, _int, _i64, _i64, _i64, _p, _p]),
     "mcq4_quantize_q4_0_llama": (_int, [_p, _i64, _i64, _i64, _p, _p]),
     "mcq4_dequantize_q4_0": (_int, [_p, _i64, _i64, _p, _i64, _int, _p]),
+    "mcq4_dequantize_q4_0_bf16": (_int, [_p, _i64, _i64, _p, _i64, _p]),
     "mcq4_matmul_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "mcq4_matmul_q4_0_f16": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _i64, _p, _sz, _p]),
     "mcq4_matmul_q4_0": (_int, [_p, _int, _i64, _p, _p, _i64, _i64, _i64, _i64, _p, _sz, _p]),

@@ -21,8 +21,7 @@
 namespace mcq4 {
 hipError_t launch_quantize(bool llama_rule, const float *W, int64_t ldw, int nb, int N,
                            uint8_t *out, hipStream_t s);
-hipError_t launch_dequant(const uint8_t *blocks, int nb, int N, void *out, int64_t ldo,
-                          bool f16, hipStream_t s);
+hipError_t launch_dequant(const uint8_t *blocks, int nb, int N, void *out, int64_t ldo, int out_dt, hipStream_t s);
 size_t skinny_workspace_bytes(int64_t M, int64_t K, int64_t N);
 hipError_t launch_skinny(const _Float16 *X, int64_t ldx, const uint8_t *W, _Float16 *Y,
                          int64_t ldy, int M, int K, int N, void *ws, hipStream_t s);
@@ -242,20 +241,30 @@ int mcq4_quantize_q4_0_llama(const float *W, int64_t ldw, int64_t K, int64_t N,
     return quantize_common(true, W, ldw, K, N, blocks, stream);
 }
 
+static int dequantize_common(const uint8_t *blocks, int64_t K, int64_t N, void *out, int64_t ldo, int out_dtype,
+                             void *stream) {
+    if (!blocks || !out) return fail(MCQ4_ERR_INVALID_ARG, "null pointer");
+    if (int st = check_kn(K, N)) return st;
+    if (ldo < N) return fail(MCQ4_ERR_SHAPE, "ldo (%lld) < N (%lld)", (long long)ldo, (long long)N);
+    if (!aligned(blocks, 2)) return fail(MCQ4_ERR_ALIGNMENT, "blocks must be 2-byte aligned");
+    if (!aligned(out, out_dtype == MCQ4_DTYPE_F32 ? 4 : 2))
+        return fail(MCQ4_ERR_ALIGNMENT, "out is misaligned for its dtype");
+    return hip_status(mcq4::launch_dequant(blocks, (int)(K / 32), (int)N, out, ldo, out_dtype, (hipStream_t)stream),
+                      "dequantize launch");
+}
+
 int mcq4_dequantize_q4_0(const uint8_t *blocks, int64_t K, int64_t N, void *out, int64_t ldo,
                          int out_dtype, void *stream) {
     g_err[0] = 0;
     if (!blocks || !out) return fail(MCQ4_ERR_INVALID_ARG, "null pointer");
     if (out_dtype != MCQ4_DTYPE_F32 && out_dtype != MCQ4_DTYPE_F16)
         return fail(MCQ4_ERR_INVALID_ARG, "out_dtype must be MCQ4_DTYPE_F32 or MCQ4_DTYPE_F16");
-    if (int st = check_kn(K, N)) return st;
-    if (ldo < N) return fail(MCQ4_ERR_SHAPE, "ldo (%lld) < N (%lld)", (long long)ldo, (long long)N);
-    if (!aligned(blocks, 2)) return fail(MCQ4_ERR_ALIGNMENT, "blocks must be 2-byte aligned");
-    if (!aligned(out, out_dtype == MCQ4_DTYPE_F32 ? 4 : 2))
-        return fail(MCQ4_ERR_ALIGNMENT, "out is misaligned for its dtype");
-    return hip_status(mcq4::launch_dequant(blocks, (int)(K / 32), (int)N, out, ldo,
-                                           out_dtype == MCQ4_DTYPE_F16, (hipStream_t)stream),
-                      "dequantize launch");
+    return dequantize_common(blocks, K, N, out, ldo, out_dtype, stream);
+}
+
+int mcq4_dequantize_q4_0_bf16(const uint8_t *blocks, int64_t K, int64_t N, void *out, int64_t ldo, void *stream) {
+    g_err[0] = 0;
+    return dequantize_common(blocks, K, N, out, ldo, MCQ4_DTYPE_BF16, stream);
 }
 
 // What mcq4_matmul_q4_0_f16 cannot do without.

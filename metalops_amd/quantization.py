@@ -127,14 +127,18 @@ def dequantize_ggml_q4_0(blocks: torch.Tensor, dtype: Optional[torch.dtype] = No
     b = blocks if (blocks.is_contiguous() and blocks.data_ptr() % 2 == 0) else blocks.contiguous()
     if b.data_ptr() % 2:
         b = b.clone()
-    kernel_dtype = torch.float16 if dtype == torch.float16 else torch.float32
+    kernel_dtype = dtype if dtype in (torch.float16, torch.bfloat16) else torch.float32
     out = torch.empty((K, N), dtype=kernel_dtype, device=b.device)
     if K and N:
-        code = _lib.MCQ4_DTYPE_F16 if kernel_dtype == torch.float16 else _lib.MCQ4_DTYPE_F32
         with torch.cuda.device(b.device):
-            _lib.check(_lib.lib.mcq4_dequantize_q4_0(b.data_ptr(), K, N, out.data_ptr(), N, code,
-                                                     _stream(b.device)),
-                       "mcq4_dequantize_q4_0")
+            if kernel_dtype == torch.bfloat16:
+                _lib.check(_lib.lib.mcq4_dequantize_q4_0_bf16(b.data_ptr(), K, N, out.data_ptr(), N, _stream(b.device)),
+                           "mcq4_dequantize_q4_0_bf16")
+            else:
+                code = _lib.MCQ4_DTYPE_F16 if kernel_dtype == torch.float16 else _lib.MCQ4_DTYPE_F32
+                _lib.check(_lib.lib.mcq4_dequantize_q4_0(b.data_ptr(), K, N, out.data_ptr(), N, code,
+                                                         _stream(b.device)),
+                           "mcq4_dequantize_q4_0")
     return out if out.dtype == dtype else out.to(dtype)
 
 

@@ -1,0 +1,69 @@
+"""The wide conversion kernels (several columns per thread) against the oracles and,
+on special values, against the one-column kernels, which an odd row stride selects.
+
+All exact: bytes, scales, zeros and outputs are compared bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import int4_ref as R
+from oracle import q4_0_ref as Q
+
+pytestmark = pytest.mark.gpu
+
+TDT = {R.F32: torch.float32, R.F16: torch.float16, R.BF16: torch.bfloat16}
+
+
+def _odd(w):
+    """The same weight at a row stride that only the one-column kernels take."""
+    s = torch.empty(w.shape[0], w.shape[1] + 1, dtype=w.dtype, device=w.device)
+    s[:, :-1] = w
+    return s[:, :-1]
+
+
+def _bits(t):
+    return t.contiguous().view(torch.uint8)
+
+
+# Columns: one thread, the last column set of a workgroup, past it.  K: one block or group,
+# a last group that is not whole.
+@pytest.mark.parametrize("K,N,gs", [(32, 4, 32), (64, 252, 64), (128, 260, 128), (160, 1028, 128), (288, 516, 64),
+                                    (70, 8, 32), (4096, 1024, 128)])
+@pytest.mark.parametrize("dtype", [R.F32, R.F16, R.BF16])
+def test_wide_matches_oracle(dev, dtype, K, N, gs):
+    import metalops_amd as mo
+    print(f"convert {dtype} K={K} N={N} gs={gs}", flush=True)
+    w = R.round_to(np.random.default_rng(K + N).standard_normal((K, N), np.float32) * 0.02, dtype)
+    t = torch.from_numpy(w).to(TDT[dtype]).to(dev)
+    p, s, z = mo.quantize_int4(t, gs)
+    rp, rs, rz = R.quantize(w, gs, dtype)
+    assert np.array_equal(p.cpu().numpy(), rp)
+    assert np.array_equal(s.float().cpu().numpy(), rs) and np.array_equal(z.float().cpu().numpy(), rz)
+    for out in (R.F32, R.F16, R.BF16):
+        y = mo.dequantize_int4(p, s, z, gs, TDT[out])
+        assert np.array_equal(y.float().cpu().numpy(), R.dequantize(rp, rs, rz, gs, out))
+    if K % 32:
+        return
+    b = mo.quantize_ggml_q4_0(t)
+    assert np.array_equal(b.cpu().numpy(), Q.quantize_ref_rule(w, {R.F32: "float32", R.F16: "float16", R.BF16: "bfloat16"}[dtype]))
+    exact = Q.dequantize(b.cpu().numpy(), np.float32)
+    for out in (R.F32, R.F16, R.BF16):
+        y = mo.dequantize_ggml_q4_0(b, TDT[out])
+        assert np.array_equal(y.float().cpu().numpy(), R.round_to(exact, out))
+
+
+@pytest.mark.parametrize("dtype", [R.F32, R.F16, R.BF16])
+@pytest.mark.parametrize("std", [0.02, 3e3, 1e-7])
+def test_wide_matches_one_column_on_specials(dev, dtype, std):
+    import metalops_amd as mo
+    g = torch.Generator(device=dev).manual_seed(7)
+    w = (torch.randn(512, 1024, generator=g, device=dev) * std * torch.exp(3 * torch.randn(1, 1024, generator=g, device=dev))).to(TDT[dtype])
+    w[::97, ::31], w[::89, ::37], w[::83, ::41] = float("nan"), float("inf"), -float("inf")
+    w[64:96], w[::53, ::3] = 0, -0.0
+    assert torch.equal(mo.quantize_ggml_q4_0(w), mo.quantize_ggml_q4_0(_odd(w)))
+    for gs in (32, 64, 128):
+        for a, b in zip(mo.quantize_int4(w, gs), mo.quantize_int4(_odd(w), gs)):
+            assert torch.equal(_bits(a), _bits(b))
+    if dtype == R.F32:
+        for a, b in zip(mo.quantize_to_int4(w, 128), mo.quantize_to_int4(_odd(w), 128)):
+            assert torch.equal(_bits(a), _bits(b))
