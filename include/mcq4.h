@@ -223,6 +223,11 @@ int mcq4_dequantize_int4(const uint8_t *packed, const void *scales, const void *
 size_t mcq4_matmul_int4_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size,
                                         int x_dtype);
 
+/* Workspace bytes the int4 matmul entry points make use of: at least the above,
+ * plus the optional workspace of other dtypes, shapes and alignments. */
+size_t mcq4_matmul_int4_best_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size,
+                                             int x_dtype);
+
 /*
  * matmul_int4 (quantization.py:156-239; Metal binding matmul_int4_metal,
  * native/core_mps.mm:5612-5776): Y[M][ldy] = X[M][ldx] @ dequant(W) with
@@ -271,6 +276,8 @@ int mcq4_quantize_to_int4(const float *W, int64_t ldw, int64_t K, int64_t N, int
  * ------------------------------------------------------------------------- */
 size_t mcq4_matmul_int8_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size,
                                         int x_dtype);
+size_t mcq4_matmul_int8_best_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size,
+                                             int x_dtype);
 
 /* Y[M][ldy] = X[M][ldx] @ dequant(W), fp32 accumulation, X and Y in x_dtype.
  * fp16 activations with group_size % 16 == 0, K % 16 == 0 and N % 8 == 0 run

@@ -45,6 +45,8 @@ SIGNATURES = {
     "mcq4_quantize_int4": (_int, [_p, _int, _i64, _i64, _i64, _i64, _p, _p, _p, _p]),
     "mcq4_dequantize_int4": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _p, _i64, _int, _p]),
     "mcq4_matmul_int4_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _int]),
+    "mcq4_matmul_int4_best_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _int]),
+    "mcq4_matmul_int8_best_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _int]),
     "mcq4_matmul_int4": (_int, [_p, _int, _i64, _p, _p, _p, _int, _p, _i64, _i64, _i64, _i64,
                                 _i64, _p, _sz, _p]),
     "mcq4_matmul_int4_silu": (_int, [_p, _int, _i64, _p, _p, _p, _int, _p, _i64, _i64, _i64,

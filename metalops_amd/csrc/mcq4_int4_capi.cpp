@@ -216,7 +216,7 @@ int mcq4_quantize_to_int4(const float *W, int64_t ldw, int64_t K, int64_t N, int
 
 size_t mcq4_matmul_int8_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size,
                                         int x_dtype) {
-    return query_ws_bytes(M, K, N, group_size, x_dtype, 8);
+    return ws_bytes(M, K, N, group_size, x_dtype, 8);
 }
 
 int mcq4_matmul_int8(const void *X, int x_dtype, int64_t ldx, const int8_t *W, const void *scales,
@@ -247,7 +247,15 @@ int mcq4_dequantize_int4(const uint8_t *packed, const void *scales, const void *
 
 size_t mcq4_matmul_int4_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size,
                                         int x_dtype) {
+    return ws_bytes(M, K, N, group_size, x_dtype);
+}
+
+size_t mcq4_matmul_int4_best_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size, int x_dtype) {
     return query_ws_bytes(M, K, N, group_size, x_dtype);
+}
+
+size_t mcq4_matmul_int8_best_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size, int x_dtype) {
+    return query_ws_bytes(M, K, N, group_size, x_dtype, 8);
 }
 
 int mcq4_matmul_int4(const void *X, int x_dtype, int64_t ldx, const uint8_t *packed,

@@ -220,7 +220,7 @@ def _matmul(X, W_packed, scales, zeros, group_size, act):
             Y.zero_()
         else:
             xdt = _DT[x.dtype]
-            need = int(_lib.lib.mcq4_matmul_int4_workspace_bytes(M, K, N, group_size, xdt))
+            need = int(_lib.lib.mcq4_matmul_int4_best_workspace_bytes(M, K, N, group_size, xdt))
             stream = _stream(x.device)
             ws, ws_ptr, ws_bytes = None, None, 0
             if need:
@@ -350,7 +350,7 @@ def matmul_int8(
             Y.zero_()
         else:
             xdt = _DT[x.dtype]
-            need = int(_lib.lib.mcq4_matmul_int8_workspace_bytes(M, K, N, group_size, xdt))
+            need = int(_lib.lib.mcq4_matmul_int8_best_workspace_bytes(M, K, N, group_size, xdt))
             stream = _stream(x.device)
             ws, ws_ptr, ws_bytes = None, None, 0
             if need:
