@@ -41,6 +41,7 @@ constexpr int kN = sizeof(kNames) / sizeof(kNames[0]);
 struct Snapshot {
     std::string value[kN];
     bool set[kN];
+    bool any = false;        // some switch is set: nothing to look up otherwise
 };
 
 std::atomic<const Snapshot *> g_snap{nullptr};
@@ -51,6 +52,7 @@ const Snapshot *load() {
     for (int i = 0; i < kN; ++i) {
         const char *v = getenv(kNames[i]);
         s->set[i] = v != nullptr;
+        s->any = s->any || v != nullptr;
         s->value[i] = v ? v : "";
     }
     return s;
@@ -69,6 +71,7 @@ const char *opt(const char *name) {
             g_snap.store(s, std::memory_order_release);
         }
     }
+    if (!s->any) return nullptr;
     for (int i = 0; i < kN; ++i)
         if (strcmp(kNames[i], name) == 0) return s->set[i] ? s->value[i].c_str() : nullptr;
     return nullptr;

@@ -29,7 +29,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .quantization import _workspace   # split-K workspace shared with the q4_0 path
+from .quantization import _native, _workspace   # call path and workspace shared with the q4_0 path
 
 __all__ = [
     "quantize_int4",
@@ -197,6 +197,10 @@ _FN = {0: "mcq4_matmul_int4", 1: "mcq4_matmul_int4_silu", 2: "mcq4_matmul_int4_g
 
 
 def _matmul(X, W_packed, scales, zeros, group_size, act):
+    if _native is not None:
+        Y = _native.int4_matmul(X, W_packed, scales, zeros, group_size, act)
+        if Y is not None:
+            return Y
     _require_device(X, W_packed, scales, zeros)
     K, N = _check_shapes(W_packed, scales, zeros, group_size)
     batched = X.dim() == 3                                   # quantization.py:185-192
@@ -283,6 +287,10 @@ def fused_rmsnorm_linear_int4(X, W_norm, W_packed, scales, zeros, eps, group_siz
     stream with ``X_norm`` in the shared workspace.  ``X`` is ``[B, K]`` fp16 and
     ``W_norm`` ``[K]`` fp16, as the reference binding requires (core_mps.mm:3029).
     """
+    if _native is not None:
+        Y = _native.int4_rmsnorm(X, W_norm, W_packed, scales, zeros, eps, group_size)
+        if Y is not None:
+            return Y
     if X.dtype != torch.float16:
         raise RuntimeError("Fused kernel requires half precision")
     if X.dim() != 2:
@@ -326,6 +334,10 @@ def matmul_int8(
     kernels; other dtypes use weights rounded to ``X``'s dtype, as the
     reference's fallback builds ``W`` in ``X.dtype``.
     """
+    if _native is not None:
+        Y = _native.int8_matmul(X, W_packed, scales, zeros, group_size, 0)
+        if Y is not None:
+            return Y
     _require_device(X, W_packed, scales, zeros)
     if X.dim() != 2:
         raise RuntimeError(f"X must be [M, K], got shape {tuple(X.shape)}")

@@ -25,6 +25,14 @@ import torch
 
 from . import _lib
 
+# The native call path (csrc/torch_ext/mcq4_torch.cpp): checks, output, workspace and
+# launch of a call whose tensors need no conversion, None for any other.  Without the
+# extension every call goes through ctypes to the same kernels.
+try:
+    from .torch_ext import backend as _native
+except ImportError:
+    _native = None
+
 QK4_0 = 32                         # quantization.py:303
 BLOCK_Q4_0_SIZE = 2 + QK4_0 // 2   # quantization.py:304 (18 bytes)
 
@@ -151,7 +159,8 @@ class _Workspace:
     so an interrupted call cannot poison later ones.
     One buffer per (device, stream), so concurrent streams never share one; a
     larger request allocates a new buffer through PyTorch's stream-ordered
-    caching allocator.
+    caching allocator.  With the extension the buffers are its own, shared with
+    the native call path.
     """
 
     def __init__(self):
@@ -159,6 +168,8 @@ class _Workspace:
         self._lock = threading.Lock()
 
     def get(self, device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
+        if _native is not None:
+            return _native.workspace(device.index, stream, nbytes)
         key = (device, stream)   # one buffer per stream: calls on one stream never overlap
         with self._lock:
             buf = self._bufs.get(key)
@@ -194,6 +205,10 @@ def matmul_ggml_q4_0(X: torch.Tensor, W_blocks: torch.Tensor) -> torch.Tensor:
     dtype -- so bf16 activations beyond the fp16 range stay finite.  M <= 64
     runs the decode kernels, larger M the prefill GEMM.
     """
+    if _native is not None:
+        Y = _native.q4_matmul(X, W_blocks)
+        if Y is not None:
+            return Y
     num_blocks_per_col, N, _ = W_blocks.shape
     K = num_blocks_per_col * QK4_0
     assert X.shape[1] == K, f"X K dim ({X.shape[1]}) must match weight K ({K})"  # :443
@@ -258,6 +273,10 @@ def matmul_ggml_q4_0_grouped(X: torch.Tensor, weights: Sequence[torch.Tensor]) -
     weights = list(weights)
     if not weights:
         return []
+    if _native is not None:
+        Ys = _native.q4_grouped(X, weights)
+        if Ys is not None:
+            return Ys
     shape = tuple(weights[0].shape)
     for w in weights:
         if tuple(w.shape) != shape:
