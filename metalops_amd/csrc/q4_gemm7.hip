@@ -66,7 +66,8 @@ __device__ __forceinline__ void g7_copy_a(const uint8_t *base, int off, int byte
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16, vo, 0, 0, 0);
 }
 
-template <int XT>
+// RAG: N % 256 != 0 (N % 8 == 0), a wave may have fewer columns or none.
+template <int XT, bool RAG>
 __global__ void __launch_bounds__(256, 1)
 q4_gemm7_kernel(Gemm7Args a) {
     constexpr int TM = G7_BM / 32, TN = G7_WN / 32;   // 8 x 2
@@ -111,13 +112,14 @@ q4_gemm7_kernel(Gemm7Args a) {
     const int vo_a1 = (64 * wave + (lane >> 3)) * x_row + 16 * (a_c1 & 3) + 64 * (a_c1 >> 2);
 
     const int row_bytes = a.N * BLOCK_BYTES;
-    const int w_off = k_lo * row_bytes + min(n0 + wave * G7_WN, a.N - 8) * BLOCK_BYTES;
+    const int w_off = k_lo * row_bytes + (RAG ? min(n0 + wave * G7_WN, a.N - 8) : n0 + wave * G7_WN) * BLOCK_BYTES;
     const uint8_t *w_base = a.W + w_off;
     const int w_bytes = a.nb * row_bytes - w_off;                                       // readable from w_base
-    // Columns past N (N % 8 == 0): the lane re-reads the row's last bytes, whose
+    // RAG, columns past N: the lane re-reads the row's last bytes, whose
     // outputs are not stored (a wave wholly past N: any bytes in range).
     const int w_valid = max(16, min(G7_WN, a.N - (n0 + wave * G7_WN)) * BLOCK_BYTES);
-    const int vo_w0 = min(16 * lane, w_valid - 16), vo_w1 = min(1024 + 4 * min(lane, 31), w_valid - 4);
+    const int vo_w0 = RAG ? min(16 * lane, w_valid - 16) : 16 * lane;
+    const int vo_w1 = RAG ? min(1024 + 4 * min(lane, 31), w_valid - 4) : 1024 + 4 * min(lane, 31);
 
     // Copies of a stage: A copies ci = 0..7 of stage s_a, then the raw copies
     // ci = 8..11 of stage s_r: per step t the raw bytes 0..1023 (16 per lane)
@@ -454,13 +456,15 @@ static hipError_t launch_gemm7_t(const _Float16 *X, int64_t ldx, const uint8_t *
     if (e != hipSuccess) return e;
     const uint64_t bit = 1ull << (dev & 63);
     if (!(done.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void *)q4_gemm7_kernel<XT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)G7_LDS);
-        if (e != hipSuccess) return e;
+        for (const void *k : {(const void *)q4_gemm7_kernel<XT, false>, (const void *)q4_gemm7_kernel<XT, true>}) {
+            e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)G7_LDS);
+            if (e != hipSuccess) return e;
+        }
         done.fetch_or(bit, std::memory_order_acq_rel);
     }
     const int ntiles = a.tiles_m * a.tiles_n;
-    hipLaunchKernelGGL(q4_gemm7_kernel<XT>, dim3(ntiles, 1, a.S), dim3(256), G7_LDS, s, a);
+    if (N % G7_BN) hipLaunchKernelGGL((q4_gemm7_kernel<XT, true>), dim3(ntiles, 1, a.S), dim3(256), G7_LDS, s, a);
+    else hipLaunchKernelGGL((q4_gemm7_kernel<XT, false>), dim3(ntiles, 1, a.S), dim3(256), G7_LDS, s, a);
     if (a.S > 1) {
         const int64_t n4 = (int64_t)ntiles * (G7_BM * G7_BN / 4);
         hipLaunchKernelGGL(q4_gemm7_reduce_kernel<XT>, dim3((unsigned)((n4 + 256 * G7_RV - 1) / (256 * G7_RV))),

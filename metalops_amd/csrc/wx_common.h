@@ -65,7 +65,12 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     }
 }
 
-// What a lane loads of the weights for one K step and TN column tiles.
+// What a lane holds of the weights for one K step and TN column tiles: in flight
+// (WxFly) and ready for wx_values (WxRaw).  q4_0: the same.  INT4 and INT8: a
+// wave's 64 columns of a step's 16 (32) byte rows come as one (two) 16-byte loads
+// per lane, four lanes on one row, and go through a wave's own LDS scratch to the
+// lanes that own the columns (taken there directly, a row at a time, they are 8
+// (16) loads of two bytes).
 template <int WT, int TN>
 struct WxRaw;
 template <int TN>
@@ -83,11 +88,23 @@ struct WxRaw<WX_I8, TN> {
     uint32_t q[16];
     uint32_t s[TN], z[TN];
 };
+template <int WT, int TN>
+struct WxFly {
+    static_assert(TN == 2, "64 columns per wave");
+    uint4_t v[WT == WX_I4 ? 1 : 2];
+    uint32_t s[TN], z[TN];
+};
+template <int TN>
+struct WxFly<WX_Q4, TN> : WxRaw<WX_Q4, TN> {};
+
+// LDS scratch per wave: the step's rows of 64 bytes, the upper half of them (the
+// lanes l / 32 = 1 read it) 64 bytes further on, on other banks.
+constexpr int wx_scratch(int wt) { return wt == WX_Q4 ? 0 : (wt == WX_I4 ? 1024 : 2048) + 64; }
 
 // The lane's place in the weights: its columns and the address of K step 0.
-// q4_0: tile j's column is n0 + 32 j + l % 32.  INT4 and INT8: n0 + TN (l % 32) + j, so one
-// load of a byte row serves every tile.  Lanes past N take the last columns
-// again (the same values; what they store there is identical).
+// q4_0: tile j's column is n0 + 32 j + l % 32.  INT4 and INT8: p = 2 (l % 32) + j of the
+// wave's 64, in chunks of 16 columns that end at N at the latest (a chunk that
+// would not is moved back: its columns are computed twice, with equal results).
 template <int WT, int TN>
 struct WxLane {
     int n[TN];
@@ -97,7 +114,7 @@ struct WxLane {
 template <int WT, int TN>
 __device__ __forceinline__ WxLane<WT, TN> wx_lane(const WxArgs &a, int n0, int lane) {
     WxLane<WT, TN> L;
-    const int c = lane & 31, hi = lane >> 5;
+    const int c = lane & 31;
     if constexpr (WT == WX_Q4) {
         L.n0 = min(n0, a.N - 1);
 #pragma unroll
@@ -106,11 +123,10 @@ __device__ __forceinline__ WxLane<WT, TN> wx_lane(const WxArgs &a, int n0, int l
             L.off[j] = (uint32_t)(L.n[j] - L.n0) * BLOCK_BYTES;
         }
     } else {
-        L.n0 = min(n0, a.N - TN);
-        const int nb = min(n0 + TN * c, a.N - TN);
+        L.n0 = min(n0, a.N - 16);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) L.n[j] = nb + j;
-        L.off[0] = (uint32_t)hi * (WT == WX_I4 ? 8u : 16u) * (uint32_t)a.N + (uint32_t)(nb - L.n0);
+        for (int j = 0; j < TN; ++j) L.n[j] = min(n0 + 16 * (c >> 3), a.N - 16) + ((2 * c + j) & 15);
+        L.off[0] = (uint32_t)(lane >> 2) * (uint32_t)a.N + (uint32_t)(min(n0 + 16 * (lane & 3), a.N - 16) - L.n0);
     }
     return L;
 }
@@ -118,25 +134,11 @@ __device__ __forceinline__ WxLane<WT, TN> wx_lane(const WxArgs &a, int n0, int l
 template <int TN, bool SZ32>
 __device__ __forceinline__ void wx_load_sz(const void *p, int64_t row, int n, uint32_t (&out)[TN]) {
     if constexpr (SZ32) {
-        const float *q = (const float *)p + row;
-        if constexpr (TN == 2) {
-            const u32x2 v = load_u<u32x2>(q + n);
-            out[0] = v[0]; out[1] = v[1];
-        } else {
-            const uint4_t v = load_u<uint4_t>(q + n);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) out[j] = v[j];
-        }
+        const u32x2 v = load_u<u32x2>((const float *)p + row + n);
+        out[0] = v[0]; out[1] = v[1];
     } else {
-        const uint16_t *q = (const uint16_t *)p + row;
-        if constexpr (TN == 2) {
-            const uint32_t v = load_u<uint32_t>(q + n);
-            out[0] = v & 0xFFFFu; out[1] = v >> 16;
-        } else {
-            const u32x2 v = load_u<u32x2>(q + n);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) out[j] = (v[j / 2] >> (16 * (j & 1))) & 0xFFFFu;
-        }
+        const uint32_t v = load_u<uint32_t>((const uint16_t *)p + row + n);
+        out[0] = v & 0xFFFFu; out[1] = v >> 16;
     }
 }
 
@@ -145,10 +147,10 @@ __device__ __forceinline__ int wx_group(const WxArgs &a, int k) {
     return (int)(__umulhi((uint32_t)k, a.spg_mul) + ((uint32_t)k & a.spg_one));
 }
 
-// Loads K step `kb`.  TAIL: rows past K are clamped to the last
-// one (wx_dequant zeroes their weights).
+// Loads K step `kb`.  TAIL: rows past K are clamped to the last one (wx_values
+// zeroes their weights).
 template <int WT, int TN, bool SZ32, bool TAIL>
-__device__ __forceinline__ void wx_load(WxRaw<WT, TN> &r, const WxArgs &a, const WxLane<WT, TN> &L, int kb, int lane) {
+__device__ __forceinline__ void wx_load(WxFly<WT, TN> &r, const WxArgs &a, const WxLane<WT, TN> &L, int kb, int lane) {
     if constexpr (WT == WX_Q4) {
         const uint8_t *base = a.W + ((int64_t)kb * a.N + L.n0) * BLOCK_BYTES;
         const int hi = lane >> 5;
@@ -160,21 +162,44 @@ __device__ __forceinline__ void wx_load(WxRaw<WT, TN> &r, const WxArgs &a, const
             r.q[j][0] = v[0]; r.q[j][1] = v[1];
         }
     } else {
-        constexpr int ROWS = WT == WX_I4 ? 8 : 16;
-        const uint8_t *base = a.W + (int64_t)kb * (2 * ROWS) * a.N + L.n0;
-        const int last = (WT == WX_I4 ? a.K / 2 : a.K) - 1 - kb * 2 * ROWS;   // last valid row of the step
-        const int hi = lane >> 5;
+        constexpr int LD = WT == WX_I4 ? 1 : 2;
+        const uint8_t *base = a.W + (int64_t)kb * (16 * LD) * a.N + L.n0;
 #pragma unroll
-        for (int i = 0; i < ROWS; ++i) {
-            const uint8_t *p;
-            if constexpr (TAIL) p = base + (int64_t)min(hi * ROWS + i, last) * a.N + (L.off[0] - (uint32_t)hi * ROWS * (uint32_t)a.N);
-            else p = base + (int64_t)i * a.N + L.off[0];
-            if constexpr (TN == 2) r.q[i] = load_u<uint16_t>(p);
-            else r.q[i] = load_u<uint32_t>(p);
+        for (int h = 0; h < LD; ++h) {
+            const uint8_t *p = base + (int64_t)(16 * h) * a.N + L.off[0];
+            if constexpr (TAIL) {                // back from row 16 h + lane / 4 to the last valid one
+                const int over = kb * 16 * LD + 16 * h + (lane >> 2) - ((WT == WX_I4 ? a.K / 2 : a.K) - 1);
+                p -= (int64_t)max(over, 0) * a.N;
+            }
+            r.v[h] = load_u<uint4_t>(p);
         }
         const int64_t row = (int64_t)wx_group(a, kb) * a.N;
         wx_load_sz<TN, SZ32>(a.scales, row, L.n[0], r.s);
         wx_load_sz<TN, SZ32>(a.zeros, row, L.n[0], r.z);
+    }
+}
+
+// A step's weights from flight to the lanes of their columns.
+template <int WT, int TN>
+__device__ __forceinline__ WxRaw<WT, TN> wx_ready(const WxFly<WT, TN> &f, uint8_t *scratch, int lane) {
+    if constexpr (WT == WX_Q4) {
+        return f;
+    } else {
+        WxRaw<WT, TN> r;
+        const int lrow = lane & 31, hi = lane >> 5;
+        if constexpr (WT == WX_I4) {
+            *(uint4_t *)(scratch + 16 * lane + 64 * hi) = f.v[0];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) r.q[i] = *(const uint16_t *)(scratch + hi * (512 + 64) + 64 * i + 2 * lrow);
+        } else {
+            *(uint4_t *)(scratch + 16 * lane) = f.v[0];
+            *(uint4_t *)(scratch + 1024 + 64 + 16 * lane) = f.v[1];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) r.q[i] = *(const uint16_t *)(scratch + hi * (1024 + 64) + 64 * i + 2 * lrow);
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) { r.s[j] = f.s[j]; r.z[j] = f.z[j]; }
+        return r;
     }
 }
 

@@ -28,14 +28,14 @@ namespace mcq4 {
 
 constexpr int WG_BM = 128, WG_BN = 256, WG_TM = 4, WG_TN = 2;
 constexpr int WG_SLOT = WG_BM * 256;
-constexpr size_t WG_LDS = 4 * 2 * 2 * WG_TN * 16 * 64 * 4;   // phase sum: 4 column groups x 2 halves, 128 KB (the slots: 64)
-static_assert(WG_LDS >= 2 * WG_SLOT && WG_LDS <= 160 * 1024, "LDS budget");
+constexpr size_t WG_LDS = 4 * 2 * 2 * WG_TN * 16 * 64 * 4;   // phase sum: 4 column groups x 2 halves, 128 KB (the loop: 64 + scratch)
+static_assert(WG_LDS >= 2 * WG_SLOT + 8 * wx_scratch(WX_I8) && WG_LDS <= 160 * 1024, "LDS budget");
 
 template <int WT, int XT, bool SZ32, bool ANY, bool ACT>
 __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
     constexpr int ES = XT == DT_F32 ? 4 : 2;
     constexpr int SPW = XT == DT_F32 ? 1 : 2;    // K steps of 32 per wave and stage
-    constexpr int R = WT == WX_I8 ? 2 : 4;       // ring slots: R - 1 steps in flight (INT8: 20 registers a step)
+    constexpr int R = 4;                         // ring slots: R - 1 steps in flight
     extern __shared__ __attribute__((aligned(16))) uint8_t sA[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -82,8 +82,9 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
 
     // This wave's u-th K step (of the split's nk) and its weights.
     auto kstep = [&](int u) { return u / SPW * (2 * SPW) + ph * SPW + u % SPW; };
-    WxRaw<WT, WG_TN> raw[R];
-    auto load_w = [&](WxRaw<WT, WG_TN> &r, int u) {
+    WxFly<WT, WG_TN> raw[R];
+    uint8_t *const scratch = sA + 2 * WG_SLOT + wave * wx_scratch(WT);
+    auto load_w = [&](WxFly<WT, WG_TN> &r, int u) {
         wx_load<WT, WG_TN, SZ32, ANY && WT != WX_Q4>(r, a, L, k_lo + min(kstep(u), nk - 1), lane);
     };
 
@@ -95,7 +96,8 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    auto step = [&](int slot, int t, int u, const WxRaw<WT, WG_TN> &r) {
+    auto step = [&](int slot, int t, int u, const WxFly<WT, WG_TN> &f) {
+        const WxRaw<WT, WG_TN> r = wx_ready<WT, WG_TN>(f, scratch, lane);
         const int valid = a.K - (k_lo + kstep(u)) * 32 - 16 * lhi;
         const uint16_t *d = nullptr;
         if constexpr (WT == WX_Q4) d = r.d;
@@ -190,7 +192,7 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
 #pragma unroll
         for (int j = 0; j < WG_TN; ++j) {
             const int n = L.n[j];
-            const bool ok = n0 + (WT == WX_Q4 ? 32 * j + lrow : WG_TN * lrow) < a.N;
+            const bool ok = n0 + (WT == WX_Q4 ? 32 * j + lrow : 16 * (lrow >> 3)) < a.N;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = m0 + 64 * ph + 32 * i + 8 * (r >> 2) + 4 * lhi + (r & 3);
@@ -246,12 +248,10 @@ static hipError_t launch_wx_gemm_s(const WxArgs &a, int x_dt, bool any, dim3 gri
     return launch_wx_gemm_t<WT, DT_F32, SZ32>(a, any, grid, s);
 }
 
-// K splits: one workgroup per CU, at least 8 K steps of 32 each.
+// K splits: as many as keep one workgroup per CU, at least 8 K steps of 32 each.
 int wx_gemm_splits(int64_t M, int64_t K, int64_t N) {
     const int64_t t = ((M + WG_BM - 1) / WG_BM) * ((N + WG_BN - 1) / WG_BN), nks = (K + 31) / 32;
-    int S = 1;
-    while (t * S * 2 <= 256 && nks / (S * 2) >= 8 && S < 16) S *= 2;
-    return S;
+    return (int)std::max<int64_t>(1, std::min<int64_t>({256 / t, nks / 8, 16}));
 }
 
 hipError_t launch_wx_gemm(WxArgs a, int wt, int x_dt, bool any, hipStream_t s) {

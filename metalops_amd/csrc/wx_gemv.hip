@@ -131,8 +131,8 @@ __global__ void __launch_bounds__(NW * 64) wx_gemv_kernel(WxArgs a) {
 
 template <int XT, int TN>
 static hipError_t launch_wx_gemv_t(const WxArgs &a, bool any, hipStream_t s) {
-    // fp32 steps need more than the 128 registers a 16-wave workgroup has.
-    constexpr int NW = XT == DT_F32 ? 8 : 16;
+    // fp32 steps, and bf16 ones of 64 columns, need more than the 128 registers a 16-wave workgroup has.
+    constexpr int NW = XT == DT_F32 || (XT == DT_BF16 && TN == 4) ? 8 : 16;
     const dim3 grid((a.N + 16 * TN - 1) / (16 * TN));
     if (any) hipLaunchKernelGGL((wx_gemv_kernel<XT, TN, NW, true>), grid, dim3(NW * 64), 0, s, a);
     else hipLaunchKernelGGL((wx_gemv_kernel<XT, TN, NW, false>), grid, dim3(NW * 64), 0, s, a);

@@ -32,8 +32,8 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
     constexpr int ES = XT == DT_F32 ? 4 : 2;
     constexpr int XV = XT == DT_F32 ? 4 : 2;     // 16-byte activation loads per row tile and step
     // Ring slots: R - 1 K steps in flight beside the one in work.
-    constexpr int R = TM == 2 && (WT == WX_I8 || XT == DT_F32) ? 2 : 4;
-    extern __shared__ __attribute__((aligned(16))) float red[];   // [waves][TM TN][16][64]
+    constexpr int R = TM == 2 && XT == DT_F32 ? 2 : 4;
+    extern __shared__ __attribute__((aligned(16))) float red[];   // [waves][TM TN][16][64]; the loop: the waves' scratch
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lrow = lane & 31, lhi = lane >> 5;
@@ -43,12 +43,13 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
     const int k_lo = (int)((int64_t)nks * ws / wt), nk = (int)((int64_t)nks * (ws + 1) / wt) - k_lo;
 
     const WxLane<WT, TN> L = wx_lane<WT, TN>(a, n0, lane);
+    uint8_t *const scratch = (uint8_t *)red + wave * wx_scratch(WT);
     const uint8_t *xrow[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) xrow[i] = (const uint8_t *)a.X + (int64_t)min(32 * i + lrow, a.M - 1) * a.ldx * ES;
 
     struct Step {
-        WxRaw<WT, TN> r;
+        WxFly<WT, TN> r;
         uint4_t x[TM][XV];
     } ring[R];
     auto load = [&](Step &p, int kk) {
@@ -80,15 +81,16 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
 #pragma unroll
                 for (int ks = 0; ks < 2; ++ks) p.x[i][ks] = wx_order<WT>(p.x[i][ks]);
         }
+        const WxRaw<WT, TN> raw = wx_ready<WT, TN>(p.r, scratch, lane);
         const uint16_t *d = nullptr;
-        if constexpr (WT == WX_Q4) d = p.r.d;
+        if constexpr (WT == WX_Q4) d = raw.d;
         wx_if_finite<WT, XT, TN>(d, [&](auto fin) {
             constexpr bool FIN = decltype(fin)::value;
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 if constexpr (XT == DT_F32) {
                     float w[16];
-                    wx_values<WT, XT, TN, SZ32, ANY, FIN>(p.r, j, a.sz_dt, valid, w);
+                    wx_values<WT, XT, TN, SZ32, ANY, FIN>(raw, j, a.sz_dt, valid, w);
 #pragma unroll
                     for (int s = 0; s < 16; ++s) {
                         const int e = wx_slot<WT>(s);
@@ -98,7 +100,7 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
                     }
                 } else {
                     uint4_t B[2];
-                    wx_operands<WT, XT, TN, SZ32, ANY, FIN>(p.r, j, a.sz_dt, valid, B);
+                    wx_operands<WT, XT, TN, SZ32, ANY, FIN>(raw, j, a.sz_dt, valid, B);
 #pragma unroll
                     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
@@ -124,6 +126,7 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
         }
     }
 
+    if constexpr (WT != WX_Q4) __syncthreads();   // every wave is done with its scratch
     // Wave sums: lane l holds rows 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of each tile.
     constexpr int T = TM * TN;
 #pragma unroll
@@ -138,9 +141,9 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
     for (int v = tid; v < T * 1024; v += WS_NW * 64) {
         const int t = v >> 10, r = (v >> 6) & 15, i = t / TN, j = t % TN;
         const int m = 32 * i + 8 * (r >> 2) + 4 * lhi + (r & 3);
-        const int c0 = n0 + (WT == WX_Q4 ? 32 * j + lrow : TN * lrow);
+        const int c0 = n0 + (WT == WX_Q4 ? 32 * j + lrow : 16 * (lrow >> 3));
         if (m >= a.M || c0 >= a.N) continue;
-        const int n = WT == WX_Q4 ? c0 : min(c0, a.N - TN) + j;
+        const int n = WT == WX_Q4 ? c0 : min(c0, a.N - 16) + ((2 * lrow + j) & 15);
         float sum = red[v];
 #pragma unroll
         for (int w = 1; w < WS_NW; ++w) sum += red[w * T * 1024 + v];
@@ -218,12 +221,12 @@ size_t wx_workspace_bytes(int wt, int x_dt, int64_t M, int64_t K, int64_t N) {
            (wx_mid_shape(wt, x_dt, M, N) ? wx_mid_flag_bytes(N, S) : 0);
 }
 
-// Every q4_0 call; INT4 and INT8 with groups of whole K steps, at least one pair
-// of columns (a lane loads two at a time), 16 rows within a 32-bit offset and a
+// Every q4_0 call; INT4 and INT8 with groups of whole K steps, at least 16
+// columns (a lane loads 16 at a time), 16 rows within a 32-bit offset and a
 // K that keeps the group's multiply-high exact.  The fused
 // activations exist for INT4 x fp16 only.
 bool wx_supported(const WxCall &c) {
-    if (c.wt != WX_Q4 && (c.gs % 32 != 0 || c.N < 2 || c.N > (1 << 27) || c.K > 65535 * 32)) return false;
+    if (c.wt != WX_Q4 && (c.gs % 32 != 0 || c.N < 16 || c.N > (1 << 27) || c.K > 65535 * 32)) return false;
     if (c.act != ACT_NONE && (c.wt != WX_I4 || c.x_dt != DT_F16)) return false;
     return true;
 }
