@@ -59,8 +59,9 @@ __device__ __forceinline__ _Float16 rms_apply(_Float16 x, float rstd, _Float16 w
 
 // With NORM the row is the raw activation row of a fused RMSNorm: each element
 // is normalised as the kernel normalised it (rms_apply with the row's rstd and
-// the norm weight wn) before the product.
-template <int WB, bool NORM = false>
+// the norm weight wn) before the product.  BF16: xrow points at bf16
+// elements and the weight is rounded to bf16, as the kernels' operand is.
+template <int WB, bool NORM = false, bool BF16 = false>
 __device__ __forceinline__ float i4_dot_range(const _Float16 *xrow, const uint8_t *P, const void *scales,
                                            const void *zeros, int sz_dt, int N, int gs, int n, int k0,
                                            int k1, const _Float16 *wn = nullptr, float rstd = 0.f) {
@@ -70,8 +71,11 @@ __device__ __forceinline__ float i4_dot_range(const _Float16 *xrow, const uint8_
         if constexpr (WB == 4) q = (float)((P[(int64_t)(k >> 1) * N + n] >> (4 * (k & 1))) & 0xF);
         else q = (float)(int8_t)P[(int64_t)k * N + n];
         const int64_t gi = (int64_t)(k / gs) * N + n;
-        const _Float16 x = NORM ? rms_apply(xrow[k], rstd, wn[k]) : xrow[k];
-        acc += (float)x * ((q - load_dt(zeros, gi, sz_dt)) * load_dt(scales, gi, sz_dt));
+        float x;
+        if constexpr (BF16) x = bf16_bits_to_f32(((const uint16_t *)xrow)[k]);
+        else x = (float)(NORM ? rms_apply(xrow[k], rstd, wn[k]) : xrow[k]);
+        const float w = (q - load_dt(zeros, gi, sz_dt)) * load_dt(scales, gi, sz_dt);
+        acc += x * (BF16 ? round_dt(w, DT_BF16) : w);
     }
     return acc;
 }

@@ -4,7 +4,7 @@
 // i4_gemm_reduce_kernel (which applies the fused activation).
 #pragma once
 
-#include "i4_common.h"
+#include "q4_prefill.h"
 
 namespace mcq4 {
 
@@ -22,6 +22,36 @@ inline uint32_t i4_spg_magic(int spg) {
     return spg > 1 ? (uint32_t)((((uint64_t)1 << 32) + (uint64_t)spg - 1) / (uint64_t)spg) : 0u;
 }
 inline uint32_t i4_spg_ident(int spg) { return spg == 1 ? 0xFFFFFFFFu : 0u; }
+
+// A column's scale and zero as the prefill kernels apply them to a pair of
+// weights q (exact in fp16).  fp16 activations: q s + c in one packed FMA, c =
+// fp16(-z s).  bf16 activations: (q - z) s in the two fp32 roundings of the
+// general kernels, then one packed conversion.
+template <int XT>
+struct I4Scale {
+    half2_t s2, c2;
+    __device__ __forceinline__ void set(float s, float z) {
+        const _Float16 sh = (_Float16)s, ch = (_Float16)(-z * s);
+        s2 = half2_t{sh, sh};
+        c2 = half2_t{ch, ch};
+    }
+    __device__ __forceinline__ uint32_t weights(half2_t q) const {
+        return bitcast<uint32_t>(__builtin_elementwise_fma(q, s2, c2));
+    }
+};
+template <>
+struct I4Scale<DT_BF16> {
+    float s, z;
+    __device__ __forceinline__ void set(float sv, float zv) {
+        s = sv;
+        z = zv;
+    }
+    __device__ __forceinline__ uint32_t weights(half2_t q) const {
+#pragma clang fp contract(off)
+        const float2_t w = {((float)q[0] - z) * s, ((float)q[1] - z) * s};
+        return bitcast<uint32_t>(__builtin_convertvector(w, bf16x2_t));
+    }
+};
 
 struct I4GemmArgs {
     const _Float16 *X;
@@ -43,7 +73,7 @@ struct I4GemmArgs {
     uint32_t foreign = 0;    // splits treated as run on another XCD (test switch)
 };
 
-// Sums the S partial tiles per output tile in split order and stores act(sum) as fp16.
-hipError_t launch_i4_gemm_reduce(const I4GemmArgs &a, int bm, int act, hipStream_t s);
+// Sums the S partial tiles per output tile in split order and stores act(sum) as x_dt.
+hipError_t launch_i4_gemm_reduce(const I4GemmArgs &a, int bm, int act, int x_dt, hipStream_t s);
 
 }  // namespace mcq4

@@ -326,8 +326,8 @@ i4_gemm_kernel(I4GemmArgs a) {
 }
 
 // Sums the S fp32 partial tiles of every output tile in split order and stores
-// act(sum) as fp16; four consecutive columns per thread.
-template <int BM, int ACT>
+// act(sum) as XT; four consecutive columns per thread.
+template <int XT, int BM, int ACT>
 __global__ void __launch_bounds__(256)
 i4_gemm_reduce_kernel(I4GemmArgs a) {
     constexpr int TILE = BM * I4G_BN;
@@ -344,21 +344,34 @@ i4_gemm_reduce_kernel(I4GemmArgs a) {
     if (m >= a.M || n >= a.N) return;
     half4_t v;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) v[c] = (_Float16)activate<ACT>(sum[c]);
+    for (int c = 0; c < 4; ++c) v[c] = out16<XT>(activate<ACT>(sum[c]));
     *(half4_t *)((_Float16 *)a.Y + (int64_t)m * a.ldy + n) = v;
 }
 
-hipError_t launch_i4_gemm_reduce(const I4GemmArgs &a, int bm, int act, hipStream_t s) {
+template <int XT, int BM>
+static void launch_reduce(const I4GemmArgs &a, int act, dim3 grid, hipStream_t s) {
+    if constexpr (XT == DT_F16) {
+        if (act == ACT_SILU) {
+            hipLaunchKernelGGL((i4_gemm_reduce_kernel<XT, BM, ACT_SILU>), grid, dim3(256), 0, s, a);
+            return;
+        }
+        if (act == ACT_GELU) {
+            hipLaunchKernelGGL((i4_gemm_reduce_kernel<XT, BM, ACT_GELU>), grid, dim3(256), 0, s, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((i4_gemm_reduce_kernel<XT, BM, ACT_NONE>), grid, dim3(256), 0, s, a);
+}
+
+hipError_t launch_i4_gemm_reduce(const I4GemmArgs &a, int bm, int act, int x_dt, hipStream_t s) {
     const int64_t n4 = (int64_t)a.tiles_m * a.tiles_n * (bm * I4G_BN / 4);
     const dim3 grid((unsigned)((n4 + 255) / 256));
-    if (bm == 256) {
-        if (act == ACT_SILU) hipLaunchKernelGGL((i4_gemm_reduce_kernel<256, ACT_SILU>), grid, dim3(256), 0, s, a);
-        else if (act == ACT_GELU) hipLaunchKernelGGL((i4_gemm_reduce_kernel<256, ACT_GELU>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((i4_gemm_reduce_kernel<256, ACT_NONE>), grid, dim3(256), 0, s, a);
+    if (x_dt == DT_BF16) {
+        if (bm == 256) launch_reduce<DT_BF16, 256>(a, act, grid, s);
+        else launch_reduce<DT_BF16, 128>(a, act, grid, s);
     } else {
-        if (act == ACT_SILU) hipLaunchKernelGGL((i4_gemm_reduce_kernel<128, ACT_SILU>), grid, dim3(256), 0, s, a);
-        else if (act == ACT_GELU) hipLaunchKernelGGL((i4_gemm_reduce_kernel<128, ACT_GELU>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((i4_gemm_reduce_kernel<128, ACT_NONE>), grid, dim3(256), 0, s, a);
+        if (bm == 256) launch_reduce<DT_F16, 256>(a, act, grid, s);
+        else launch_reduce<DT_F16, 128>(a, act, grid, s);
     }
     return hipGetLastError();
 }
@@ -382,7 +395,7 @@ static hipError_t launch_i4g(const I4GemmArgs &a, hipStream_t s) {
     }
     hipLaunchKernelGGL((i4_gemm_kernel<BM, SZ, ACT, WB>), dim3(a.tiles_m * a.tiles_n, 1, a.S),
                        dim3(256), lds, s, a);
-    if (a.S > 1) return launch_i4_gemm_reduce(a, BM, ACT, s);
+    if (a.S > 1) return launch_i4_gemm_reduce(a, BM, ACT, DT_F16, s);
     return hipGetLastError();
 }
 
@@ -432,14 +445,14 @@ bool i4_gemm6_supported(int wb, int sz_dt, int64_t M, int64_t K, int64_t N, int6
 size_t i4_gemm6_workspace_bytes(int64_t M, int64_t K, int64_t N);
 hipError_t launch_i4_gemm6(const _Float16 *X, int64_t ldx, const uint8_t *P, const void *scales,
                            const void *zeros, int sz_dt, _Float16 *Y, int64_t ldy, int M, int K, int N,
-                           int gs, int act, void *ws, hipStream_t s);
+                           int gs, int act, int x_dt, void *ws, hipStream_t s);
 
 bool i4_gemm7_supported(int wb, int sz_dt, int64_t M, int64_t K, int64_t N, int64_t gs, const _Float16 *X,
                         int64_t ldx, const void *Y, int64_t ldy);
 size_t i4_gemm7_workspace_bytes(int64_t M, int64_t K, int64_t N);
 hipError_t launch_i4_gemm7(const _Float16 *X, int64_t ldx, const uint8_t *P, const void *scales,
                            const void *zeros, int sz_dt, _Float16 *Y, int64_t ldy, int M, int K, int N,
-                           int gs, int act, void *ws, hipStream_t s);
+                           int gs, int act, int x_dt, void *ws, hipStream_t s);
 
 // Covers the three prefill kernels (i4_gemm7 and i4_gemm6 for 4-bit weights
 // with 16-bit scales/zeros, this one otherwise).
@@ -454,9 +467,9 @@ hipError_t launch_i4_gemm(const _Float16 *X, int64_t ldx, const uint8_t *P, cons
                           const void *zeros, int sz_dt, _Float16 *Y, int64_t ldy, int M, int K,
                           int N, int gs, int act, void *ws, hipStream_t s, int wb) {
     if (i4_gemm7_supported(wb, sz_dt, M, K, N, gs, X, ldx, Y, ldy))
-        return launch_i4_gemm7(X, ldx, P, scales, zeros, sz_dt, Y, ldy, M, K, N, gs, act, ws, s);
+        return launch_i4_gemm7(X, ldx, P, scales, zeros, sz_dt, Y, ldy, M, K, N, gs, act, DT_F16, ws, s);
     if (i4_gemm6_supported(wb, sz_dt, M, K, N, gs, ldx, Y, ldy))
-        return launch_i4_gemm6(X, ldx, P, scales, zeros, sz_dt, Y, ldy, M, K, N, gs, act, ws, s);
+        return launch_i4_gemm6(X, ldx, P, scales, zeros, sz_dt, Y, ldy, M, K, N, gs, act, DT_F16, ws, s);
     const I4GCfg c = i4_gemm_config(M, K, N);
     I4GemmArgs a;
     a.X = X; a.ldx = ldx; a.P = P; a.scales = scales; a.zeros = zeros; a.Y = Y; a.ldy = ldy;
@@ -475,6 +488,28 @@ hipError_t launch_i4_gemm(const _Float16 *X, int64_t ldx, const uint8_t *P, cons
     }
     if (c.bm == 256) return launch_i4g_sz<256, 4>(a, sz_dt, act, s);
     return launch_i4g_sz<128, 4>(a, sz_dt, act, s);
+}
+
+// bf16 activations, 4-bit weights with 16-bit scales and zeros: i4_gemm7 and
+// i4_gemm6 on the bf16 MFMA, in the shapes and alignments they take, where the
+// (optional) workspace covers their splits.
+size_t i4_gemm_bf16_workspace_bytes(int64_t M, int64_t K, int64_t N) {
+    return std::max(i4_gemm6_workspace_bytes(M, K, N), i4_gemm7_workspace_bytes(M, K, N));
+}
+
+bool i4_gemm_bf16_supported(const void *X, int64_t ldx, const void *P, const void *scales, const void *zeros, int sz_dt,
+                            const void *Y, int64_t ldy, int64_t M, int64_t K, int64_t N, int64_t gs) {
+    return K / 32 < (1 << 16) && i4_gemm_supported(K, N, gs, X, ldx, P, scales, zeros, Y, ldy) &&
+           i4_gemm6_supported(4, sz_dt, M, K, N, gs, ldx, Y, ldy);
+}
+
+hipError_t launch_i4_gemm_bf16(const void *X, int64_t ldx, const uint8_t *P, const void *scales, const void *zeros,
+                               int sz_dt, void *Y, int64_t ldy, int M, int K, int N, int gs, void *ws, hipStream_t s) {
+    const _Float16 *x = (const _Float16 *)X;
+    _Float16 *y = (_Float16 *)Y;
+    if (i4_gemm7_supported(4, sz_dt, M, K, N, gs, x, ldx, y, ldy))
+        return launch_i4_gemm7(x, ldx, P, scales, zeros, sz_dt, y, ldy, M, K, N, gs, ACT_NONE, DT_BF16, ws, s);
+    return launch_i4_gemm6(x, ldx, P, scales, zeros, sz_dt, y, ldy, M, K, N, gs, ACT_NONE, DT_BF16, ws, s);
 }
 
 }  // namespace mcq4

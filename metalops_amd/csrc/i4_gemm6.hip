@@ -26,6 +26,11 @@
 //     xcd_ticket_inc).  Otherwise split-K partials and their
 //     reduction (with the fused activation) are i4_gemm's.
 //
+// bf16 activations (XT): the bf16 MFMA; the pair q becomes (q - z) s in fp32 and
+// is packed to bf16, 8 VALU per two weights instead of 4, which bounds it (two
+// waves per SIMD: VALU issue above the 1024 clocks of MFMA per step).  M=256
+// 4096x11008: 55.3 us (fp16 46.8; wx_gemm in bf16 60.9).
+//
 // MFMA 32x32 output layout: lane l holds D[8*(r/4) + 4*(l/32) + r%4][l%32], r = 0..15.
 #include <algorithm>
 #include <atomic>
@@ -57,7 +62,7 @@ __device__ __forceinline__ void j6_copy16(const void *base, int bytes, uint32_t 
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16, voff, soff, 0, 0);
 }
 
-template <int SZ, int ACT>
+template <int XT, int SZ, int ACT>
 __global__ void __launch_bounds__(256, 2)
 i4_gemm6_kernel(I4GemmArgs a) {
     static_assert(SZ == DT_F16 || SZ == DT_BF16, "16-bit scales and zeros");
@@ -158,8 +163,8 @@ i4_gemm6_kernel(I4GemmArgs a) {
     const uint32_t mlo = opaque_sgpr(0x000F000Fu);
     const half2_t m1024 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
 
-    // fp16 scale and offset pairs of the lane's two columns (2 lrow + j).
-    auto scale_pairs = [&](const lds_u8 *Rs, half2_t (&s2)[TN], half2_t (&c2)[TN]) {
+    // Scales and zeros of the lane's two columns (2 lrow + j).
+    auto scale_pairs = [&](const lds_u8 *Rs, I4Scale<XT> (&sc)[TN]) {
         const uint32_t sv = *(const lds_u32 *)(Rs + J6_RAW + 4 * lrow);
         const uint32_t zv = *(const lds_u32 *)(Rs + J6_RAW + 128 + 4 * lrow);
 #pragma unroll
@@ -172,21 +177,19 @@ i4_gemm6_kernel(I4GemmArgs a) {
                 s = __uint_as_float(j ? (sv & 0xFFFF0000u) : (sv << 16));
                 zz = __uint_as_float(j ? (zv & 0xFFFF0000u) : (zv << 16));
             }
-            const _Float16 sh = (_Float16)s, ch = (_Float16)(-zz * s);
-            s2[j] = half2_t{sh, sh};
-            c2[j] = half2_t{ch, ch};
+            sc[j].set(s, zz);
         }
     };
     // Pair of byte row r for tile j: {1024 + q(2r), 1024 + q(2r+1)} of column 2 lrow + j.
-    auto b_pair = [&](uint32_t w, int j, half2_t s2, half2_t c2) {
+    auto b_pair = [&](uint32_t w, int j, const I4Scale<XT> &sc) {
         const uint32_t sel = (uint32_t)j | (uint32_t)j << 8 | (uint32_t)(4 + j) << 16 | (uint32_t)(4 + j) << 24;
         const half2_t q = bitcast<half2_t>(and_or(__builtin_amdgcn_perm(w >> 4, w, sel), mlo, c64)) + m1024;
-        return bitcast<uint32_t>(__builtin_elementwise_fma(q, s2, c2));
+        return sc.weights(q);
     };
     auto load_b = [&](int k, half8_t (&bv)[2][TN]) {
         const lds_u8 *Rs = lds_ptr(lds_addr(ring + (k % J6_RAW_N) * J6_SLOT));
-        half2_t s2[TN], c2[TN];
-        scale_pairs(Rs, s2, c2);
+        I4Scale<XT> sc[TN];
+        scale_pairs(Rs, sc);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             uint32_t w[4];
@@ -196,7 +199,7 @@ i4_gemm6_kernel(I4GemmArgs a) {
             for (int j = 0; j < TN; ++j) {
                 uint4_t d;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) d[r] = b_pair(w[r], j, s2[j], c2[j]);
+                for (int r = 0; r < 4; ++r) d[r] = b_pair(w[r], j, sc[j]);
                 bv[ks][j] = bitcast<half8_t>(d);
             }
         }
@@ -219,13 +222,13 @@ i4_gemm6_kernel(I4GemmArgs a) {
                     half8_t (&Bn)[2][TN], int a_s, int a_t) {
         const lds_u8 *Rs = lds_ptr(lds_addr(ring + (k_next % J6_RAW_N) * J6_SLOT));
         uint32_t w[2][4];
-        half2_t s2[TN], c2[TN];
+        I4Scale<XT> sc[TN];
         uint32_t d[2][TN][4];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int idx = 0; idx < NMF; ++idx) {
             const int ks = idx / (TM * TN), i = (idx / TN) % TM, j = idx % TN;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[ks][i], B[ks][j], acc[i][j], 0, 0, 0);
+            acc[i][j] = mfma32<XT>(A[ks][i], B[ks][j], acc[i][j]);
             if (j == TN - 1) A[ks][i] = read_a1(a_s, a_t, ks, i);
             if constexpr (decltype(with_copies)::value) {
                 if ((idx & 1) == 1 && (idx >> 1) < GROUP) issue_one(cs, idx >> 1);
@@ -236,11 +239,11 @@ i4_gemm6_kernel(I4GemmArgs a) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
                         w[kk][r] = *(const lds_u16 *)(Rs + (8 * kk + 4 * lhi + r) * J6_WN + 2 * lrow);
-                scale_pairs(Rs, s2, c2);
+                scale_pairs(Rs, sc);
             } else if (idx <= 8) {
                 const int c = idx - 1, uk = c >> 2, uj = (c >> 1) & 1, rh = c & 1;
 #pragma unroll
-                for (int r = 2 * rh; r < 2 * rh + 2; ++r) d[uk][uj][r] = b_pair(w[uk][r], uj, s2[uj], c2[uj]);
+                for (int r = 2 * rh; r < 2 * rh + 2; ++r) d[uk][uj][r] = b_pair(w[uk][r], uj, sc[uj]);
                 if (rh == 1) Bn[uk][uj] = bitcast<half8_t>(uint4_t{d[uk][uj][0], d[uk][uj][1], d[uk][uj][2], d[uk][uj][3]});
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -273,7 +276,7 @@ i4_gemm6_kernel(I4GemmArgs a) {
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[ks][i], B0[ks][j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = mfma32<XT>(A[ks][i], B0[ks][j], acc[i][j]);
     }
     wait_vmcnt<0>();
 
@@ -291,7 +294,7 @@ i4_gemm6_kernel(I4GemmArgs a) {
                 if (m < a.M) {
                     half2_t v;
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) v[j] = (_Float16)activate<ACT>(acc[i][j][r]);
+                    for (int j = 0; j < TN; ++j) v[j] = out16<XT>(activate<ACT>(acc[i][j][r]));
                     *(half2_t *)(Y + (int64_t)m * a.ldy + n) = v;
                 }
             }
@@ -345,7 +348,7 @@ i4_gemm6_kernel(I4GemmArgs a) {
 #pragma unroll 1
         for (int v = tid; v < BM * I4G_BN; v += 256) {
             const int m = min(m0 + v / I4G_BN, a.M - 1), nn = min(n0 + v % I4G_BN, N - 1);
-            other[v] = i4_dot_range<4>(a.X + (int64_t)m * a.ldx, a.P, a.scales, a.zeros, SZ, N, a.spg * 32, nn,
+            other[v] = i4_dot_range<4, false, XT == DT_BF16>(a.X + (int64_t)m * a.ldx, a.P, a.scales, a.zeros, SZ, N, a.spg * 32, nn,
                                        o_lo, o_hi);
         }
         wait_vmcnt<0>();
@@ -369,7 +372,7 @@ i4_gemm6_kernel(I4GemmArgs a) {
                 half2_t v;
 #pragma unroll
                 for (int j = 0; j < TN; ++j)     // p0 + p1 in split order
-                    v[j] = (_Float16)activate<ACT>(z == 0 ? acc[i][j][r] + o[r][j] : o[r][j] + acc[i][j][r]);
+                    v[j] = out16<XT>(activate<ACT>(z == 0 ? acc[i][j][r] + o[r][j] : o[r][j] + acc[i][j][r]));
                 *(half2_t *)(Y + (int64_t)m * a.ldy + n) = v;
             }
         }
@@ -415,7 +418,7 @@ size_t i4_gemm6_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     return COUNTER_BYTES + (size_t)t * c.S * J6_BM * I4G_BN * sizeof(float);
 }
 
-template <int SZ, int ACT>
+template <int XT, int SZ, int ACT>
 static hipError_t launch_j6(const I4GemmArgs &a, hipStream_t s) {
     static std::atomic<uint64_t> done{0};
     int dev = 0;
@@ -423,28 +426,30 @@ static hipError_t launch_j6(const I4GemmArgs &a, hipStream_t s) {
     if (e != hipSuccess) return e;
     const uint64_t bit = 1ull << (dev & 63);
     if (!(done.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void *)i4_gemm6_kernel<SZ, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        e = hipFuncSetAttribute((const void *)i4_gemm6_kernel<XT, SZ, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)J6_LDS);
         if (e != hipSuccess) return e;
         done.fetch_or(bit, std::memory_order_acq_rel);
     }
     const int ntiles = a.tiles_m * a.tiles_n;
     const int gx = a.tickets ? (ntiles + 7) / 8 * 8 : ntiles;
-    hipLaunchKernelGGL((i4_gemm6_kernel<SZ, ACT>), dim3(gx, 1, a.S), dim3(256), J6_LDS, s, a);
-    if (a.S > 1 && !a.tickets) return launch_i4_gemm_reduce(a, J6_BM, ACT, s);
+    hipLaunchKernelGGL((i4_gemm6_kernel<XT, SZ, ACT>), dim3(gx, 1, a.S), dim3(256), J6_LDS, s, a);
+    if (a.S > 1 && !a.tickets) return launch_i4_gemm_reduce(a, J6_BM, ACT, XT, s);
     return hipGetLastError();
 }
 
-template <int SZ>
+template <int XT, int SZ>
 static hipError_t launch_j6_act(const I4GemmArgs &a, int act, hipStream_t s) {
-    if (act == ACT_SILU) return launch_j6<SZ, ACT_SILU>(a, s);
-    if (act == ACT_GELU) return launch_j6<SZ, ACT_GELU>(a, s);
-    return launch_j6<SZ, ACT_NONE>(a, s);
+    if constexpr (XT == DT_F16) {            // the fused activations are fp16 calls
+        if (act == ACT_SILU) return launch_j6<XT, SZ, ACT_SILU>(a, s);
+        if (act == ACT_GELU) return launch_j6<XT, SZ, ACT_GELU>(a, s);
+    }
+    return launch_j6<XT, SZ, ACT_NONE>(a, s);
 }
 
 hipError_t launch_i4_gemm6(const _Float16 *X, int64_t ldx, const uint8_t *P, const void *scales,
                            const void *zeros, int sz_dt, _Float16 *Y, int64_t ldy, int M, int K, int N,
-                           int gs, int act, void *ws, hipStream_t s) {
+                           int gs, int act, int x_dt, void *ws, hipStream_t s) {
     const J6Cfg c = i4_gemm6_config(M, K, N);
     I4GemmArgs a;
     a.foreign = split_foreign_mask();
@@ -462,8 +467,12 @@ hipError_t launch_i4_gemm6(const _Float16 *X, int64_t ldx, const uint8_t *P, con
         if (c.S == 2 && !opt_is("MCQ4_XCD_LOCAL", '0') && (a.tiles_m * a.tiles_n + 7) / 8 <= 4096)
             a.tickets = (uint64_t *)ws;
     }
-    if (sz_dt == DT_F16) return launch_j6_act<DT_F16>(a, act, s);
-    return launch_j6_act<DT_BF16>(a, act, s);
+    if (x_dt == DT_BF16) {
+        if (sz_dt == DT_F16) return launch_j6_act<DT_BF16, DT_F16>(a, act, s);
+        return launch_j6_act<DT_BF16, DT_BF16>(a, act, s);
+    }
+    if (sz_dt == DT_F16) return launch_j6_act<DT_F16, DT_F16>(a, act, s);
+    return launch_j6_act<DT_F16, DT_BF16>(a, act, s);
 }
 
 }  // namespace mcq4

@@ -25,6 +25,9 @@
 //   * Split K (grid.z) for outputs with few tiles: fp32 partial tiles summed in
 //     split order, with the fused activation, by i4_gemm_reduce_kernel.
 //
+// bf16 activations (XT): as in i4_gemm6; half the dequant per MFMA.  M=2048
+// 4096x11008: 239.1 us (fp16 226.8; wx_gemm in bf16 282.7).
+//
 // MFMA 32x32 output layout: lane l holds D[8*(r/4) + 4*(l/32) + r%4][l%32], r = 0..15.
 #include <algorithm>
 #include <atomic>
@@ -61,7 +64,7 @@ __device__ __forceinline__ void j7_copy_w(const uint8_t *P, uint32_t so, uint8_t
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16, voff, so, 0, 0);
 }
 
-template <int SZ, int ACT>
+template <int XT, int SZ, int ACT>
 __global__ void __launch_bounds__(256, 1)
 i4_gemm7_kernel(I4GemmArgs a) {
     static_assert(SZ == DT_F16 || SZ == DT_BF16, "16-bit scales and zeros");
@@ -163,9 +166,8 @@ i4_gemm7_kernel(I4GemmArgs a) {
             rw.zv = *(const lds_u32 *)(Rs + J7_RAW + 128 + 4 * lrow);
         }
     };
-    // fp16 scale and offset pair of tile j's column (2 lrow + j): s and
-    // c = fp16(-z * s) (fp32 product).
-    auto scale_pair = [&](const Raw &rw, int j, half2_t &s2, half2_t &c2) {
+    // Scale and zero of tile j's column (2 lrow + j).
+    auto scale_pair = [&](const Raw &rw, int j, I4Scale<XT> &sc) {
         float s, zz;
         if constexpr (SZ == DT_F16) {
             s = (float)bitcast<half2_t>(rw.sv)[j];
@@ -174,9 +176,7 @@ i4_gemm7_kernel(I4GemmArgs a) {
             s = __uint_as_float(j ? (rw.sv & 0xFFFF0000u) : (rw.sv << 16));
             zz = __uint_as_float(j ? (rw.zv & 0xFFFF0000u) : (rw.zv << 16));
         }
-        const _Float16 sh = (_Float16)s, ch = (_Float16)(-zz * s);
-        s2 = half2_t{sh, sh};
-        c2 = half2_t{ch, ch};
+        sc.set(s, zz);
     };
     uint32_t bsel[TN];
 #pragma unroll
@@ -187,8 +187,8 @@ i4_gemm7_kernel(I4GemmArgs a) {
         const half2_t off = {(_Float16)1024.0f, (_Float16)64.0f};
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            half2_t s2, c2;
-            scale_pair(rw, j, s2, c2);
+            I4Scale<XT> sc;
+            scale_pair(rw, j, sc);
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
                 uint4_t d;
@@ -196,7 +196,7 @@ i4_gemm7_kernel(I4GemmArgs a) {
                 for (int r = 0; r < 4; ++r) {
                     const half2_t h = bitcast<half2_t>(and_or(__builtin_amdgcn_perm(rw.w[ks][r], rw.w[ks][r], bsel[j]),
                                                               nib_mask, exp_bits));
-                    d[r] = bitcast<uint32_t>(__builtin_elementwise_fma(h - off, s2, c2));
+                    d[r] = sc.weights(h - off);
                 }
                 bv[ks][j] = bitcast<half8_t>(d);
             }
@@ -224,22 +224,21 @@ i4_gemm7_kernel(I4GemmArgs a) {
                     Raw &rn, int k_read, int a_slot, int a_t) {
 #pragma clang fp contract(off)
         const half2_t off = {(_Float16)1024.0f, (_Float16)64.0f};
-        half2_t s2[TN], c2[TN];
+        I4Scale<XT> sc[TN];
         uint32_t xw[16];
         uint4_t bb[2 * TN];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int idx = 0; idx < NMF; ++idx) {
             const int ks = idx / (TM * TN), i = (idx / TN) % TM, j = idx % TN;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[ks][i], B[ks][j], acc[i][j], 0, 0, 0);
+            acc[i][j] = mfma32<XT>(A[ks][i], B[ks][j], acc[i][j]);
             {
                 const int d = idx >> 1, unit = d >> 2, r = d & 3, uj = unit >> 1, uk = unit & 1;
                 if ((idx & 1) == 0) {
-                    if ((idx & 15) == 0) scale_pair(rc, uj, s2[uj], c2[uj]);
+                    if ((idx & 15) == 0) scale_pair(rc, uj, sc[uj]);
                     xw[d] = and_or(__builtin_amdgcn_perm(rc.w[uk][r], rc.w[uk][r], bsel[uj]), nib_mask, exp_bits);
                 } else {
-                    bb[unit][r] = bitcast<uint32_t>(__builtin_elementwise_fma(bitcast<half2_t>(xw[d]) - off,
-                                                                               s2[uj], c2[uj]));
+                    bb[unit][r] = sc[uj].weights(bitcast<half2_t>(xw[d]) - off);
                     if (r == 3) Bn[uk][uj] = bitcast<half8_t>(bb[unit]);
                 }
             }
@@ -300,7 +299,7 @@ i4_gemm7_kernel(I4GemmArgs a) {
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A0[ks][i], B0[ks][j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = mfma32<XT>(A0[ks][i], B0[ks][j], acc[i][j]);
     }
     wait_vmcnt<0>();
 
@@ -318,7 +317,7 @@ i4_gemm7_kernel(I4GemmArgs a) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int m = m0 + i * 32 + 8 * (r >> 2) + rsub + (r & 3);
-                    if (m < a.M && n < N) Y[(int64_t)m * a.ldy + n] = (_Float16)activate<ACT>(acc[i][j][r]);
+                    if (m < a.M && n < N) Y[(int64_t)m * a.ldy + n] = out16<XT>(activate<ACT>(acc[i][j][r]));
                 }
             }
         return;
@@ -373,7 +372,7 @@ size_t i4_gemm7_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     return COUNTER_BYTES + (size_t)t * S * J7_BM * I4G_BN * sizeof(float);
 }
 
-template <int SZ, int ACT>
+template <int XT, int SZ, int ACT>
 static hipError_t launch_j7(const I4GemmArgs &a, hipStream_t s) {
     static std::atomic<uint64_t> done{0};
     int dev = 0;
@@ -381,27 +380,29 @@ static hipError_t launch_j7(const I4GemmArgs &a, hipStream_t s) {
     if (e != hipSuccess) return e;
     const uint64_t bit = 1ull << (dev & 63);
     if (!(done.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void *)i4_gemm7_kernel<SZ, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        e = hipFuncSetAttribute((const void *)i4_gemm7_kernel<XT, SZ, ACT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)J7_LDS);
         if (e != hipSuccess) return e;
         done.fetch_or(bit, std::memory_order_acq_rel);
     }
     const int ntiles = a.tiles_m * a.tiles_n;
-    hipLaunchKernelGGL((i4_gemm7_kernel<SZ, ACT>), dim3(ntiles, 1, a.S), dim3(256), J7_LDS, s, a);
-    if (a.S > 1) return launch_i4_gemm_reduce(a, J7_BM, ACT, s);
+    hipLaunchKernelGGL((i4_gemm7_kernel<XT, SZ, ACT>), dim3(ntiles, 1, a.S), dim3(256), J7_LDS, s, a);
+    if (a.S > 1) return launch_i4_gemm_reduce(a, J7_BM, ACT, XT, s);
     return hipGetLastError();
 }
 
-template <int SZ>
+template <int XT, int SZ>
 static hipError_t launch_j7_act(const I4GemmArgs &a, int act, hipStream_t s) {
-    if (act == ACT_SILU) return launch_j7<SZ, ACT_SILU>(a, s);
-    if (act == ACT_GELU) return launch_j7<SZ, ACT_GELU>(a, s);
-    return launch_j7<SZ, ACT_NONE>(a, s);
+    if constexpr (XT == DT_F16) {            // the fused activations are fp16 calls
+        if (act == ACT_SILU) return launch_j7<XT, SZ, ACT_SILU>(a, s);
+        if (act == ACT_GELU) return launch_j7<XT, SZ, ACT_GELU>(a, s);
+    }
+    return launch_j7<XT, SZ, ACT_NONE>(a, s);
 }
 
 hipError_t launch_i4_gemm7(const _Float16 *X, int64_t ldx, const uint8_t *P, const void *scales,
                            const void *zeros, int sz_dt, _Float16 *Y, int64_t ldy, int M, int K, int N,
-                           int gs, int act, void *ws, hipStream_t s) {
+                           int gs, int act, int x_dt, void *ws, hipStream_t s) {
     I4GemmArgs a;
     a.X = X; a.ldx = ldx; a.P = P; a.scales = scales; a.zeros = zeros; a.Y = Y; a.ldy = ldy;
     a.M = M; a.nsteps = K / 32; a.N = N; a.spg = gs / 32; a.spg_magic = i4_spg_magic(a.spg); a.spg_ident = i4_spg_ident(a.spg);
@@ -413,8 +414,12 @@ hipError_t launch_i4_gemm7(const _Float16 *X, int64_t ldx, const uint8_t *P, con
         if (!ws) return hipErrorInvalidValue;
         a.partials = (float *)((char *)ws + COUNTER_BYTES);
     }
-    if (sz_dt == DT_F16) return launch_j7_act<DT_F16>(a, act, s);
-    return launch_j7_act<DT_BF16>(a, act, s);
+    if (x_dt == DT_BF16) {
+        if (sz_dt == DT_F16) return launch_j7_act<DT_BF16, DT_F16>(a, act, s);
+        return launch_j7_act<DT_BF16, DT_BF16>(a, act, s);
+    }
+    if (sz_dt == DT_F16) return launch_j7_act<DT_F16, DT_F16>(a, act, s);
+    return launch_j7_act<DT_F16, DT_BF16>(a, act, s);
 }
 
 }  // namespace mcq4

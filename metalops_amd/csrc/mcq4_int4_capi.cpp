@@ -45,6 +45,11 @@ size_t i4_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N);
 hipError_t launch_i4_gemm(const _Float16 *X, int64_t ldx, const uint8_t *P, const void *scales,
                           const void *zeros, int sz_dt, _Float16 *Y, int64_t ldy, int M, int K,
                           int N, int gs, int act, void *ws, hipStream_t s, int wb);
+size_t i4_gemm_bf16_workspace_bytes(int64_t M, int64_t K, int64_t N);
+bool i4_gemm_bf16_supported(const void *X, int64_t ldx, const void *P, const void *scales, const void *zeros, int sz_dt,
+                            const void *Y, int64_t ldy, int64_t M, int64_t K, int64_t N, int64_t gs);
+hipError_t launch_i4_gemm_bf16(const void *X, int64_t ldx, const uint8_t *P, const void *scales, const void *zeros,
+                               int sz_dt, void *Y, int64_t ldy, int M, int K, int N, int gs, void *ws, hipStream_t s);
 hipError_t launch_i4_rmsnorm(const _Float16 *X, int64_t ldx, const _Float16 *w, float eps, int M,
                              int K, _Float16 *out, int64_t ldo, hipStream_t s);
 bool i4_gemv1_rms_supported(int64_t K, int64_t N, int64_t gs, const void *X, const void *wn,
@@ -100,6 +105,14 @@ I4Path i4_path(const void *X, int x_dt, int64_t ldx, const uint8_t *P, const voi
                                                                      : I4Path::Generic;
 }
 
+// bf16 activations, INT4: the prefill kernels' bf16 instances from 65 rows and K =
+// 2048 on, in the shapes they take; wx_gemm otherwise.  us, wx_gemm / these: M=128
+// 4096x4096 28.2 / 26.5, M=256 4096x11008 60.9 / 55.3, M=2048 4096x11008 282.7 /
+// 239.1; K = 1024 (M=200 1024x1024) 17.1 / 21.1.
+bool bf16_prefill(int64_t M, int64_t K, int wb, int x_dt) {
+    return x_dt == MCQ4_DTYPE_BF16 && wb == 4 && M > 64 && K >= 2048;
+}
+
 // Upper bound over the kernels a shape can take (the general kernel needs none).
 size_t ws_bytes(int64_t M, int64_t K, int64_t N, int64_t gs, int x_dt, int wb = 4) {
     const int ks = wb == 4 ? 32 : 16;
@@ -119,7 +132,10 @@ size_t query_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t gs, int x_dt, int
     const size_t need = ws_bytes(M, K, N, gs, x_dt, wb);
     if (M <= 0 || K <= 0 || N <= 0 || gs <= 0 || gs % 32) return need;
     if (x_dt == MCQ4_DTYPE_F16 && N % 128 == 0 && K % 32 == 0) return need;
-    return std::max(need, mcq4::wx_workspace_bytes(wb == 4 ? mcq4::WX_I4 : mcq4::WX_I8, x_dt, M, K, N));
+    const size_t wx = mcq4::wx_workspace_bytes(wb == 4 ? mcq4::WX_I4 : mcq4::WX_I8, x_dt, M, K, N);
+    if (bf16_prefill(M, K, wb, x_dt) && N % 128 == 0 && K % 32 == 0)
+        return std::max({need, wx, mcq4::i4_gemm_bf16_workspace_bytes(M, K, N)});
+    return std::max(need, wx);
 }
 
 int matmul_common(int act, const void *X, int x_dtype, int64_t ldx, const uint8_t *packed,
@@ -147,6 +163,14 @@ int matmul_common(int act, const void *X, int x_dtype, int64_t ldx, const uint8_
     if (path == I4Path::Gemm && (K % 32 || gs % 32)) path = I4Path::Generic;
     const mcq4::WxCall wx = {wb == 4 ? mcq4::WX_I4 : mcq4::WX_I8, x_dtype, sz_dtype, act, X, ldx, packed, scales, zeros,
                              Y, ldy, M, K, N, gs};
+    if (act == 0 && bf16_prefill(M, K, wb, x_dtype) && !mcq4::opt_is("MCQ4_I4_PATH", 'g') &&
+        mcq4::i4_gemm_bf16_supported(X, ldx, packed, scales, zeros, sz_dtype, Y, ldy, M, K, N, gs)) {
+        const size_t use = mcq4::i4_gemm_bf16_workspace_bytes(M, K, N);
+        if (!use || (workspace && workspace_bytes >= use && aligned(workspace, 16)))
+            return hip_status(mcq4::launch_i4_gemm_bf16(X, ldx, packed, scales, zeros, sz_dtype, Y, ldy, (int)M, (int)K,
+                                                        (int)N, (int)gs, workspace, (hipStream_t)stream),
+                              "int4 matmul launch");
+    }
     if (path == I4Path::Generic && !mcq4::opt_is("MCQ4_I4_PATH", 'g') && mcq4::wx_supported(wx)) {
         if (workspace && !aligned(workspace, 16)) workspace = nullptr;   // optional here: K stays whole
         return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, (hipStream_t)stream), "int4 matmul launch");

@@ -1,0 +1,64 @@
+"""INT4 products of bf16 activations on the prefill kernels (the bf16 instances of
+csrc/i4_gemm6.hip and i4_gemm7.hip).
+
+Bar per output: W is the oracle's dequantized weight rounded once to X's dtype
+(bit-exact in the kernels), so only fp32 sums and the output's rounding remain:
+|Y - Y64| <= u |Y64| + K 2^-24 sum|x w|, u = 2^-8 (bf16), 2^-11 (fp16); a fused
+activation (slope at most 1.13, fp32 evaluation) adds 2^-20 |y| and scales the second
+term by 1.13.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import int4_ref as R
+
+pytestmark = pytest.mark.gpu
+
+TDT = {R.F16: torch.float16, R.BF16: torch.bfloat16}
+ULP = {R.F16: 2.0 ** -11, R.BF16: 2.0 ** -8}
+ACT = {None: lambda y: y, "silu": lambda y: y / (1 + np.exp(-y)),
+       "gelu": lambda y: 0.5 * y * (1 + np.tanh(np.sqrt(2 / np.pi) * (y + 0.044715 * y ** 3)))}
+
+
+def _check(Y, X, W, xdt, act=None):
+    X = X.double().numpy()
+    W = np.asarray(W, np.float64)
+    y = X @ W
+    Yr, S = ACT[act](y), np.abs(X) @ np.abs(W)
+    Y = Y.double().cpu().numpy()
+    assert np.isfinite(Y).all()
+    bound = ULP[xdt] * np.abs(Yr) + 1.13 * X.shape[1] * 2.0 ** -24 * S + (2.0 ** -20 * np.abs(y) if act else 0) + 1e-30
+    bad = np.abs(Y - Yr) / bound
+    assert bad.max() <= 1, f"err/bound {bad.max():.3g} at {np.unravel_index(bad.argmax(), bad.shape)}"
+
+
+def _int4(dev, M, K, N, gs, xdt, sdt):
+    w = R.round_to(np.random.default_rng(M * 3 + N).standard_normal((K, N), np.float32) * 0.02, sdt)
+    p, s, z = R.quantize(w, gs, sdt)
+    X = torch.randn(M, K, generator=torch.Generator().manual_seed(M + K)).to(TDT[xdt])
+    args = [torch.from_numpy(p).to(dev)] + [torch.from_numpy(np.asarray(t, np.float32)).to(TDT[sdt]).to(dev) for t in (s, z)]
+    return X, args, R.dequantize(p, s, z, gs, xdt)
+
+
+# Rows around the line (64 / 65), the 128-row tile and the second tile; columns of one
+# wave pair, of a workgroup with waves past N and of whole tiles; an odd number of K
+# steps; eight, two and one K splits; the 256-row kernel by its switch.
+@pytest.mark.parametrize("M,K,N,gs,sdt,env", [
+    (65, 2048, 128, 128, R.BF16, {}), (127, 2080, 384, 32, R.BF16, {}), (129, 4096, 256, 128, R.F16, {}),
+    (200, 2048, 16384, 128, R.BF16, {}), (200, 2048, 16384, 64, R.BF16, {"MCQ4_SPLIT_FOREIGN": "3"}),
+    (300, 2080, 640, 160, R.BF16, {"MCQ4_I4_GEMM7": "1"}), (129, 4096, 256, 64, R.F16, {"MCQ4_I4_GEMM7": "1"}),
+    (300, 2048, 5000, 128, R.BF16, {})])
+def test_bf16_prefill(dev, monkeypatch, M, K, N, gs, sdt, env):
+    import metalops_amd as mo
+    print(f"bf16 M={M} K={K} N={N} gs={gs} {env}", flush=True)
+    for k in ("MCQ4_I4_GEMM6", "MCQ4_I4_GEMM7", "MCQ4_I4_PATH", "MCQ4_XCD_LOCAL"):
+        monkeypatch.delenv(k, raising=False)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    X, args, W = _int4(dev, M, K, N, gs, R.BF16, sdt)
+    x = X.to(dev)
+    Y = mo.matmul_int4(x, *args, gs)
+    _check(Y, X, W, R.BF16)
+    if not env:
+        assert torch.equal(mo.matmul_int4(x, *args, gs).view(torch.int16), Y.view(torch.int16))
