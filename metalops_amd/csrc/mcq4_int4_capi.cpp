@@ -113,6 +113,16 @@ bool bf16_prefill(int64_t M, int64_t K, int wb, int x_dt) {
     return x_dt == MCQ4_DTYPE_BF16 && wb == 4 && M > 64 && K >= 2048;
 }
 
+// fp16 activations, up to 64 rows beyond the GEMVs' range: wx_skinny instead of the
+// GEMMs, whose 128-row tiles are mostly padding there.  us, GEMM / wx_skinny: INT4
+// M=33 4096x4096 24.5 / 13.7, M=48 4096x11008 29.4 / 22.5, M=64 4096x14336 31.9 /
+// 27.8; INT8 M=17 4096x4096 25.7 / 13.5, M=64 11008x4096 31.2 / 29.1.  At 128 rows
+// the GEMMs win: INT4 4096x4096 24.3 / 28.2.  Not where a test switch names a GEMM.
+bool f16_mid(int64_t M, int wb, int x_dt) {
+    return x_dt == MCQ4_DTYPE_F16 && M <= 64 && M > (wb == 4 ? 32 : 16) && !mcq4::opt("MCQ4_I4_GEMM6") &&
+           !mcq4::opt("MCQ4_I4_GEMM7");
+}
+
 // Upper bound over the kernels a shape can take (the general kernel needs none).
 size_t ws_bytes(int64_t M, int64_t K, int64_t N, int64_t gs, int x_dt, int wb = 4) {
     const int ks = wb == 4 ? 32 : 16;
@@ -131,7 +141,7 @@ size_t ws_bytes(int64_t M, int64_t K, int64_t N, int64_t gs, int x_dt, int wb = 
 size_t query_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t gs, int x_dt, int wb = 4) {
     const size_t need = ws_bytes(M, K, N, gs, x_dt, wb);
     if (M <= 0 || K <= 0 || N <= 0 || gs <= 0 || gs % 32) return need;
-    if (x_dt == MCQ4_DTYPE_F16 && N % 128 == 0 && K % 32 == 0) return need;
+    if (x_dt == MCQ4_DTYPE_F16 && N % 128 == 0 && K % 32 == 0 && !f16_mid(M, wb, x_dt)) return need;
     const size_t wx = mcq4::wx_workspace_bytes(wb == 4 ? mcq4::WX_I4 : mcq4::WX_I8, x_dt, M, K, N);
     if (bf16_prefill(M, K, wb, x_dt) && N % 128 == 0 && K % 32 == 0)
         return std::max({need, wx, mcq4::i4_gemm_bf16_workspace_bytes(M, K, N)});
@@ -183,6 +193,9 @@ int matmul_common(int act, const void *X, int x_dtype, int64_t ldx, const uint8_
         return fail(MCQ4_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
     hipError_t e;
+    if (path == I4Path::Gemm && f16_mid(M, wb, x_dtype) && mcq4::wx_supported(wx) &&
+        mcq4::wx_workspace_bytes(wx.wt, x_dtype, M, K, N) <= (workspace ? workspace_bytes : (size_t)0))
+        return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, st), "int4 matmul launch");
     switch (path) {
         case I4Path::Gemv:
             e = mcq4::launch_i4_gemv((const _Float16 *)X, ldx, packed, scales, zeros, sz_dtype,

@@ -1,5 +1,6 @@
-"""INT4 products of bf16 activations on the prefill kernels (the bf16 instances of
-csrc/i4_gemm6.hip and i4_gemm7.hip).
+"""INT4 / INT8 products between the decode kernels and the large tiles: bf16 prefill
+(the bf16 instances of csrc/i4_gemm6.hip and i4_gemm7.hip) and fp16 up to 64 rows
+(csrc/wx_skinny.hip).
 
 Bar per output: W is the oracle's dequantized weight rounded once to X's dtype
 (bit-exact in the kernels), so only fp32 sums and the output's rounding remain:
@@ -62,3 +63,27 @@ def test_bf16_prefill(dev, monkeypatch, M, K, N, gs, sdt, env):
     _check(Y, X, W, R.BF16)
     if not env:
         assert torch.equal(mo.matmul_int4(x, *args, gs).view(torch.int16), Y.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,K,N,gs,act", [(33, 96, 128, 32, None), (33, 4096, 384, 128, "silu"), (48, 2080, 256, 32, "gelu"),
+                                          (64, 4096, 1024, 128, None)])
+def test_fp16_rows_int4(dev, M, K, N, gs, act):
+    import metalops_amd as mo
+    print(f"i4 f16 M={M} K={K} N={N} {act}", flush=True)
+    X, args, W = _int4(dev, M, K, N, gs, R.F16, R.F16)
+    f = {None: mo.matmul_int4, "silu": mo.matmul_int4_silu, "gelu": mo.matmul_int4_gelu}[act]
+    _check(f(X.to(dev), *args, gs), X, W, R.F16, act)
+
+
+@pytest.mark.parametrize("M,K,N,gs", [(17, 64, 128, 32), (32, 4096, 384, 128), (33, 2080, 256, 32), (64, 4096, 640, 128)])
+def test_fp16_rows_int8(dev, M, K, N, gs):
+    import metalops_amd as mo
+    print(f"i8 f16 M={M} K={K} N={N}", flush=True)
+    rng = np.random.default_rng(M + N)
+    G = -(-K // gs)
+    q = rng.integers(-128, 128, (K, N)).astype(np.int8)
+    s = R.round_to(rng.uniform(0.5e-3, 2e-3, (G, N)).astype(np.float32), R.F16)
+    z = R.round_to(rng.uniform(-20, 20, (G, N)).astype(np.float32), R.F16)
+    X = torch.randn(M, K, generator=torch.Generator().manual_seed(M + K)).half()
+    Y = mo.matmul_int8(X.to(dev), torch.from_numpy(q).to(dev), torch.from_numpy(s).half().to(dev), torch.from_numpy(z).half().to(dev), gs)
+    _check(Y, X, R.dequantize_int8(q, s, z, gs, R.F16), R.F16)
