@@ -314,12 +314,14 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
     hipError_t e;
     // 33..64 rows: q4_gemm6 (flat ~31 us for any M <= 128 on 4096x14336) beats the
     // register-load decode kernel (40-77 us) wherever its alignment rules hold.
-    // 17..64 rows: the kernel between the decode and the prefill ones.  MCQ4_GEMVM_SPLIT,
+    // 17..64 rows: the kernel between the decode and the prefill ones; up to 32 rows from
+    // K = 4096 on (us, q4_gemvm / wx_mid: M=32 4096x14336 18.4 / 13.5, M=17 4096x4096 9.3 /
+    // 8.8; M=32 2048x4096 7.3 / 7.6, M=17 1024x4096 4.7 / 6.4).  MCQ4_GEMVM_SPLIT,
     // MCQ4_GEMV_PATH, MCQ4_DECODE_PATH (tests) leave these rows to the decode kernels.
-    const mcq4::WxCall mid = {mcq4::WX_Q4, mcq4::DT_F16, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32};
-    if (M > 16 && M <= 64 && mcq4::wx_mid_supported(mid) && !mcq4::opt("MCQ4_GEMVM_SPLIT") && !mcq4::opt("MCQ4_GEMV_PATH") &&
+    const mcq4::WxCall wx = {mcq4::WX_Q4, mcq4::DT_F16, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32};
+    if (M > 16 && M <= 64 && (M > 32 || K >= 4096) && mcq4::wx_mid_supported(wx) && !mcq4::opt("MCQ4_GEMVM_SPLIT") && !mcq4::opt("MCQ4_GEMV_PATH") &&
         !mcq4::opt("MCQ4_DECODE_PATH"))
-        return hip_status(mcq4::launch_wx(mid, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
+        return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
     const bool skinny = M <= 32 || (M <= 64 && !mcq4::gemm6_supported((const _Float16 *)X, ldx, W, M, K, N));
     if (skinny)
         e = mcq4::launch_skinny((const _Float16 *)X, ldx, W, (_Float16 *)Y, ldy, (int)M, (int)K,
@@ -333,7 +335,7 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
             case Prefill::Wide7: e = mcq4::launch_gemm7(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, mcq4::DT_F16, workspace, st); break;
             case Prefill::Few8: e = mcq4::launch_gemm8(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, mcq4::DT_F16, workspace, st); break;
             case Prefill::Async2: e = mcq4::launch_gemm2(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, st); break;
-            case Prefill::Any: e = mcq4::launch_wx({mcq4::WX_Q4, mcq4::DT_F16, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32}, workspace, workspace_bytes, st); break;
+            case Prefill::Any: e = mcq4::launch_wx(wx, workspace, workspace_bytes, st); break;
             default: e = mcq4::launch_gemm(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, workspace, st); break;
         }
     }

@@ -259,6 +259,18 @@ __device__ __forceinline__ void q4_values8(uint32_t q, float d, float *w) {
         w[2 * i + 1] = __builtin_fmaf((float)v[1], d, FIN ? c[i & 1] : 0.0f);
     }
 }
+// q - 8 of the eight in fp16, exact, in slot order.
+__device__ __forceinline__ uint4_t q4_exact8(uint32_t q) {
+    uint32_t p[4];
+    q4_pairs(q, p);
+    uint4_t r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const half2_t off = (i & 1) ? half2_t{(_Float16)72.0f, (_Float16)72.0f} : half2_t{(_Float16)1032.0f, (_Float16)1032.0f};
+        r[i] = bitcast<uint32_t>(bitcast<half2_t>(p[i]) - off);
+    }
+    return r;
+}
 // The same eight as a B operand of 16-bit activations (fp16: one packed multiply,
 // the single rounding of the exact product).
 template <int XT, bool FIN>

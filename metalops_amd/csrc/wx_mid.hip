@@ -18,6 +18,9 @@
 //     splits of a tile share an XCD, split 0 sums their partials from its L2 once
 //     their flags show them stored, as in q4_gemv_span.hip (above 32 rows, or with
 //     MCQ4_XCD_LOCAL=0, wx_reduce_kernel sums).
+//   * fp16 up to 32 rows: the decode kernels' arithmetic, sum x (q - 8) of a block
+//     exact in the MFMA and scaled by d in fp32.  Otherwise the weight (q - 8) d is
+//     rounded to the activations' dtype first, as the prefill kernels do.
 //   * MFMA lane rows g = 0..3 take K quarters 0, 2, 1, 3 of a block (both operands):
 //     fewer LDS bank conflicts on the nibble reads.
 //
@@ -122,6 +125,20 @@ __global__ void __launch_bounds__(WM_NW * 64) wx_mid_kernel(WxArgs a) {
         uint4_t x[RT];
 #pragma unroll
         for (int i = 0; i < RT; ++i) x[i] = wx_order<WX_Q4>(bitcast<uint4_t>(*(const lds_half8 *)(Xs + xoff + 1024 * i)));
+        if constexpr (XT == DT_F16 && RT == 2) {
+#pragma unroll
+            for (int j = 0; j < WM_CT; ++j) {
+                const float df = (float)bitcast<_Float16>(d[j]);
+                const uint4_t B = q4_exact8(q[j]);
+#pragma unroll
+                for (int i = 0; i < RT; ++i) {
+                    const float4_t t = wx_mfma16<XT>(x[i], B, float4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[i][j][r] = __builtin_fmaf(df, t[r], acc[i][j][r]);
+                }
+            }
+            return;
+        }
         wx_if_finite<WX_Q4, XT, WM_CT>(d, [&](auto fin) {
 #pragma unroll
             for (int j = 0; j < WM_CT; ++j) {

@@ -61,6 +61,20 @@ def test_q4(dev, xdt, M, K, N):
     _check(Y, X, R.round_to(Q.dequantize(b, np.float32), xdt), xdt)
 
 
+# fp16, 17..32 rows, whole 16-byte weight rows: the weight stays unrounded (exact block
+# sums, d applied in fp32), so the bar is that of fp32 sums against (q - 8) d itself.
+@pytest.mark.parametrize("M,K,N,exact", [(17, 64, 8, True), (24, 4096, 136, True), (32, 14336, 64, True), (31, 4128, 4096, True)])
+def test_q4_fp16_rows(dev, M, K, N, exact):
+    import metalops_amd as mo
+    print(f"q4 fp16 M={M} K={K} N={N}", flush=True)
+    w = np.random.default_rng(M * 5 + N).standard_normal((K, N), np.float32) * 0.02
+    b = Q.quantize_llama_rule(w)
+    X = _x(M, K, R.F16, M + K)
+    Y = mo.matmul_ggml_q4_0(X.to(dev), torch.from_numpy(b).to(dev))
+    W = Q.dequantize(b, np.float32)
+    _check(Y, X, W if exact else R.round_to(W, R.F16), R.F16)
+
+
 @pytest.mark.parametrize("M,K,N,pad,off", [(5, 256, 33, 3, 0), (40, 256, 66, 8, 1), (100, 544, 70, 5, 3), (70, 512, 64, 0, 2)])
 @pytest.mark.parametrize("xdt", [R.BF16, R.F32])
 def test_q4_row_strides(dev, xdt, M, K, N, pad, off):
