@@ -322,6 +322,17 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
     if (M > 16 && M <= 64 && (M > 32 || K >= 4096) && mcq4::wx_mid_supported(wx) && !mcq4::opt("MCQ4_GEMVM_SPLIT") && !mcq4::opt("MCQ4_GEMV_PATH") &&
         !mcq4::opt("MCQ4_DECODE_PATH"))
         return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
+    // Up to 64 rows of weights the strip kernels do not take (odd column counts or
+    // addresses): LDS sums over 16 or 8 waves instead of q4_skinny's 4, from K = 4096 on
+    // (same arithmetic: weights rounded to fp16).  us, q4_skinny / wx_gemv, wx_skinny: M=1
+    // 4096x4101 9.5 / 7.8, 14336x4099 29.3 / 16.1, M=16 4096x12289 19.8 / 15.7, M=17
+    // 4096x4101 15.8 / 12.5, M=64 4096x12289 45.0 / 28.6; K = 2048: M=1 x1025 4.5 / 4.9,
+    // M=17 x4097 9.0 / 9.5.
+    const bool strips = N % 8 == 0 && aligned(W, 16);
+    if (M <= 64 && K >= 4096 && !strips && !mcq4::opt("MCQ4_GEMVM_SPLIT") && !mcq4::opt("MCQ4_GEMV_PATH") &&
+        !mcq4::opt("MCQ4_DECODE_PATH") &&
+        mcq4::wx_workspace_bytes(mcq4::WX_Q4, mcq4::DT_F16, M, K, N) <= (workspace ? workspace_bytes : (size_t)0))
+        return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
     const bool skinny = M <= 32 || (M <= 64 && !mcq4::gemm6_supported((const _Float16 *)X, ldx, W, M, K, N));
     if (skinny)
         e = mcq4::launch_skinny((const _Float16 *)X, ldx, W, (_Float16 *)Y, ldy, (int)M, (int)K,
