@@ -10,22 +10,18 @@
 //   * Split K over workgroups (grid.z) where the columns alone leave CUs idle:
 //     fp32 partial rows summed in split order by wx_reduce_kernel.
 //
-// Measured: q4_0 x bf16 M = 4 4096x11008 13.0 us, was 199 (one thread per column,
-// 2-byte weight loads); INT4 x fp32 M = 32 4096x4096 26 us, was 811.
+// Bound by the latency of its loads (no LDS staging: a lane's 8 or 16 weight bytes and
+// its row's activations per request) rather than by the bytes.  Sixteen waves instead of
+// eight: slower (14.9 against 13.4 us).  Measured, against one thread per column with
+// 2-byte weight loads: INT4 x bf16 M = 64 4096x14336 27.4 us (was 2472), INT4 x fp32 M =
+// 32 4096x4096 19.8 (was 811).
 #include <algorithm>
 
 #include "wx_common.h"
 
 namespace mcq4 {
 
-#ifndef WS_NW_SET
-constexpr int WS_NW = 8;
-#else
-constexpr int WS_NW = WS_NW_SET;
-#endif
-#ifndef WS_TN_SET
-#define WS_TN_SET 2
-#endif
+constexpr int WS_NW = 8, WS_TN = 2;
 
 template <int WT, int XT, int TM, int TN, bool SZ32, bool ANY>
 __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
@@ -175,7 +171,7 @@ static hipError_t launch_wx_skinny_k(const WxArgs &a, hipStream_t s) {
 }
 template <int WT, int XT, bool SZ32>
 static hipError_t launch_wx_skinny_t(const WxArgs &a, bool any, hipStream_t s) {
-    constexpr int TN = WS_TN_SET;
+    constexpr int TN = WS_TN;
     if (a.M <= 32)
         return any ? launch_wx_skinny_k<WT, XT, 1, TN, SZ32, true>(a, s) : launch_wx_skinny_k<WT, XT, 1, TN, SZ32, false>(a, s);
     return any ? launch_wx_skinny_k<WT, XT, 2, TN, SZ32, true>(a, s) : launch_wx_skinny_k<WT, XT, 2, TN, SZ32, false>(a, s);
@@ -195,7 +191,7 @@ static hipError_t launch_wx_skinny_w(const WxArgs &a, int x_dt, bool any, hipStr
 
 // K splits: one workgroup per CU, every wave at least 2 K steps.
 static int wx_skinny_splits(int64_t K, int64_t N) {
-    const int64_t t = (N + 32 * WS_TN_SET - 1) / (32 * WS_TN_SET), nks = (K + 31) / 32;
+    const int64_t t = (N + 32 * WS_TN - 1) / (32 * WS_TN), nks = (K + 31) / 32;
     int S = 1;
     while (t * S * 2 <= 256 && nks / (S * 2 * WS_NW) >= 2 && S < 16) S *= 2;
     return S;
