@@ -17,23 +17,28 @@
 //     16-byte aligned, or a K that is no multiple of 32, are read element by
 //     element, zero past K.
 //   * 16-bit activations: v_mfma_f32_32x32x16_{f16,bf16}, a B operand feeding
-//     four MFMAs.  fp32: v_mfma_f32_32x32x2_f32, weights kept in fp32.
+//     four MFMAs.  fp32: v_mfma_f32_32x32x2_f32, weights kept in fp32, 64 x 256 tiles: the
+//     other half of the accumulators holds the running sums, to which each step's 32
+//     products are added as a sum of their own (error against 64 bits, K = 4096: 1.3e-7 of
+//     the result; 5e-7 in one chain of K / 2, 3.9e-7 in eight of K / 8).
 //   * Split K (grid.z) for outputs with few tiles: fp32 partial rows summed in
 //     split order by wx_reduce_kernel.
 //
 // Measured: INT4 x bf16 M = 256 4096x11008 60.9 us (one thread per column: 8165), INT4 x
-// fp32 267.8, q4_0 x fp16 M = 300 11008x4101 83.9.  INT4 in 16 bits is bound by waits
+// fp32 243.2, q4_0 x fp16 M = 300 11008x4101 83.9.  INT4 in 16 bits is bound by waits
 // (counters: MFMA busy 15 %, 43 % of the wave cycles waiting, LDS conflicts 28 % of the
-// LDS cycles); fp32 by the fp32 MFMA, whose library rate is 153 TFLOP/s here (86 at M =
-// 256, 115 at 512x4096x4096).  Operands prepared one step ahead of their MFMAs: 61.5 us.
+// LDS cycles); fp32 by the fp32 MFMA, whose library rate is 153 TFLOP/s here (95 at M =
+// 256, 108 at 512x4096x4096).  Operands prepared one step ahead of their MFMAs: 61.5 us.
 #include <algorithm>
+#include <type_traits>
 
 #include "wx_common.h"
 
 namespace mcq4 {
 
-constexpr int WG_BM = 128, WG_BN = 256, WG_TM = 4, WG_TN = 2;
-constexpr int WG_SLOT = WG_BM * 256;
+constexpr int WG_BN = 256, WG_TN = 2;
+constexpr int wg_tm(int xt) { return xt == DT_F32 ? 2 : 4; }   // row tiles of 32
+constexpr int WG_SLOT = 128 * 256;               // 128 rows (fp32: 64)
 constexpr size_t WG_LDS = 4 * 2 * 2 * WG_TN * 16 * 64 * 4;   // phase sum: 4 column groups x 2 halves, 128 KB (the loop: 64 + scratch)
 static_assert(WG_LDS >= 2 * WG_SLOT + 8 * wx_scratch(WX_I8) && WG_LDS <= 160 * 1024, "LDS budget");
 
@@ -41,6 +46,7 @@ template <int WT, int XT, bool SZ32, bool ANY, bool ACT>
 __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
     constexpr int ES = XT == DT_F32 ? 4 : 2;
     constexpr int SPW = XT == DT_F32 ? 1 : 2;    // K steps of 32 per wave and stage
+    constexpr int TM = wg_tm(XT), BM = 32 * TM;
     constexpr int R = 4;                         // ring slots: R - 1 steps in flight
     extern __shared__ __attribute__((aligned(16))) uint8_t sA[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -51,7 +57,7 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
     const int bid = blockIdx.x, gx = gridDim.x;
     int tile_id = bid;
     if (gx % 8 == 0) tile_id = (bid % 8) * (gx / 8) + bid / 8;   // consecutive tiles on one XCD
-    const int m0 = (tile_id % a.tiles_m) * WG_BM, n0 = (tile_id / a.tiles_m) * WG_BN + 64 * wc;
+    const int m0 = (tile_id % a.tiles_m) * BM, n0 = (tile_id / a.tiles_m) * WG_BN + 64 * wc;
     const int nks = (a.K + 31) / 32;
     const int z = blockIdx.z;
     const int k_lo = (int)((int64_t)nks * z / a.S), nk = (int)((int64_t)nks * (z + 1) / a.S) - k_lo;
@@ -59,17 +65,17 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
 
     const WxLane<WT, WG_TN> L = wx_lane<WT, WG_TN>(a, n0, lane);
 
-    // Activation copies: thread t moves chunks (row t / 16 + 32 u, chunk t % 16), u < 4.
-    const uint8_t *xrow[4];
+    // Activation copies: thread t moves chunks (row t / 16 + 32 u, chunk t % 16), u < TM.
+    const uint8_t *xrow[TM];
     const int xc = tid & 15;
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < TM; ++u)
         xrow[u] = (const uint8_t *)a.X + (int64_t)min(m0 + (tid >> 4) + 32 * u, a.M - 1) * a.ldx * ES;
-    uint4_t xs[4];
+    uint4_t xs[TM];
     auto load_a = [&](int st) {
         const int k = (k_lo + min(st, nst - 1) * (2 * SPW)) * 32 + xc * (16 / ES);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < TM; ++u) {
             if constexpr (ANY) xs[u] = wx_load_x_any<XT>(xrow[u], k, a.K);
             // Past the split's end (a last stage that is not whole): any valid chunk, no MFMA uses it.
             else xs[u] = *(const uint4_t *)(xrow[u] + (int64_t)min(k, a.K - 16 / ES) * ES);
@@ -77,7 +83,7 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
     };
     auto store_a = [&](int slot) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < TM; ++u) {
             const int r = (tid >> 4) + 32 * u;
             *(uint4_t *)(sA + slot * WG_SLOT + r * 256 + ((xc ^ (r & 7)) << 4)) = XT == DT_F32 ? xs[u] : wx_order<WT>(xs[u]);
         }
@@ -94,9 +100,9 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
         wx_load<WT, WG_TN, SZ32, ANY && WT != WX_Q4>(r, a, L, k_lo + min(kstep(u), nk - 1), lane);
     };
 
-    float16_t acc[WG_TM][WG_TN];
+    std::conditional_t<XT == DT_F32, float[TM][WG_TN][16], float16_t[TM][WG_TN]> acc;
 #pragma unroll
-    for (int i = 0; i < WG_TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < WG_TN; ++j)
 #pragma unroll
@@ -108,7 +114,9 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
         const uint16_t *d = nullptr;
         if constexpr (WT == WX_Q4) d = r.d;
         if constexpr (XT == DT_F32) {
+            // A step's 32 products are summed from zero and then added: chains of 32 and K / 64.
             float w[WG_TN][16];
+            float16_t part[TM][WG_TN];
             wx_if_finite<WT, XT, WG_TN>(d, [&](auto fin) {
 #pragma unroll
                 for (int j = 0; j < WG_TN; ++j)
@@ -116,21 +124,32 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
             });
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                float4_t x[WG_TM][2];
+                float4_t x[TM][2];
 #pragma unroll
-                for (int i = 0; i < WG_TM; ++i)
+                for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int q = 0; q < 2; ++q) x[i][q] = bitcast<float4_t>(read_a(slot, i, 8 * ph + 4 * lhi + 2 * h + q));
 #pragma unroll
                 for (int s = 0; s < 8; ++s) {
                     const int e = wx_slot<WT>(s);
 #pragma unroll
-                    for (int i = 0; i < WG_TM; ++i)
+                    for (int i = 0; i < TM; ++i)
 #pragma unroll
                         for (int j = 0; j < WG_TN; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i][e / 4][e % 4], w[j][8 * h + s], acc[i][j], 0, 0, 0);
+                            part[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i][e / 4][e % 4], w[j][8 * h + s],
+                                                                              h + s ? part[i][j] : float16_t{}, 0, 0, 0);
                 }
             }
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < WG_TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        float v = acc[i][j][r] + part[i][j][r];
+                        asm volatile("" : "+v"(v));   // else the add sinks to the next step, part with it
+                        acc[i][j][r] = v;
+                    }
         } else {
             uint4_t B[WG_TN][2];
             wx_if_finite<WT, XT, WG_TN>(d, [&](auto fin) {
@@ -141,7 +160,7 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                for (int i = 0; i < WG_TM; ++i) {
+                for (int i = 0; i < TM; ++i) {
                     const uint4_t x = read_a(slot, i, 8 * ph + 4 * t + 2 * lhi + ks);
 #pragma unroll
                     for (int j = 0; j < WG_TN; ++j) acc[i][j] = wx_mfma<XT>(x, B[j][ks], acc[i][j]);
@@ -180,30 +199,31 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
     for (; (s0 + GRP) * 2 * SPW <= nk; s0 += GRP) group(std::false_type{}, s0);
     if (s0 < nst) group(std::true_type{}, s0);
 
-    // Phase sum: each wave gives the other phase's half of its rows (32 (2 (1 - ph)) ..)
+    // Phase sum: each wave gives the other phase's half of its rows
     // away and adds the other's share of its own.
-    static_assert(GRP % 2 == 0 && WG_TM == 4, "slot parity; halves of two row tiles");
-    float *const sum = (float *)sA + (wc * 2 + ph) * (2 * WG_TN * 16 * 64) + lane;
-    float *const mine = (float *)sA + (wc * 2 + (1 - ph)) * (2 * WG_TN * 16 * 64) + lane;
+    constexpr int H = TM / 2;
+    static_assert(GRP % 2 == 0 && TM % 2 == 0, "slot parity; halves of the row tiles");
+    float *const sum = (float *)sA + (wc * 2 + ph) * (H * WG_TN * 16 * 64) + lane;
+    float *const mine = (float *)sA + (wc * 2 + (1 - ph)) * (H * WG_TN * 16 * 64) + lane;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < H; ++i)
 #pragma unroll
         for (int j = 0; j < WG_TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sum[((i * WG_TN + j) * 16 + r) * 64] = ph ? acc[i][j][r] : acc[2 + i][j][r];
+            for (int r = 0; r < 16; ++r) sum[((i * WG_TN + j) * 16 + r) * 64] = ph ? acc[i][j][r] : acc[H + i][j][r];
     lds_barrier();
     // Lane l holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < H; ++i)
 #pragma unroll
         for (int j = 0; j < WG_TN; ++j) {
             const int n = L.n[j];
             const bool ok = n0 + (WT == WX_Q4 ? 32 * j + lrow : 16 * (lrow >> 3)) < a.N;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int m = m0 + 64 * ph + 32 * i + 8 * (r >> 2) + 4 * lhi + (r & 3);
+                const int m = m0 + 32 * H * ph + 32 * i + 8 * (r >> 2) + 4 * lhi + (r & 3);
                 const float o = mine[((i * WG_TN + j) * 16 + r) * 64];
-                const float v = ph ? o + acc[2 + i][j][r] : acc[i][j][r] + o;   // phase 0 + phase 1
+                const float v = ph ? o + acc[H + i][j][r] : acc[i][j][r] + o;   // phase 0 + phase 1
                 if (m >= a.M || !ok) continue;
                 if (a.S > 1) a.part[((int64_t)z * a.M + m) * a.ldp + n] = v;
                 else store_dt(a.Y, (int64_t)m * a.ldy + n, ACT ? wx_activate(v, a.act) : v, XT);
@@ -254,14 +274,30 @@ static hipError_t launch_wx_gemm_s(const WxArgs &a, int x_dt, bool any, dim3 gri
     return launch_wx_gemm_t<WT, DT_F32, SZ32>(a, any, grid, s);
 }
 
-// K splits: as many as keep one workgroup per CU, at least 8 K steps of 32 each.
-int wx_gemm_splits(int64_t M, int64_t K, int64_t N) {
-    const int64_t t = ((M + WG_BM - 1) / WG_BM) * ((N + WG_BN - 1) / WG_BN), nks = (K + 31) / 32;
-    return (int)std::max<int64_t>(1, std::min<int64_t>({256 / t, nks / 8, 16}));
+// K splits, at least 8 K steps of 32 each.  16 bits: as many as keep one workgroup per
+// CU.  fp32 is bound by its MFMAs, so a last round of workgroups that leaves CUs idle
+// costs in full: the split with the least rounds(t S) / S, plus the partials' traffic (8
+// bytes an output and split at about 5 TB/s against 2 K operations at about 100 TFLOP/s:
+// 80 / K of a full round).  us, at most one per CU / this: 256x4096x11008 (172 tiles)
+// 279.6 / 237.0, 512x4096x4100 (136 tiles) 289.4 / 202.6.
+int wx_gemm_splits(int x_dt, int64_t M, int64_t K, int64_t N) {
+    const int64_t bm = 32 * wg_tm(x_dt), t = ((M + bm - 1) / bm) * ((N + WG_BN - 1) / WG_BN), nks = (K + 31) / 32;
+    if (x_dt != DT_F32 || t >= 1024) return (int)std::max<int64_t>(1, std::min<int64_t>({256 / t, nks / 8, 16}));
+    int best = 1;
+    double least = 0;
+    for (int S = 1; S <= 16 && (S == 1 || nks / S >= 8); ++S) {
+        const double cost = (double)((t * S + 255) / 256) / S + S * (t / 256.0) * (80.0 / (double)K);
+        if (S == 1 || cost < least) {
+            best = S;
+            least = cost;
+        }
+    }
+    return best;
 }
 
 hipError_t launch_wx_gemm(WxArgs a, int wt, int x_dt, bool any, hipStream_t s) {
-    a.tiles_m = (a.M + WG_BM - 1) / WG_BM;
+    const int bm = 32 * wg_tm(x_dt);
+    a.tiles_m = (a.M + bm - 1) / bm;
     a.tiles_n = (a.N + WG_BN - 1) / WG_BN;
     const dim3 grid((unsigned)(a.tiles_m * a.tiles_n), 1, a.S);
     const bool sz32 = a.sz_dt == DT_F32;

@@ -11,10 +11,11 @@
 //     per weight for bf16.  So the columns are spread over the CUs
 //     as evenly as 16-column groups allow (TN below), with no K split over
 //     workgroups and one launch.
-//   * fp32: v_mfma_f32_16x16x4_f32, half the matrix time of the 32-row form.
+//   * fp32: v_mfma_f32_16x16x4_f32, half the matrix time of the 32-row form;
+//     64 products at a time are summed from zero, then added (error as in wx_gemm).
 //
 // Measured: fp16 M = 1 / 16 4096x12289 12.4 / 15.7 us (q4_skinny 16.7 / 19.8), fp32 M = 8
-// 4096x11008 21.7.  Fewer VALU per weight (3.3 to 2.1) changed nothing: the unaligned
+// 4096x11008 22.7.  Fewer VALU per weight (3.3 to 2.1) changed nothing: the unaligned
 // 16-byte loads at 18-byte stride take the time.
 #include "wx_common.h"
 
@@ -87,11 +88,19 @@ __global__ void __launch_bounds__(NW * 64) wx_gemv_kernel(WxArgs a) {
                     r.q[0][0] = p.q[j][2 * h]; r.q[0][1] = p.q[j][2 * h + 1];
                     if constexpr (XT == DT_F32) {
                         float w[16];
+                        float4_t part;       // 64 products, summed from zero
                         wx_values<WX_Q4, XT, 1, false, false, FIN>(r, 0, 0, 16, w);
 #pragma unroll
                         for (int s = 0; s < 16; ++s) {
                             const int e = wx_slot<WX_Q4>(s);
-                            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(p.x[4 * h + e / 4][e % 4]), w[s], acc[j], 0, 0, 0);
+                            part = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(p.x[4 * h + e / 4][e % 4]), w[s],
+                                                                        s ? part : float4_t{}, 0, 0, 0);
+                        }
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            float v = acc[j][r] + part[r];
+                            asm volatile("" : "+v"(v));
+                            acc[j][r] = v;
                         }
                     } else {
                         uint4_t B[2];

@@ -7,6 +7,7 @@
 //     Each weight is read and dequantized once.
 //   * 32 TM activation rows (rows past M repeat the last one, their outputs are
 //     not stored): the weights' bytes bound the kernel, not its MFMAs.
+//   * fp32: a step's 32 products are summed from zero, then added (error as in wx_gemm).
 //   * Split K over workgroups (grid.z) where the columns alone leave CUs idle:
 //     fp32 partial rows summed in split order by wx_reduce_kernel.
 //
@@ -16,6 +17,7 @@
 // 2-byte weight loads: INT4 x bf16 M = 64 4096x14336 27.4 us (was 2472), INT4 x fp32 M =
 // 32 4096x4096 19.8 (was 811).
 #include <algorithm>
+#include <type_traits>
 
 #include "wx_common.h"
 
@@ -61,7 +63,7 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
             }
     };
 
-    float16_t acc[TM][TN];
+    std::conditional_t<XT == DT_F32, float[TM][TN][16], float16_t[TM][TN]> acc;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -86,14 +88,24 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
             for (int j = 0; j < TN; ++j) {
                 if constexpr (XT == DT_F32) {
                     float w[16];
+                    float16_t part[TM];      // the step's 32 products, summed from zero
                     wx_values<WT, XT, TN, SZ32, ANY, FIN>(raw, j, a.sz_dt, valid, w);
 #pragma unroll
                     for (int s = 0; s < 16; ++s) {
                         const int e = wx_slot<WT>(s);
 #pragma unroll
                         for (int i = 0; i < TM; ++i)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(p.x[i][e / 4][e % 4]), w[s], acc[i][j], 0, 0, 0);
+                            part[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(p.x[i][e / 4][e % 4]), w[s],
+                                                                           s ? part[i] : float16_t{}, 0, 0, 0);
                     }
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            float v = acc[i][j][r] + part[i][r];
+                            asm volatile("" : "+v"(v));   // else the add sinks to the next step, part with it
+                            acc[i][j][r] = v;
+                        }
                 } else {
                     uint4_t B[2];
                     wx_operands<WT, XT, TN, SZ32, ANY, FIN>(raw, j, a.sz_dt, valid, B);
@@ -156,7 +168,7 @@ int wx_mid_splits(int64_t K, int64_t N);
 size_t wx_mid_flag_bytes(int64_t N, int S);
 hipError_t launch_wx_mid(WxArgs a, int x_dt, bool *reduce, hipStream_t s);
 hipError_t launch_wx_gemm(WxArgs a, int wt, int x_dt, bool any, hipStream_t s);
-int wx_gemm_splits(int64_t M, int64_t K, int64_t N);
+int wx_gemm_splits(int x_dt, int64_t M, int64_t K, int64_t N);
 
 template <int WT, int XT, int TM, int TN, bool SZ32, bool ANY>
 static hipError_t launch_wx_skinny_k(const WxArgs &a, hipStream_t s) {
@@ -203,7 +215,7 @@ static int64_t wx_ldp(int64_t N) { return (N + 3) / 4 * 4; }
 static int wx_splits(int wt, int x_dt, int64_t M, int64_t K, int64_t N) {
     if (wt == WX_Q4 && M <= 16) return 1;         // wx_gemv
     // One plan for a shape, whatever the alignment: wx_mid and wx_skinny share it.
-    int S = wx_mid_shape(wt, x_dt, M, N) ? wx_mid_splits(K, N) : M <= 64 ? wx_skinny_splits(K, N) : wx_gemm_splits(M, K, N);
+    int S = wx_mid_shape(wt, x_dt, M, N) ? wx_mid_splits(K, N) : M <= 64 ? wx_skinny_splits(K, N) : wx_gemm_splits(x_dt, M, K, N);
     if (wt == WX_Q4 && x_dt == DT_F16)
         while (S > 1 && (int64_t)S * M * wx_ldp(N) * 4 > ((int64_t)16 << 20)) S /= 2;
     return S;

@@ -64,7 +64,7 @@ def test_q4(dev, xdt, M, K, N):
 # fp16, 17..32 rows, whole 16-byte weight rows: the weight stays unrounded (exact block
 # sums, d applied in fp32), so the bar is that of fp32 sums against (q - 8) d itself.
 # Then weights the strip kernels do not take, at the K from which wx runs them.
-@pytest.mark.parametrize("M,K,N,exact", [(17, 64, 8, True), (24, 4096, 136, True), (32, 14336, 64, True), (31, 4128, 4096, True),
+@pytest.mark.parametrize("M,K,N,exact", [(17, 4096, 8, True), (24, 4096, 136, True), (32, 14336, 64, True), (31, 4128, 4096, True),
                                          (1, 4096, 33, False), (16, 4128, 257, False), (17, 4096, 65, False), (64, 4096, 1025, False)])
 def test_q4_fp16_rows(dev, M, K, N, exact):
     import metalops_amd as mo
