@@ -52,6 +52,7 @@ def _int4(dev, M, K, N, gs, xdt, sdt):
     (300, 2048, 5000, 128, R.BF16, {})])
 def test_bf16_prefill(dev, monkeypatch, M, K, N, gs, sdt, env):
     import metalops_amd as mo
+    from metalops_amd import _lib
     print(f"bf16 M={M} K={K} N={N} gs={gs} {env}", flush=True)
     for k in ("MCQ4_I4_GEMM6", "MCQ4_I4_GEMM7", "MCQ4_I4_PATH", "MCQ4_XCD_LOCAL"):
         monkeypatch.delenv(k, raising=False)
@@ -60,6 +61,8 @@ def test_bf16_prefill(dev, monkeypatch, M, K, N, gs, sdt, env):
     X, args, W = _int4(dev, M, K, N, gs, R.BF16, sdt)
     x = X.to(dev)
     Y = mo.matmul_int4(x, *args, gs)
+    redone = _lib.split_fallback_count(reset=True)
+    assert (redone > 0) == ("MCQ4_SPLIT_FOREIGN" in env)
     _check(Y, X, W, R.BF16)
     if not env:
         assert torch.equal(mo.matmul_int4(x, *args, gs).view(torch.int16), Y.view(torch.int16))
