@@ -251,7 +251,7 @@ def matmul_int4(
 
     fp32 accumulation; the result has ``X``'s dtype.  fp16 activations run the
     MFMA kernels (decode GEMV for M <= 16 rows, and up to 32 rows when N is a
-    multiple of 128; prefill GEMM above); fp32 and
+    multiple of 128; a register kernel up to 64; prefill GEMM above); fp32 and
     bf16 activations, and fp16 ones at other shapes, use the weight rounded to
     ``X``'s dtype, as the reference builds ``W`` in ``X.dtype``
     (quantization.py:220-239), on the matrix cores of that dtype; group sizes
