@@ -51,6 +51,28 @@ __device__ __forceinline__ To bitcast(const From &f) {
     return __builtin_bit_cast(To, f);
 }
 
+// A wave's copy of its `cols` columns' K row piece (64 columns: 1152 bytes, 0..1023 as
+// 16 bytes per lane, the rest as 4 bytes for lanes 0..31, which lanes 32..63
+// repeat), for N % 8 == 0.  Columns past N: the lane re-reads the piece's last bytes
+// inside the row, whose outputs are not stored; a wave wholly past N copies the row's last
+// 8 columns.  So no lane reads outside [0, 18 N) of the row.
+struct Q4Piece {
+    uint32_t start, bytes;   // byte offset in the row, bytes of the piece inside it (>= 144)
+    __host__ __device__ __forceinline__ Q4Piece(int n, int cols, int N) {
+        const int c = n < N - 8 ? n : N - 8;
+        start = (uint32_t)c * BLOCK_BYTES;
+        bytes = (uint32_t)(cols < N - c ? cols : N - c) * BLOCK_BYTES;
+    }
+    // The lane's offsets from `start` in the 16-byte and the 4-byte copy.
+    __host__ __device__ __forceinline__ uint32_t off16(int lane) const {
+        return 16u * lane < bytes - 16 ? 16u * lane : bytes - 16;
+    }
+    __host__ __device__ __forceinline__ uint32_t off4(int lane) const {
+        const uint32_t o = 1024u + 4u * (lane < 31 ? lane : 31);
+        return o < bytes - 4 ? o : bytes - 4;
+    }
+};
+
 __device__ __forceinline__ int64_t imin64(int64_t x, int64_t y) { return x < y ? x : y; }
 
 // s_waitcnt with only vmcnt constrained (gfx9 encoding: vmcnt[3:0] | [15:14]).

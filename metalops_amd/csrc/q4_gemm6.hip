@@ -97,14 +97,11 @@ q4_gemm6_kernel(Gemm6Args a) {
     }
 
     const uint32_t row_bytes = (uint32_t)a.N * BLOCK_BYTES;
-    const bool wcols = n0 + wn * WN < a.N;
     const __amdgpu_buffer_rsrc_t w_rs =
         __builtin_amdgcn_make_buffer_rsrc((void *)a.W, (short)0, (int)0x7fffffff, 0x00020000);
-    const uint32_t w_so0 = (uint32_t)k_lo * row_bytes + (wcols ? (uint32_t)(n0 + wn * WN) * BLOCK_BYTES : 0u);
-    // Columns past N (N % 8 == 0): the lane re-reads the row's last bytes, whose
-    // outputs are not stored, so nothing past the row is read.
-    const uint32_t w_valid = wcols ? (uint32_t)min(WN, a.N - (n0 + wn * WN)) * BLOCK_BYTES : G6_RAW_W;
-    const uint32_t w_vo16 = min(16u * lane, w_valid - 16), w_vo4 = min(1024u + 4u * min(lane, 31), w_valid - 4);
+    const Q4Piece piece(n0 + wn * WN, WN, a.N);
+    const uint32_t w_so0 = (uint32_t)k_lo * row_bytes + piece.start;
+    const uint32_t w_vo16 = piece.off16(lane), w_vo4 = piece.off4(lane);
 
     // Copy ci (0 .. GROUP-1) of stage s_dst: A copies, then per step t the raw
     // bytes 0..1023 (16 per lane) and 1024..1151 (4 per lane for lanes 0..31;

@@ -61,6 +61,20 @@ def test_q4(dev, xdt, M, K, N):
     _check(Y, X, R.round_to(Q.dequantize(b, np.float32), xdt), xdt)
 
 
+# Fewer columns than one wave's 64 (N % 8 == 0): the prefill tiles' other waves have none; a
+# K split, one K step, two row tiles.
+@pytest.mark.parametrize("M,K,N", [(65, 4096, 8), (65, 32, 24), (130, 1056, 56), (300, 4096, 72)])
+@pytest.mark.parametrize("xdt", [R.BF16, R.F16])
+def test_q4_narrow_prefill(dev, xdt, M, K, N):
+    import metalops_amd as mo
+    print(f"q4 narrow {xdt} M={M} K={K} N={N}", flush=True)
+    w = np.random.default_rng(M + N).standard_normal((K, N), np.float32) * 0.02
+    b = Q.quantize_llama_rule(w)
+    X = _x(M, K, xdt, M + K)
+    Y = mo.matmul_ggml_q4_0(X.to(dev), torch.from_numpy(b).to(dev))
+    _check(Y, X, R.round_to(Q.dequantize(b, np.float32), xdt), xdt)
+
+
 # fp16, 17..32 rows, whole 16-byte weight rows: the weight stays unrounded (exact block
 # sums, d applied in fp32), so the bar is that of fp32 sums against (q - 8) d itself.
 # Then weights the strip kernels do not take, at the K from which wx runs them.
