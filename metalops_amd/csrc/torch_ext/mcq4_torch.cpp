@@ -4,8 +4,8 @@
 // fp16 X [M, K] and uint8 W_blocks [K/32, N, 18] on the GPU, contiguous copies
 // made by the callee, Y [M, N] fp16 allocated by the callee, errors as
 // RuntimeError (TORCH_CHECK), work enqueued on the current stream without a
-// synchronisation.  The split-K workspace is kept per (device, stream),
-// zero-filled once (every call leaves its counters zero).
+// synchronisation.  The split-K workspace is kept per (device, stream), its counters
+// zeroed once (every call leaves them zero); a HIP graph's calls have their own.
 //
 // It also holds the native call path of the Python functions (q4_matmul, q4_grouped,
 // int4_matmul, int8_matmul, int4_rmsnorm below): the checks, the output, the
@@ -27,17 +27,40 @@
 
 namespace {
 
+// The workspaces of one (device, stream).  `eager` serves the calls that run as they are
+// made: on one stream they never overlap, and a larger request replaces it through the
+// stream-ordered allocator.  `captured` serves the calls recorded into the stream capture
+// `capture`: it comes from the graph's memory pool, so its addresses stay the graph's
+// for as long as that can be replayed, whatever later calls on the stream ask for, and no
+// eager call or other graph works in it while a replay runs on another stream.  Its
+// counters are zeroed by a recorded fill kernel (one per graph and size).  It is kept
+// until the next capture on the stream, so a stream holds at most two buffers.
+struct Buffers {
+    torch::Tensor eager, captured;
+    unsigned long long capture = 0;
+};
 std::mutex g_ws_mu;
-std::map<std::pair<int, hipStream_t>, torch::Tensor> g_ws;
+std::map<std::pair<int, hipStream_t>, Buffers> g_ws;
 
-// One buffer per (device, stream): calls on one stream never overlap.  A larger
-// request allocates anew through the stream-ordered allocator.
 torch::Tensor workspace(int device, hipStream_t stream, size_t need) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {   // the null stream beside another capture
+        (void)hipGetLastError();
+        status = hipStreamCaptureStatusNone;
+    }
+    const bool capturing = status == hipStreamCaptureStatusActive;
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    auto &buf = g_ws[{device, stream}];
-    if (!buf.defined() || (size_t)buf.numel() < need)
-        buf = torch::zeros({(int64_t)std::max<size_t>(need, 1 << 20)},
-                           torch::TensorOptions().dtype(torch::kUInt8).device(torch::kCUDA, device));
+    Buffers &b = g_ws[{device, stream}];
+    torch::Tensor &buf = capturing ? b.captured : b.eager;
+    if (!buf.defined() || (size_t)buf.numel() < need || (capturing && b.capture != id)) {
+        const size_t bytes = std::max<size_t>(need, 1 << 20);
+        torch::Tensor t = torch::empty({(int64_t)bytes}, torch::TensorOptions().dtype(torch::kUInt8).device(torch::kCUDA, device));
+        const int st = mcq4_reset_workspace(t.data_ptr(), bytes, stream);
+        TORCH_CHECK(st == MCQ4_OK, "workspace: ", mcq4_last_error());
+        buf = std::move(t);
+        if (capturing) b.capture = id;
+    }
     return buf;
 }
 

@@ -151,16 +151,18 @@ def dequantize_ggml_q4_0(blocks: torch.Tensor, dtype: Optional[torch.dtype] = No
 
 
 class _Workspace:
-    """Per-device, zero-initialised split-K workspace reused across calls.
+    """Per-device split-K workspace, its counters zero, reused across calls.
 
-    The kernels leave the arrival counters at zero after every call, so the
-    buffer is zero-filled once when (re)allocated; a call that fails is
+    The kernels leave the arrival counters at zero after every call, so they are
+    zeroed once when the buffer is (re)allocated; a call that fails is
     followed by a reset of its counter area on the same stream (``guard``),
     so an interrupted call cannot poison later ones.
     One buffer per (device, stream), so concurrent streams never share one; a
     larger request allocates a new buffer through PyTorch's stream-ordered
-    caching allocator.  With the extension the buffers are its own, shared with
-    the native call path.
+    caching allocator.  A call under HIP graph capture never gets that buffer,
+    whose place may change while the graph lives, but one of the graph's memory
+    pool (here one per call).  With the extension the buffers are its own, shared
+    with the native call path.
     """
 
     def __init__(self):
@@ -170,11 +172,14 @@ class _Workspace:
     def get(self, device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
         if _native is not None:
             return _native.workspace(device.index, stream, nbytes)
+        size = max(nbytes, 1 << 20)
+        with torch.cuda.device(device):
+            if torch.cuda.is_current_stream_capturing():
+                return torch.zeros(size, dtype=torch.uint8, device=device)
         key = (device, stream)   # one buffer per stream: calls on one stream never overlap
         with self._lock:
             buf = self._bufs.get(key)
             if buf is None or buf.numel() < nbytes:
-                size = max(nbytes, 1 << 20)
                 buf = torch.zeros(size, dtype=torch.uint8, device=device)
                 self._bufs[key] = buf
             return buf
