@@ -16,6 +16,7 @@
 #include <string>
 #include <torch/extension.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/core/DeviceGuard.h>
 
@@ -55,10 +56,12 @@ torch::Tensor workspace(int device, hipStream_t stream, size_t need) {
     torch::Tensor &buf = capturing ? b.captured : b.eager;
     if (!buf.defined() || (size_t)buf.numel() < need || (capturing && b.capture != id)) {
         const size_t bytes = std::max<size_t>(need, 1 << 20);
-        torch::Tensor t = torch::empty({(int64_t)bytes}, torch::TensorOptions().dtype(torch::kUInt8).device(torch::kCUDA, device));
+        // Straight from the allocator: through the dispatcher, a call under a tracing or transform
+        // mode would leave that mode's tensor, which has no memory, for every later call.
+        const torch::Tensor t = at::detail::empty_cuda({(int64_t)bytes}, at::kByte, at::Device(at::kCUDA, (c10::DeviceIndex)device), std::nullopt);
         const int st = mcq4_reset_workspace(t.data_ptr(), bytes, stream);
         TORCH_CHECK(st == MCQ4_OK, "workspace: ", mcq4_last_error());
-        buf = std::move(t);
+        buf = t;
         if (capturing) b.capture = id;
     }
     return buf;
