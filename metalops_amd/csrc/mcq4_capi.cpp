@@ -311,6 +311,7 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
                     workspace ? workspace_bytes : (size_t)0);
     if (need && !aligned(workspace, 16))
         return fail(MCQ4_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
+    if (!aligned(workspace, 16)) workspace = nullptr;   // optional from here on: K stays whole
     hipError_t e;
     // 33..64 rows: q4_gemm6 (flat ~31 us for any M <= 128 on 4096x14336) beats the
     // register-load decode kernel (40-77 us) wherever its alignment rules hold.

@@ -191,6 +191,7 @@ int matmul_common(int act, const void *X, int x_dtype, int64_t ldx, const uint8_
                     workspace ? workspace_bytes : (size_t)0);
     if (need && !aligned(workspace, 16))
         return fail(MCQ4_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
+    if (!aligned(workspace, 16)) workspace = nullptr;   // optional from here on
     hipStream_t st = (hipStream_t)stream;
     hipError_t e;
     if (path == I4Path::Gemm && f16_mid(M, wb, x_dtype) && mcq4::wx_supported(wx) &&
