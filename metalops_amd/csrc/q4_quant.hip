@@ -1,9 +1,8 @@
 // block_q4_0 quantize / dequantize kernels for gfx950.
 //
-// The wide kernels (the default where the columns and pointers allow) give a
-// thread C neighbouring columns of one K block: vector loads and stores along the
-// rows, and the 18 C contiguous bytes of its blocks as whole dwords.  The
-// one-column kernels below them take every other shape.
+// A thread owns one block (quantize) or two neighbouring ones (16-bit dequantize; four
+// to fp32 in large calls) of a K block row; the one-column dequantize kernel takes
+// every other shape.
 #include "convert_common.h"
 
 namespace mcq4 {
@@ -11,12 +10,22 @@ namespace mcq4 {
 // Reference rule, quantization.py:333-369, for a weight of dtype DT (fp32,
 // fp16 or bf16).  The reference runs every step as a torch op on the weight's
 // own dtype, so each step here is one fp32 IEEE operation (the file is
-// compiled with -ffp-contract=off, and '/' is the correctly rounded divide)
-// followed by a rounding to DT: amax (exact), amax/7, x/d, +8, round half to
-// even (rintf, exact in DT), clamp.  For fp16 and bf16 the fp32 result rounded
-// to DT equals the correctly rounded DT operation (fp32 carries more than
-// 2p + 2 bits for both, so the double rounding is innocuous).  d is stored as
-// fp16 (d.to(float16), quantization.py:352), one more rounding for bf16.
+// compiled with -ffp-contract=off) followed by a rounding to DT: amax (exact),
+// amax/7, x/d, +8, round half to even (rintf, exact in DT), clamp.  For fp16
+// and bf16 the fp32 result rounded to DT equals the correctly rounded DT
+// operation (fp32 carries more than 2p + 2 bits for both, so the double rounding
+// is innocuous).  d is stored as fp16 (d.to(float16), quantization.py:352), one
+// more rounding for bf16.
+//
+// Quotients come from one IEEE reciprocal per block (div_by, bit-equal to the
+// division) and roundings to DT from the hardware: with a division per element the
+// arithmetic was half the time again in large calls.  One column per thread,
+// although the accesses are narrow: the arithmetic of a block is a serial chain,
+// and two or four columns of it in one thread leave too few waves in flight.
+// us on fresh inputs, division per element / this / four (fp32: two) columns per thread:
+// bf16 4096x14336 56.7 / 29.7 / 35.6 (a copy of the bytes 29), 4096x4096 18.7 / 11.1 /
+// 15.1, 32x4096 5.3 / 3.2 / 6.5; fp16 1024x1024 4.0 / 3.6 / 6.9; fp32 4096x2048 10.6 /
+// 9.1 / 11.4.
 template <int DT>
 __global__ void __launch_bounds__(256)
 quantize_ref_kernel(const void *__restrict__ W, int64_t ldw, int nb, int N,
@@ -33,86 +42,31 @@ quantize_ref_kernel(const void *__restrict__ W, int64_t ldw, int nb, int N,
         x[j] = load_dt(W, base + (int64_t)j * ldw, DT);
         amax = fmaxf(amax, fabsf(x[j]));
     }
-    float d = round_dt(amax / 7.0f, DT);
+    float d = round_hw<DT>(amax / 7.0f);
     d = (d > 0.0f) ? d : 1.0f;
-    uint32_t q[QK];
-#pragma unroll
-    for (int j = 0; j < QK; ++j) {
-        const float t = round_dt(round_dt(x[j] / d, DT) + 8.0f, DT);
-        float r = __builtin_rintf(t);
-        r = fminf(fmaxf(r, 0.0f), 15.0f);
-        q[j] = (uint32_t)r;
-    }
     uint16_t *dst = (uint16_t *)(out + ((int64_t)kb * N + n) * BLOCK_BYTES);
+    uint32_t h[8];
+    auto codes = [&](auto fast) {
+        const float y = 1.0f / d;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            h[i] = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                float t0 = div_by<decltype(fast)::value, DT>(x[4 * i + e], d, y);
+                float t1 = div_by<decltype(fast)::value, DT>(x[4 * i + e + 1], d, y);
+                round_hw2<DT>(t0, t1);
+                t0 += 8.0f; t1 += 8.0f;
+                round_hw2<DT>(t0, t1);
+                h[i] |= code4(t0, 15.0f) << (4 * e) | code4(t1, 15.0f) << (4 * e + 4);
+            }
+        }
+    };
+    if (__all(div_by_fits(d))) codes(std::true_type{});
+    else codes(std::false_type{});
     dst[0] = bitcast<uint16_t>(to_half_exact(d));
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-        dst[1 + i] = (uint16_t)(q[4 * i] | (q[4 * i + 1] << 4) | (q[4 * i + 2] << 8) |
-                                (q[4 * i + 3] << 12));
-}
-
-// The same rule, C neighbouring columns of one K block per thread (N % C == 0, rows
-// aligned to C elements).  Bound by the weight's bytes beside the arithmetic:
-// quotients from one IEEE reciprocal per block (div_by, bit-equal to the
-// division) and hardware rounding to the dtype.  Weights and block bytes move as
-// whole dwords (the one-column kernel: 2-byte loads, 2-byte stores 18 bytes apart).
-// 4096x14336 bf16 38 us, fp32 60 (copies of the bytes moved: 29, 52).
-template <int DT, int C>
-__global__ void __launch_bounds__(256)
-quantize_ref_wide_kernel(const void *__restrict__ W, int64_t ldw, int nb, int N, uint8_t *__restrict__ out) {
-#pragma clang fp contract(off)
-    constexpr int ES = DT == DT_F32 ? 4 : 2, DW = C * ES / 4;   // dwords per row
-    typedef uint32_t vec_t __attribute__((ext_vector_type(DW)));
-    const int n = (blockIdx.x * 256 + threadIdx.x) * C, kb = blockIdx.y;
-    if (n >= N) return;
-    const uint8_t *src = (const uint8_t *)W + ((int64_t)kb * QK * ldw + n) * ES;
-    vec_t raw[QK];
-#pragma unroll
-    for (int j = 0; j < QK; ++j) raw[j] = *(const vec_t *)(src + (int64_t)j * ldw * ES);
-    uint32_t ob[(18 * C + 3) / 4];
-#pragma unroll
-    for (int i = 0; i < (18 * C + 3) / 4; ++i) ob[i] = 0u;
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        auto val = [&](int j) { return elem_f32<DT>(raw[j][DW == 1 ? 0 : c * ES / 4], c); };
-        float amax = 0.0f;
-#pragma unroll
-        for (int j = 0; j < QK; ++j) amax = fmaxf(amax, fabsf(val(j)));
-        float d = round_hw<DT>(amax / 7.0f);
-        d = (d > 0.0f) ? d : 1.0f;
-        uint32_t h[9];                           // the block's 2-byte words
-        h[0] = bitcast<uint16_t>(to_half_exact(d));
-        auto body = [&](auto fast) {
-            const float y = 1.0f / d;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                uint32_t w = 0;
-#pragma unroll
-                for (int e = 0; e < 4; e += 2) {
-                    float t0 = div_by<decltype(fast)::value, DT>(val(4 * i + e), d, y);
-                    float t1 = div_by<decltype(fast)::value, DT>(val(4 * i + e + 1), d, y);
-                    round_hw2<DT>(t0, t1);
-                    t0 += 8.0f; t1 += 8.0f;
-                    round_hw2<DT>(t0, t1);
-                    w |= code4(t0, 15.0f) << (4 * e) | code4(t1, 15.0f) << (4 * e + 4);
-                }
-                h[1 + i] = w;
-            }
-        };
-        if (__all(div_by_fits(d))) body(std::true_type{});
-        else body(std::false_type{});
-#pragma unroll
-        for (int i = 0; i < 9; ++i) ob[(9 * c + i) / 2] |= h[i] << (16 * ((9 * c + i) & 1));
-    }
-    // 18 C bytes at a multiple of 2 C: dwords (C even), pairs of them for C == 4.
-    uint32_t *dst = (uint32_t *)(out + ((int64_t)kb * N + n) * BLOCK_BYTES);
-    if constexpr (C == 4) {
-#pragma unroll
-        for (int i = 0; i < 9; ++i) ((u32x2 *)dst)[i] = u32x2{ob[2 * i], ob[2 * i + 1]};
-    } else {
-#pragma unroll
-        for (int i = 0; i < 9; ++i) dst[i] = ob[i];
-    }
+    for (int i = 0; i < 8; ++i) dst[1 + i] = (uint16_t)h[i];
 }
 
 // llama.cpp quantize_row_q4_0_ref rule in the same layout: d = max_signed / -8,
@@ -237,21 +191,9 @@ dequant_wide_kernel(const uint8_t *__restrict__ blocks, int nb, int N, void *__r
 // ---- launchers (called from the C ABI layer) -------------------------------
 namespace mcq4 {
 
-template <int DT, int C>
-static bool quantize_wide(const void *W, int64_t ldw, int nb, int N, uint8_t *out, hipStream_t s) {
-    const int64_t es = DT == DT_F32 ? 4 : 2;
-    if (N % C || ldw % C || (uintptr_t)W % (C * es) || (uintptr_t)out % (C == 4 ? 8 : 4)) return false;
-    hipLaunchKernelGGL((quantize_ref_wide_kernel<DT, C>), dim3((N / C + 255) / 256, nb), dim3(256), 0, s, W, ldw, nb, N, out);
-    return true;
-}
-
 hipError_t launch_quantize_typed(int w_dtype, const void *W, int64_t ldw, int nb, int N,
                                  uint8_t *out, hipStream_t s) {
     dim3 grid((N + 255) / 256, nb), block(256);
-    const bool wide = w_dtype == DT_F16    ? quantize_wide<DT_F16, 4>(W, ldw, nb, N, out, s)
-                      : w_dtype == DT_BF16 ? quantize_wide<DT_BF16, 4>(W, ldw, nb, N, out, s)
-                                           : quantize_wide<DT_F32, 2>(W, ldw, nb, N, out, s);
-    if (wide) return hipGetLastError();
     if (w_dtype == DT_F16)
         hipLaunchKernelGGL(quantize_ref_kernel<DT_F16>, grid, block, 0, s, W, ldw, nb, N, out);
     else if (w_dtype == DT_BF16)

@@ -1,5 +1,6 @@
-"""The wide conversion kernels (several columns per thread) against the oracles and,
-on special values, against the one-column kernels, which an odd row stride selects.
+"""The conversion kernels (one or several columns per thread) against the oracles and, on
+special values, against the rule in numpy (q4_0) and the one-column kernels, which an odd
+row stride selects (INT4).
 
 All exact: bytes, scales, zeros and outputs are compared bit for bit."""
 import numpy as np
@@ -67,3 +68,34 @@ def test_wide_matches_one_column_on_specials(dev, dtype, std):
     if dtype == R.F32:
         for a, b in zip(mo.quantize_to_int4(w, 128), mo.quantize_to_int4(_odd(w), 128)):
             assert torch.equal(_bits(a), _bits(b))
+
+
+def _q4_rule(w, dtype):
+    """The q4_0 rule of the kernels, a NaN weight left out of amax and coded 0: one IEEE operation and one
+    rounding to the dtype per step."""
+    x = w.reshape(w.shape[0] // 32, 32, w.shape[1])
+    amax = np.fmax.reduce(np.abs(x), axis=1, initial=np.float32(0))
+    d = R.round_to(amax / np.float32(7), dtype)
+    d = np.where(d > 0, d, np.float32(1))
+    t = R.round_to(R.round_to(x / d[:, None], dtype) + np.float32(8), dtype)
+    q = np.fmin(np.fmax(np.rint(t), 0), 15).astype(np.uint8).reshape(x.shape[0], 8, 4, -1).astype(np.uint16)
+    words = q[:, :, 0] | q[:, :, 1] << 4 | q[:, :, 2] << 8 | q[:, :, 3] << 12
+    out = np.empty((x.shape[0], x.shape[2], 9), np.uint16)
+    out[:, :, 0] = R.round_to(d, R.F16).astype(np.float16).view(np.uint16)
+    out[:, :, 1:] = words.transpose(0, 2, 1)
+    return out.view(np.uint8)
+
+
+# Scales inside the range of the reciprocal form and outside it, and both in one wave.
+@pytest.mark.parametrize("dtype", [R.F32, R.F16, R.BF16])
+@pytest.mark.parametrize("std", [0.02, 3e3, 1e-7, 1e-25])
+@pytest.mark.parametrize("N", [1, 257, 1024])
+def test_q4_rule_on_specials(dev, dtype, std, N):
+    import metalops_amd as mo
+    g = torch.Generator().manual_seed(11)
+    w = (torch.randn(320, N, generator=g) * std * torch.exp(6 * torch.randn(1, N, generator=g))).to(TDT[dtype])
+    w[::97, ::31], w[::89, ::37], w[::83, ::41] = float("nan"), float("inf"), -float("inf")
+    w[64:96], w[::53, ::3] = 0, -0.0
+    with np.errstate(all="ignore"):
+        want = _q4_rule(w.float().numpy(), dtype)
+    assert np.array_equal(mo.quantize_ggml_q4_0(w.to(dev)).cpu().numpy(), want)
