@@ -131,33 +131,38 @@ dequant_kernel(const uint8_t *__restrict__ blocks, int nb, int N, void *__restri
     }
 }
 
-// Four neighbouring columns of one K block per thread (N % 4 == 0, 8-byte aligned
-// blocks, rows aligned to four elements): the 72 block bytes as nine 8-byte loads,
-// every output row as one 8- or 16-byte store.  fp16: the exact q - 8 times d in
-// one multiply, the single rounding of the exact product; bf16: that product
-// rounded from fp32, where it is exact; fp32: exact.  4096x14336 to fp16 27 us, to
-// fp32 45, what copies of the bytes moved take (29, 52).
-template <int DT>
+// C neighbouring columns of one K block per thread (N % C == 0, blocks aligned to 2 C
+// bytes, rows to C elements): the 18 C block bytes in dwords (C = 4: pairs), every
+// output row as one store.  fp16: the exact q - 8 times d in one multiply, the
+// single rounding of the exact product; bf16: that product rounded from fp32,
+// where it is exact; fp32: exact.
+// Bound by the output's bytes.  16 bits: C = 2 everywhere (us on fresh blocks, one
+// column / 2 / 4: fp16 4096x4096 9.8 / 8.5 / 12.0, 4096x14336 35.2 / 27.3 / 28.8, 1024x1024
+// 3.6 / 2.9 / 3.3; with four, 4096 columns leave two workgroups a CU).  fp32:
+// dequant_wide_f32 below.
+template <int DT, int C>
 __global__ void __launch_bounds__(256)
 dequant_wide_kernel(const uint8_t *__restrict__ blocks, int nb, int N, void *__restrict__ out, int64_t ldo) {
 #pragma clang fp contract(off)
-    const int n = (blockIdx.x * 256 + threadIdx.x) * 4, kb = blockIdx.y;
+    typedef uint32_t in_t __attribute__((ext_vector_type(C / 2)));
+    const int n = (blockIdx.x * 256 + threadIdx.x) * C, kb = blockIdx.y;
     if (n >= N) return;
-    const u32x2 *src = (const u32x2 *)(blocks + ((int64_t)kb * N + n) * BLOCK_BYTES);
-    uint32_t raw[18];
+    const in_t *src = (const in_t *)(blocks + ((int64_t)kb * N + n) * BLOCK_BYTES);
+    uint32_t raw[9 * C / 2];
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
-        const u32x2 v = src[i];
-        raw[2 * i] = v[0]; raw[2 * i + 1] = v[1];
+        const in_t v = src[i];
+#pragma unroll
+        for (int j = 0; j < C / 2; ++j) raw[C / 2 * i + j] = v[j];
     }
     auto half_at = [&](int c, int i) { return (raw[(9 * c + i) / 2] >> (16 * ((9 * c + i) & 1))) & 0xFFFFu; };   // 2-byte word i of column c
     const int64_t o0 = (int64_t)kb * QK * ldo + n;
     const half2_t o1024 = {(_Float16)1032.0f, (_Float16)1032.0f};
 #pragma unroll
     for (int i = 0; i < 8; ++i) {                 // rows 4 i .. 4 i + 3
-        half2_t q01[4], q23[4];                   // q - 8 of the rows' pairs, per column
+        half2_t q01[C], q23[C];                   // q - 8 of the rows' pairs, per column
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < C; ++c) {
             const uint32_t w = half_at(c, 1 + i);
             q01[c] = bitcast<half2_t>((w & 0xFu) | ((w & 0xF0u) << 12) | 0x64006400u) - o1024;
             q23[c] = bitcast<half2_t>(((w >> 8) & 0xFu) | ((w & 0xF000u) << 4) | 0x64006400u) - o1024;
@@ -166,21 +171,26 @@ dequant_wide_kernel(const uint8_t *__restrict__ blocks, int nb, int N, void *__r
         for (int e = 0; e < 4; ++e) {
             const int64_t o = o0 + (int64_t)(4 * i + e) * ldo;
             if constexpr (DT == DT_F16) {
-                half4_t v;
+                typedef _Float16 out_t __attribute__((ext_vector_type(C)));
+                out_t v;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) v[c] = (e < 2 ? q01[c][e] : q23[c][e - 2]) * bitcast<_Float16>((uint16_t)half_at(c, 0));
-                *(half4_t *)((_Float16 *)out + o) = v;
+                for (int c = 0; c < C; ++c) v[c] = (e < 2 ? q01[c][e] : q23[c][e - 2]) * bitcast<_Float16>((uint16_t)half_at(c, 0));
+                *(out_t *)((_Float16 *)out + o) = v;
             } else {
-                float v[4];
+                typedef float out_t __attribute__((ext_vector_type(C)));
+                out_t v;
 #pragma unroll
-                for (int c = 0; c < 4; ++c)
+                for (int c = 0; c < C; ++c)
                     v[c] = (float)(e < 2 ? q01[c][e] : q23[c][e - 2]) * (float)bitcast<_Float16>((uint16_t)half_at(c, 0));
-                if constexpr (DT == DT_F32)
-                    *(float4_t *)((float *)out + o) = float4_t{v[0], v[1], v[2], v[3]};
-                else
-                    *(u32x2 *)((uint16_t *)out + o) =
-                        u32x2{bitcast<uint32_t>(__builtin_convertvector((float2_t{v[0], v[1]}), bf16x2_t)),
-                              bitcast<uint32_t>(__builtin_convertvector((float2_t{v[2], v[3]}), bf16x2_t))};
+                if constexpr (DT == DT_F32) {
+                    *(out_t *)((float *)out + o) = v;
+                } else {
+                    in_t u;
+#pragma unroll
+                    for (int j = 0; j < C / 2; ++j)
+                        u[j] = bitcast<uint32_t>(__builtin_convertvector((float2_t{v[2 * j], v[2 * j + 1]}), bf16x2_t));
+                    *(in_t *)((uint16_t *)out + o) = u;
+                }
             }
         }
     }
@@ -211,10 +221,20 @@ hipError_t launch_quantize(bool llama_rule, const float *W, int64_t ldw, int nb,
     return hipGetLastError();
 }
 
+// fp32 out: four columns per thread above 8 M weights, unless more than a sixteenth of
+// the last workgroup's threads in a row would be idle; one column otherwise.  us on fresh
+// blocks, one / four: 4096x4096 17.0 / 13.4, 2048x8192 16.2 / 13.0, 14336x14336 180 / 180,
+// 4096x2048 8.1 / 8.0; 1024x1024 2.9 / 3.8, 8192x1536 10.2 / 11.5.
+static bool dequant_wide_f32(int nb, int N) {
+    return (int64_t)nb * QK * N > ((int64_t)1 << 23) && (N + 1023) / 1024 * 1024 - N <= N / 16;
+}
+
 template <int DT>
 static hipError_t launch_dequant_t(const uint8_t *blocks, int nb, int N, void *out, int64_t ldo, hipStream_t s) {
-    const bool wide = N % 4 == 0 && ldo % 4 == 0 && (uintptr_t)blocks % 8 == 0 && (uintptr_t)out % (DT == DT_F32 ? 16 : 8) == 0;
-    if (wide) hipLaunchKernelGGL(dequant_wide_kernel<DT>, dim3((N / 4 + 255) / 256, nb), dim3(256), 0, s, blocks, nb, N, out, ldo);
+    constexpr int C = DT == DT_F32 ? 4 : 2;
+    const bool wide = N % C == 0 && ldo % C == 0 && (uintptr_t)blocks % (2 * C) == 0 && (uintptr_t)out % (DT == DT_F32 ? 16 : 4) == 0 &&
+                      (DT != DT_F32 || dequant_wide_f32(nb, N));
+    if (wide) hipLaunchKernelGGL((dequant_wide_kernel<DT, C>), dim3((N / C + 255) / 256, nb), dim3(256), 0, s, blocks, nb, N, out, ldo);
     else hipLaunchKernelGGL(dequant_kernel<DT>, dim3((N + 255) / 256, nb), dim3(256), 0, s, blocks, nb, N, out, ldo);
     return hipGetLastError();
 }

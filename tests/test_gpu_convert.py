@@ -99,3 +99,32 @@ def test_q4_rule_on_specials(dev, dtype, std, N):
     with np.errstate(all="ignore"):
         want = _q4_rule(w.float().numpy(), dtype)
     assert np.array_equal(mo.quantize_ggml_q4_0(w.to(dev)).cpu().numpy(), want)
+
+
+# Widths around two and four columns per thread, row strides and addresses that leave them, and the
+# fp32 sizes (above 8 M weights) on both sides of the idle-thread line.
+@pytest.mark.parametrize("K,N,pad,off", [(64, 2, 0, 0), (64, 510, 1, 0), (96, 514, 2, 1), (32, 1023, 0, 0), (64, 1026, 0, 2),
+                                         (64, 260, 4, 0), (8224, 1024, 0, 0), (5504, 1536, 0, 0), (8224, 1024, 0, 1)])
+def test_q4_dequantize_layouts(dev, K, N, pad, off):
+    """dequantize through the C entry: padded rows and an `out` at an odd element."""
+    from metalops_amd import _lib
+    L = _lib.lib
+    b = torch.randint(0, 256, (K // 32, N, 18), dtype=torch.uint8, generator=torch.Generator().manual_seed(K + N))
+    b[:, :, 1] = (b[:, :, 1] & 0x83) | 0x20          # finite scales, both signs
+    exact = Q.dequantize(b.numpy(), np.float32)
+    d = b.to(dev)
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    for out in (R.F32, R.F16, R.BF16):
+        store = torch.full((K * (N + pad) + off + 8,), -1.0, dtype=TDT[out], device=dev)
+        y = store[off:off + K * (N + pad)].view(K, N + pad)
+        if out == R.BF16:
+            st = L.mcq4_dequantize_q4_0_bf16(d.data_ptr(), K, N, y.data_ptr(), N + pad, stream)
+        else:
+            st = L.mcq4_dequantize_q4_0(d.data_ptr(), K, N, y.data_ptr(), N + pad,
+                                        _lib.MCQ4_DTYPE_F16 if out == R.F16 else _lib.MCQ4_DTYPE_F32, stream)
+        assert st == _lib.MCQ4_OK
+        torch.cuda.synchronize(dev)
+        want = R.round_to(exact, out)
+        assert np.array_equal(y[:, :N].float().cpu().numpy(), want)
+        assert np.array_equal(np.signbit(y[:, :N].float().cpu().numpy()), np.signbit(want))
+        assert bool((store[:off] == -1).all()) and bool((y[:, N:] == -1).all()) and bool((store[-8:] == -1).all())
