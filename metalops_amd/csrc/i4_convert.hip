@@ -199,7 +199,10 @@ __global__ void __launch_bounds__(64 * SL) i4_quantize_wide_kernel(I4QuantArgs a
 // The wide dequantizer: four columns and eight byte rows per thread (N % 4 == 0,
 // group sizes that are multiples of 16, aligned pointers): one scale and zero load
 // per 16 rows, 4-byte packed loads, every output row as one 8- or 16-byte store.
-// 4096x14336 to fp16 32.7 us, what a copy of the bytes moved takes.
+// 4096x14336 to fp16 32.7 us, what a copy of the bytes moved takes.  From 384 K
+// weights on: below, 16 rows of four columns a thread leave most of the CUs idle (us on
+// fresh codes, one byte per thread / this: fp32 1024x256 3.2 / 3.4, fp16 128x1024 3.0 / 3.3,
+// 32x4096 3.1 / 3.4; 512x1024 3.7 / 3.4, 32x14336 3.6 / 3.5).
 template <int SZ, int OUT>
 __global__ void __launch_bounds__(256) i4_dequant_wide_kernel(I4DequantArgs a) {
 #pragma clang fp contract(off)
@@ -288,7 +291,7 @@ hipError_t launch_i4_dequant(const uint8_t *packed, const void *scales, const vo
     a.packed = packed; a.scales = scales; a.zeros = zeros;
     a.sz_dt = sz_dt; a.out_dt = out_dt;
     a.Kh = K / 2; a.N = N; a.gs = gs; a.ldo = ldo; a.out = out;
-    if (N % 4 == 0 && ldo % 4 == 0 && gs % 16 == 0 && (uintptr_t)packed % 4 == 0 && (uintptr_t)out % (out_dt == DT_F32 ? 16 : 8) == 0) {
+    if (K * N >= 3 << 17 && N % 4 == 0 && ldo % 4 == 0 && gs % 16 == 0 && (uintptr_t)packed % 4 == 0 && (uintptr_t)out % (out_dt == DT_F32 ? 16 : 8) == 0) {
         const int64_t ry = (a.Kh + 7) / 8;
         const dim3 grid((unsigned)((N / 4 + 255) / 256), (unsigned)(ry < 65535 ? ry : 65535));
         auto go = [&](auto sz) {

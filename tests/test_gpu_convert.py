@@ -27,9 +27,9 @@ def _bits(t):
 
 
 # Columns: one thread, the last column set of a workgroup, past it.  K: one block or group,
-# a last group that is not whole.
+# a last group that is not whole.  From 384 K weights on INT4 dequantizes four columns a thread.
 @pytest.mark.parametrize("K,N,gs", [(32, 4, 32), (64, 252, 64), (128, 260, 128), (160, 1028, 128), (288, 516, 64),
-                                    (70, 8, 32), (4096, 1024, 128)])
+                                    (70, 8, 32), (4096, 1024, 128), (1030, 516, 32), (1550, 260, 128), (98310, 4, 64)])
 @pytest.mark.parametrize("dtype", [R.F32, R.F16, R.BF16])
 def test_wide_matches_oracle(dev, dtype, K, N, gs):
     import metalops_amd as mo
