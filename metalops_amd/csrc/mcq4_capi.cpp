@@ -129,6 +129,38 @@ size_t prefill_ws_bytes(int64_t M, int64_t K, int64_t N) {
                      mcq4::gemm8_workspace_bytes(M, K, N)});
 }
 
+// Switches (tests) that leave 17..64 fp16 rows to the decode kernels.
+bool decode_switch() {
+    return mcq4::opt("MCQ4_GEMVM_SPLIT") || mcq4::opt("MCQ4_GEMV_PATH") || mcq4::opt("MCQ4_DECODE_PATH");
+}
+
+// 33..64 fp16 rows that the strip kernels keep (8 columns: q4_skinny): at most 4096 columns in
+// strips of 16 are one round of workgroups, and wx_mid's K split and its reduction
+// launch cost more than they save on short K.  us, strips / wx_mid: M=48 1024x528 5.7 / 8.7, M=33 2048x1040
+// 8.3 / 8.6, M=64 1536x1040 9.6 / 9.8, M=33 128x8 3.8 / 4.7; M=48 3072x528 11.1 / 9.4, M=64
+// 2048x512 10.2 / 9.3, M=48 1024x4112 9.2 / 9.3.
+bool strip_rows(int64_t M, int64_t K, int64_t N) {
+    return ((N % 16 == 0 && N <= 4096) || N == 8) && K < (M <= 48 ? 2560 : 2048);
+}
+
+// 17..64 fp16 rows of the kernel between the decode and the prefill ones (wx_mid).  Up to 32
+// rows from K = 4096 on (us, q4_gemvm / wx_mid: M=32 4096x14336 18.4 / 13.5, M=17 4096x4096
+// 9.3 / 8.8; M=32 2048x4096 7.3 / 7.6, M=17 1024x4096 4.7 / 6.4).  Above, where the strips do
+// not keep them, up to 16384 columns (256 tiles of 64, one per CU) at any K; in further
+// rounds of tiles once K is long enough for the weights' bytes to count, and above 56 rows
+// not where the few-tile prefill kernel (q4_gemm8) has one round of workgroups, up to K = 4096.
+// us, prefill kernel / wx_mid: M=64 4096x14336 29.3 / 17.6, 256x16384 10.7 / 6.3, 256x17920
+// 10.7 / 10.1; M=48 128x17920 8.8 / 8.6, 128x128256 24.4 / 29.2, 512x128256 39.9 / 40.7; M=64
+// 512x32000 11.9 / 13.0, 3072x32000 30.8 / 32.8, 4096x32000 39.7 / 36.5, 3072x49152 70.6 / 48.0.
+bool mid_rows(int64_t M, int64_t K, int64_t N) {
+    if (M <= 16 || M > 64) return false;
+    if (M <= 32) return K >= 4096;
+    if (strip_rows(M, K, N)) return false;
+    if (N <= 16384) return true;
+    const int64_t g8 = N % 128 == 0 ? mcq4::gemm8_workgroups(M, K, N) : 0;
+    return K >= (N <= 65536 ? 256 : 512) && !(M > 56 && K < 4096 && g8 >= 192 && g8 <= 256);
+}
+
 int check_kn(int64_t K, int64_t N) {
     if (K <= 0 || N <= 0) return fail(MCQ4_ERR_SHAPE, "K (%lld) and N (%lld) must be positive",
                                       (long long)K, (long long)N);
@@ -313,15 +345,8 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
         return fail(MCQ4_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
     if (!aligned(workspace, 16)) workspace = nullptr;   // optional from here on: K stays whole
     hipError_t e;
-    // 33..64 rows: q4_gemm6 (flat ~31 us for any M <= 128 on 4096x14336) beats the
-    // register-load decode kernel (40-77 us) wherever its alignment rules hold.
-    // 17..64 rows: the kernel between the decode and the prefill ones; up to 32 rows from
-    // K = 4096 on (us, q4_gemvm / wx_mid: M=32 4096x14336 18.4 / 13.5, M=17 4096x4096 9.3 /
-    // 8.8; M=32 2048x4096 7.3 / 7.6, M=17 1024x4096 4.7 / 6.4).  MCQ4_GEMVM_SPLIT,
-    // MCQ4_GEMV_PATH, MCQ4_DECODE_PATH (tests) leave these rows to the decode kernels.
     const mcq4::WxCall wx = {mcq4::WX_Q4, mcq4::DT_F16, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32};
-    if (M > 16 && M <= 64 && (M > 32 || K >= 4096) && mcq4::wx_mid_supported(wx) && !mcq4::opt("MCQ4_GEMVM_SPLIT") && !mcq4::opt("MCQ4_GEMV_PATH") &&
-        !mcq4::opt("MCQ4_DECODE_PATH"))
+    if (mid_rows(M, K, N) && mcq4::wx_mid_supported(wx) && !decode_switch())
         return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
     // Up to 64 rows of weights the strip kernels do not take (odd column counts or
     // addresses): LDS sums over 16 or 8 waves instead of q4_skinny's 4, from K = 4096 on
@@ -334,7 +359,10 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
         !mcq4::opt("MCQ4_DECODE_PATH") &&
         mcq4::wx_workspace_bytes(mcq4::WX_Q4, mcq4::DT_F16, M, K, N) <= (workspace ? workspace_bytes : (size_t)0))
         return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
-    const bool skinny = M <= 32 || (M <= 64 && !mcq4::gemm6_supported((const _Float16 *)X, ldx, W, M, K, N));
+    // 33..64 rows left to here: the strips' shapes, and q4_gemm6 beyond them (by a switch,
+    // where N % 128 == 0).
+    const bool skinny = M <= 32 || (M <= 64 && (!mcq4::gemm6_supported((const _Float16 *)X, ldx, W, M, K, N) ||
+                                                (decode_switch() ? N % 128 != 0 : strip_rows(M, K, N))));
     if (skinny)
         e = mcq4::launch_skinny((const _Float16 *)X, ldx, W, (_Float16 *)Y, ldy, (int)M, (int)K,
                                 (int)N, workspace, (hipStream_t)stream);
