@@ -161,6 +161,19 @@ bool mid_rows(int64_t M, int64_t K, int64_t N) {
     return K >= (N <= 65536 ? 256 : 512) && !(M > 56 && K < 4096 && g8 >= 192 && g8 <= 256);
 }
 
+// Up to 64 fp16 rows of weights the strip kernels do not take (odd column counts or addresses)
+// that run wx_gemv / wx_skinny, LDS sums over 16 or 8 waves instead of q4_skinny's 4, with the
+// same arithmetic (weights rounded to fp16): more than 4096 columns from K = 4096 on, where
+// q4_skinny has a second round of workgroups; with fewer, once K outweighs the longer sums.
+// us, q4_skinny / wx: M=1 4096x4097 9.4 / 8.6, 4096x8193 14.7 / 10.5, M=16 4096x4097 13.9 / 11.7,
+// M=64 4096x8193 43.7 / 28.9; up to 4096 columns M=1 4096x1001 6.7 / 5.9, M=8 4096x33 7.1 / 7.5,
+// 5120x33 8.7 / 8.5, M=16 4096x3001 9.1 / 10.0, 8192x33 13.2 / 14.0, 10240x33 16.7 / 16.2, M=17
+// 4096x3001 9.7 / 11.0, 5120x3001 12.0 / 11.5, M=33 4096x4095 13.7 / 14.2, M=48 4096x3001 16.2 / 15.4.
+bool loose_rows(int64_t M, int64_t K, int64_t N) {
+    if (M > 64 || K < 4096) return false;
+    return N > 4096 || M <= 4 || M > 40 || K >= (M > 8 && M <= 16 ? 10240 : 5120);
+}
+
 int check_kn(int64_t K, int64_t N) {
     if (K <= 0 || N <= 0) return fail(MCQ4_ERR_SHAPE, "K (%lld) and N (%lld) must be positive",
                                       (long long)K, (long long)N);
@@ -348,15 +361,7 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
     const mcq4::WxCall wx = {mcq4::WX_Q4, mcq4::DT_F16, 0, mcq4::ACT_NONE, X, ldx, W, nullptr, nullptr, Y, ldy, M, K, N, 32};
     if (mid_rows(M, K, N) && mcq4::wx_mid_supported(wx) && !decode_switch())
         return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
-    // Up to 64 rows of weights the strip kernels do not take (odd column counts or
-    // addresses): LDS sums over 16 or 8 waves instead of q4_skinny's 4, from K = 4096 on
-    // (same arithmetic: weights rounded to fp16).  us, q4_skinny / wx_gemv, wx_skinny: M=1
-    // 4096x4101 9.5 / 7.8, 14336x4099 29.3 / 16.1, M=16 4096x12289 19.8 / 15.7, M=17
-    // 4096x4101 15.8 / 12.5, M=64 4096x12289 45.0 / 28.6; K = 2048: M=1 x1025 4.5 / 4.9,
-    // M=17 x4097 9.0 / 9.5.
-    const bool strips = N % 8 == 0 && aligned(W, 16);
-    if (M <= 64 && K >= 4096 && !strips && !mcq4::opt("MCQ4_GEMVM_SPLIT") && !mcq4::opt("MCQ4_GEMV_PATH") &&
-        !mcq4::opt("MCQ4_DECODE_PATH") &&
+    if (loose_rows(M, K, N) && !(N % 8 == 0 && aligned(W, 16)) && !decode_switch() &&
         mcq4::wx_workspace_bytes(mcq4::WX_Q4, mcq4::DT_F16, M, K, N) <= (workspace ? workspace_bytes : (size_t)0))
         return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, (hipStream_t)stream), "matmul launch");
     // 33..64 rows left to here: the strips' shapes, and q4_gemm6 beyond them (by a switch,

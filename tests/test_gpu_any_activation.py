@@ -79,12 +79,14 @@ def test_q4_narrow_prefill(dev, xdt, M, K, N):
 # sums, d applied in fp32), so the bar is that of fp32 sums against (q - 8) d itself.
 # Then 33..64 rows on both sides of each line of the dispatch: strips (unrounded too), the
 # kernel above them, prefill tiles beyond 16384 columns; the few-tile kernel's round.
-# Then weights the strip kernels do not take, at the K from which wx runs them.
+# Then weights the strip kernels do not take, on both sides of the K from which wx runs them.
 @pytest.mark.parametrize("M,K,N,exact", [(17, 4096, 8, True), (24, 4096, 136, True), (32, 14336, 64, True), (31, 4128, 4096, True),
                                          (33, 2528, 16, True), (64, 1024, 4096, True), (48, 32, 8, False), (33, 2560, 16, False),
                                          (40, 1024, 4112, False), (64, 2048, 24, False), (33, 224, 16392, False),
                                          (64, 256, 16392, False), (57, 256, 24576, False), (56, 256, 24576, False), (64, 2016, 32, True), (64, 2048, 32, False),
-                                         (1, 4096, 33, False), (16, 4128, 257, False), (17, 4096, 65, False), (64, 4096, 1025, False)])
+                                         (1, 4096, 33, False), (16, 4128, 257, False), (17, 4096, 65, False), (64, 4096, 1025, False),
+                                         (4, 4096, 33, False), (5, 4096, 33, False), (5, 5120, 33, False), (9, 10208, 33, False),
+                                         (9, 10240, 33, False), (16, 4096, 4097, False), (40, 5120, 65, False), (41, 4096, 65, False)])
 def test_q4_fp16_rows(dev, M, K, N, exact):
     import metalops_amd as mo
     print(f"q4 fp16 M={M} K={K} N={N}", flush=True)
