@@ -82,11 +82,12 @@ bool aligned(const void *p, uintptr_t a) { return ((uintptr_t)p % a) == 0; }
 // one round of workgroups, the 256 x 256-tile GEMM (q4_gemm7) on grids that
 // nearly fill the CUs, else the 128 x 256-tile LDS-staged GEMM with two waves per
 // SIMD (q4_gemm6).  Otherwise the kernel without alignment needs (wx_gemm).
+// fp16 on short K, unless N % 128 == 0 and aligned: the register-staged q4_gemm.
 // MCQ4_GEMM_PATH=sync|async|6|7|8 forces one kernel (tests; sync and async are
 // the fp16 kernels q4_gemm and q4_gemm2).
 enum class Prefill { Sync, Async2, Staged6, Wide7, Few8, Any };
 Prefill prefill_kernel(const _Float16 *X, int64_t ldx, const uint8_t *W, int64_t M, int64_t K,
-                       int64_t N) {
+                       int64_t N, bool f16) {
     const bool ok2 = mcq4::gemm2_supported(X, ldx, W, K, N);
     const bool ok6 = mcq4::gemm6_supported(X, ldx, W, M, K, N);
     if (const char *env = mcq4::opt("MCQ4_GEMM_PATH")) {
@@ -96,6 +97,15 @@ Prefill prefill_kernel(const _Float16 *X, int64_t ldx, const uint8_t *W, int64_t
         if (env[0] == '7' && mcq4::gemm7_supported(X, ldx, W, M, K, N)) return Prefill::Wide7;
         if (env[0] == '8' && mcq4::gemm8_supported(X, ldx, W, M, K, N)) return Prefill::Few8;
     }
+    // Short K: filling wx_gemm's register ring and two LDS slots and summing its phases takes
+    // about 10 us whatever K is, q4_gemm6's stages about 8; q4_gemm starts sooner, takes
+    // longer per K step and needs more rounds of workgroups on wide outputs.  us, q4_gemm /
+    // q4_gemm6: 300x32x1032 5.5 / 7.7, x128 8.1 / 8.9, x160 9.0 / 9.4, 2048x32x4104 16.3 / 11.3; /
+    // wx_gemm: 300x32x1001 5.4 / 10.7, x256 11.6 / 13.1, x384 15.2 / 14.9; 512x256x8193 13.5 /
+    // 14.8, 1024x128x6001 11.2 / 13.5, 300x192x14335 15.3 / 13.8; 2048x32x8193 40.3 / 32.3.
+    const int64_t t6 = ((M + 127) / 128) * ((N + 255) / 256);
+    if (f16 && (ok6 ? N % 128 != 0 && K < 160 && t6 <= 128 : K < (t6 <= 144 ? 384 : t6 <= 288 ? 160 : 0)))
+        return Prefill::Sync;
     // Measured (us per launch, `python bench.py --part prefill-routing`, one box;
     // default / q4_gemm6 / q4_gemm7 / q4_gemm8 forced):
     //   M=512 11008x4096 55.8 / 59.5 / 64.1 / 56.5, 4096x4096 29.3 / 31.7 / 35.6 / 29.3
@@ -375,7 +385,7 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y, 
         const _Float16 *x = (const _Float16 *)X;
         _Float16 *y = (_Float16 *)Y;
         hipStream_t st = (hipStream_t)stream;
-        switch (prefill_kernel(x, ldx, W, M, K, N)) {
+        switch (prefill_kernel(x, ldx, W, M, K, N, true)) {
             case Prefill::Staged6: e = mcq4::launch_gemm6(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, mcq4::DT_F16, workspace, st); break;
             case Prefill::Wide7: e = mcq4::launch_gemm7(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, mcq4::DT_F16, workspace, st); break;
             case Prefill::Few8: e = mcq4::launch_gemm8(x, ldx, W, y, ldy, (int)M, (int)K, (int)N, mcq4::DT_F16, workspace, st); break;
@@ -443,7 +453,7 @@ int mcq4_matmul_q4_0(const void *X, int x_dtype, int64_t ldx, const uint8_t *W, 
             _Float16 *y = (_Float16 *)Y;
             hipStream_t st = (hipStream_t)stream;
             const int m = (int)M, k = (int)K, n = (int)N, dt = mcq4::DT_BF16;
-            switch (prefill_kernel(x, ldx, W, M, K, N)) {
+            switch (prefill_kernel(x, ldx, W, M, K, N, false)) {
                 case Prefill::Staged6: return hip_status(mcq4::launch_gemm6(x, ldx, W, y, ldy, m, k, n, dt, workspace, st), "matmul launch");
                 case Prefill::Wide7: return hip_status(mcq4::launch_gemm7(x, ldx, W, y, ldy, m, k, n, dt, workspace, st), "matmul launch");
                 case Prefill::Few8: return hip_status(mcq4::launch_gemm8(x, ldx, W, y, ldy, m, k, n, dt, workspace, st), "matmul launch");

@@ -212,10 +212,14 @@ static int wx_skinny_splits(int64_t K, int64_t N) {
 static int64_t wx_ldp(int64_t N) { return (N + 3) / 4 * 4; }
 
 // Partials of q4_0 x fp16 stay within 16 MiB, what the allocation-free entry point holds.
+// q4_0 in 16 bits below K = 768 with 1 M outputs or more: no split, whose partials (16 bytes of
+// traffic an output, at about 5 TB/s) and second launch cost more than half the K steps: us,
+// two splits / none: 2048x512x1001 24.7 / 18.2, 300x512x6001 24.7 / 18.3, 128x640x14335 25.4 / 20.7.
 static int wx_splits(int wt, int x_dt, int64_t M, int64_t K, int64_t N) {
     if (wt == WX_Q4 && M <= 16) return 1;         // wx_gemv
     // One plan for a shape, whatever the alignment: wx_mid and wx_skinny share it.
     int S = wx_mid_shape(wt, x_dt, M, N) ? wx_mid_splits(K, N) : M <= 64 ? wx_skinny_splits(K, N) : wx_gemm_splits(x_dt, M, K, N);
+    if (wt == WX_Q4 && x_dt != DT_F32 && M > 64 && K < 768 && M * N >= (1 << 20)) S = 1;
     if (wt == WX_Q4 && x_dt == DT_F16)
         while (S > 1 && (int64_t)S * M * wx_ldp(N) * 4 > ((int64_t)16 << 20)) S /= 2;
     return S;

@@ -98,6 +98,22 @@ def test_q4_fp16_rows(dev, M, K, N, exact):
     _check(Y, X, W if exact else R.round_to(W, R.F16), R.F16)
 
 
+# Prefill on both sides of the short-K lines: N % 8 == 0 (K = 160, 128 tiles of 128 x 256), odd (K = 384,
+# up to 144 tiles, 160 up to 288), and the K split of 1 M outputs (K = 768).
+@pytest.mark.parametrize("M,K,N", [(65, 32, 8), (130, 128, 136), (130, 160, 136), (2048, 96, 2048 + 8), (65, 32, 1), (129, 352, 257),
+                                   (129, 384, 257), (1100, 352, 4001), (1153, 128, 4001), (1153, 160, 4001), (4736, 96, 2047), (1100, 736, 1001),
+                                   (1100, 768, 1001)])
+@pytest.mark.parametrize("xdt", [R.F16, R.BF16])
+def test_q4_short_k(dev, xdt, M, K, N):
+    import metalops_amd as mo
+    print(f"q4 short K {xdt} M={M} K={K} N={N}", flush=True)
+    w = np.random.default_rng(M + N).standard_normal((K, N), np.float32) * 0.02
+    b = Q.quantize_llama_rule(w)
+    X = _x(M, K, xdt, M + K)
+    Y = mo.matmul_ggml_q4_0(X.to(dev), torch.from_numpy(b).to(dev))
+    _check(Y, X, R.round_to(Q.dequantize(b, np.float32), xdt), xdt)
+
+
 @pytest.mark.parametrize("M,K,N,pad,off", [(5, 256, 33, 3, 0), (40, 256, 66, 8, 1), (100, 544, 70, 5, 3), (70, 512, 64, 0, 2)])
 @pytest.mark.parametrize("xdt", [R.BF16, R.F32])
 def test_q4_row_strides(dev, xdt, M, K, N, pad, off):
