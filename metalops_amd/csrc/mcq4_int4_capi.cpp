@@ -115,12 +115,30 @@ bool bf16_prefill(int64_t M, int64_t K, int wb, int x_dt) {
 
 // fp16 activations, up to 64 rows beyond the GEMVs' range: wx_skinny instead of the
 // GEMMs, whose 128-row tiles are mostly padding there.  us, GEMM / wx_skinny: INT4
-// M=33 4096x4096 24.5 / 13.7, M=48 4096x11008 29.4 / 22.5, M=64 4096x14336 31.9 /
-// 27.8; INT8 M=17 4096x4096 25.7 / 13.5, M=64 11008x4096 31.2 / 29.1.  At 128 rows
-// the GEMMs win: INT4 4096x4096 24.3 / 28.2.  Not where a test switch names a GEMM.
-bool f16_mid(int64_t M, int wb, int x_dt) {
-    return x_dt == MCQ4_DTYPE_F16 && M <= 64 && M > (wb == 4 ? 32 : 16) && !mcq4::opt("MCQ4_I4_GEMM6") &&
-           !mcq4::opt("MCQ4_I4_GEMM7");
+// M=33 4096x4096 24.2 / 13.3, M=48 4096x11008 29.7 / 23.2, M=64 4096x14336 30.1 / 27.7;
+// INT8 M=17 4096x4096 25.5 / 12.5, M=64 4096x14336 33.3 / 33.3.  At 128 rows the GEMMs win:
+// INT4 4096x4096 24.3 / 28.2.  Where wx_skinny's own work is the larger:
+//   * more than 16384 columns, 256 of its tiles, a second round of workgroups.  INT4 M=33
+//     256x128256 28.5 / 45.3, 1024x32000 21.3 / 17.9, 1024x65536 30.8 / 35.7; M=48 2048x65536
+//     51.6 / 55.7; M=64 256x32000 10.2 / 16.8, 4096x20480 42.8 / 52.2; from K = 8192 on M=48
+//     8192x20480 66.4 / 75.0, and M=64 8192x32000 106 / 88, the GEMM of 24576 columns being
+//     the 256-row one (i4_gemm7).  INT8 M=32 128x32000 8.0 / 8.8, 4096x32000 54.3 / 49.4,
+//     14336x20480 150 / 174; M=33 4096x65536 158 / 111; M=64 4096x32000 54.3 / 61.9, 4096x65536
+//     163 / 137.
+//   * above 56 rows, long K times wide N: INT4 M=64 8192x16384 49.9 / 43.5, 11008x8192 37.5 /
+//     37.9, 11008x11008 53.2 / 57.5, 14336x14336 67.9 / 75.4; INT8 8192x4096 27.6 / 25.1,
+//     4096x16384 35.7 / 34.3, 8192x8192 35.8 / 37.2, 14336x14336 82.1 / 93.6.
+// Not where a test switch names a GEMM.
+bool f16_mid(int64_t M, int64_t K, int64_t N, int wb, int x_dt) {
+    if (x_dt != MCQ4_DTYPE_F16 || M > 64 || M <= (wb == 4 ? 32 : 16) || mcq4::opt("MCQ4_I4_GEMM6") || mcq4::opt("MCQ4_I4_GEMM7"))
+        return false;
+    if (N > 16384) {
+        if (wb == 4) return K >= 8192 ? N >= 24576 : M <= 48 && K >= (N <= 32768 ? 1024 : 2048);
+        if (M <= 32) return K >= 512 && K <= 12288;
+        return K <= 8192 && (M <= 40 ? K >= 1024 : N >= 65536 && K >= 2048);
+    }
+    if (M <= 56) return true;
+    return wb == 4 ? K <= 8192 || K * N < 96 << 20 : K < 8192 || N < 8192;
 }
 
 // Upper bound over the kernels a shape can take (the general kernel needs none).
@@ -141,7 +159,7 @@ size_t ws_bytes(int64_t M, int64_t K, int64_t N, int64_t gs, int x_dt, int wb = 
 size_t query_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t gs, int x_dt, int wb = 4) {
     const size_t need = ws_bytes(M, K, N, gs, x_dt, wb);
     if (M <= 0 || K <= 0 || N <= 0 || gs <= 0 || gs % 32) return need;
-    if (x_dt == MCQ4_DTYPE_F16 && N % 128 == 0 && K % 32 == 0 && !f16_mid(M, wb, x_dt)) return need;
+    if (x_dt == MCQ4_DTYPE_F16 && N % 128 == 0 && K % 32 == 0 && !f16_mid(M, K, N, wb, x_dt)) return need;
     const size_t wx = mcq4::wx_workspace_bytes(wb == 4 ? mcq4::WX_I4 : mcq4::WX_I8, x_dt, M, K, N);
     if (bf16_prefill(M, K, wb, x_dt) && N % 128 == 0 && K % 32 == 0)
         return std::max({need, wx, mcq4::i4_gemm_bf16_workspace_bytes(M, K, N)});
@@ -194,7 +212,7 @@ int matmul_common(int act, const void *X, int x_dtype, int64_t ldx, const uint8_
     if (!aligned(workspace, 16)) workspace = nullptr;   // optional from here on
     hipStream_t st = (hipStream_t)stream;
     hipError_t e;
-    if (path == I4Path::Gemm && f16_mid(M, wb, x_dtype) && mcq4::wx_supported(wx) &&
+    if (path == I4Path::Gemm && f16_mid(M, K, N, wb, x_dtype) && mcq4::wx_supported(wx) &&
         mcq4::wx_workspace_bytes(wx.wt, x_dtype, M, K, N) <= (workspace ? workspace_bytes : (size_t)0))
         return hip_status(mcq4::launch_wx(wx, workspace, workspace_bytes, st), "int4 matmul launch");
     switch (path) {

@@ -22,14 +22,14 @@ ACT = {None: lambda y: y, "silu": lambda y: y / (1 + np.exp(-y)),
        "gelu": lambda y: 0.5 * y * (1 + np.tanh(np.sqrt(2 / np.pi) * (y + 0.044715 * y ** 3)))}
 
 
-def _check(Y, X, W, xdt, act=None):
+def _check(Y, X, W, xdt, act=None, E=0.0):
     X = X.double().numpy()
     W = np.asarray(W, np.float64)
     y = X @ W
     Yr, S = ACT[act](y), np.abs(X) @ np.abs(W)
     Y = Y.double().cpu().numpy()
     assert np.isfinite(Y).all()
-    bound = ULP[xdt] * np.abs(Yr) + 1.13 * X.shape[1] * 2.0 ** -24 * S + (2.0 ** -20 * np.abs(y) if act else 0) + 1e-30
+    bound = ULP[xdt] * np.abs(Yr) + 1.13 * (X.shape[1] * 2.0 ** -24 * S + E) + (2.0 ** -20 * np.abs(y) if act else 0) + 1e-30
     bad = np.abs(Y - Yr) / bound
     assert bad.max() <= 1, f"err/bound {bad.max():.3g} at {np.unravel_index(bad.argmax(), bad.shape)}"
 
@@ -69,7 +69,7 @@ def test_bf16_prefill(dev, monkeypatch, M, K, N, gs, sdt, env):
 
 
 @pytest.mark.parametrize("M,K,N,gs,act", [(33, 96, 128, 32, None), (33, 4096, 384, 128, "silu"), (48, 2080, 256, 32, "gelu"),
-                                          (64, 4096, 1024, 128, None)])
+                                          (64, 4096, 1024, 128, None), (33, 64, 16384, 32, None)])
 def test_fp16_rows_int4(dev, M, K, N, gs, act):
     import metalops_amd as mo
     print(f"i4 f16 M={M} K={K} N={N} {act}", flush=True)
@@ -78,7 +78,7 @@ def test_fp16_rows_int4(dev, M, K, N, gs, act):
     _check(f(X.to(dev), *args, gs), X, W, R.F16, act)
 
 
-@pytest.mark.parametrize("M,K,N,gs", [(17, 64, 128, 32), (32, 4096, 384, 128), (33, 2080, 256, 32), (64, 4096, 640, 128)])
+@pytest.mark.parametrize("M,K,N,gs", [(17, 64, 128, 32), (32, 4096, 384, 128), (33, 2080, 256, 32), (64, 4096, 640, 128), (17, 512, 16512, 128)])
 def test_fp16_rows_int8(dev, M, K, N, gs):
     import metalops_amd as mo
     print(f"i8 f16 M={M} K={K} N={N}", flush=True)
@@ -90,3 +90,29 @@ def test_fp16_rows_int8(dev, M, K, N, gs):
     X = torch.randn(M, K, generator=torch.Generator().manual_seed(M + K)).half()
     Y = mo.matmul_int8(X.to(dev), torch.from_numpy(q).to(dev), torch.from_numpy(s).half().to(dev), torch.from_numpy(z).half().to(dev), gs)
     _check(Y, X, R.dequantize_int8(q, s, z, gs, R.F16), R.F16)
+
+
+# Beyond 16384 columns at short K, and above 56 rows with long K times wide N, the GEMM tiles
+# take these rows: w = fma(q, s, c) with c = -z s rounded to fp16, so each weight is off W by at
+# most 2^-11 (|z s| + 2 |W|) (c's rounding, the fma's, W's own).  Both sides of the column and K lines.
+@pytest.mark.parametrize("wb,M,K,N,gs,act", [(4, 33, 64, 16512, 32, "silu"), (4, 48, 992, 16512, 32, None), (4, 48, 1024, 16512, 32, None),
+                                             (4, 49, 1024, 16512, 128, None), (4, 64, 64, 24576, 32, "gelu"), (8, 17, 480, 16512, 32, None),
+                                             (8, 33, 992, 16512, 32, None), (8, 40, 1024, 16512, 128, None), (8, 41, 1024, 16512, 128, None)])
+def test_fp16_rows_gemm(dev, wb, M, K, N, gs, act):
+    import metalops_amd as mo
+    print(f"i{wb} f16 GEMM rows M={M} K={K} N={N} {act}", flush=True)
+    rng = np.random.default_rng(M + N)
+    G = -(-K // gs)
+    s = rng.uniform(0.5e-3, 2e-3, (G, N)).astype(np.float16).astype(np.float32)
+    z = rng.uniform(4, 12, (G, N)).astype(np.float16).astype(np.float32)
+    X = torch.randn(M, K, generator=torch.Generator().manual_seed(M + K)).half()
+    if wb == 4:
+        p = rng.integers(0, 256, (K // 2, N), np.uint8)
+        f, W = {None: mo.matmul_int4, "silu": mo.matmul_int4_silu, "gelu": mo.matmul_int4_gelu}[act], R.dequantize(p, s, z, gs, R.F16)
+    else:
+        p = rng.integers(-128, 128, (K, N)).astype(np.int8)
+        f, W = mo.matmul_int8, R.dequantize_int8(p, s, z, gs, R.F16)
+    Y = f(X.to(dev), torch.from_numpy(p).to(dev), torch.from_numpy(s).half().to(dev), torch.from_numpy(z).half().to(dev), gs)
+    zs = np.repeat(np.abs(z * s), gs, axis=0)[:K]
+    E = 2.0 ** -11 * (np.abs(X.float().numpy()) @ (zs + 2 * np.abs(np.asarray(W, np.float32)))).astype(np.float64)
+    _check(Y, X, W, R.F16, act, E)
