@@ -322,14 +322,18 @@ int mcq4_dequantize_q4_0_bf16(const uint8_t *blocks, int64_t K, int64_t N, void 
     return dequantize_common(blocks, K, N, out, ldo, MCQ4_DTYPE_BF16, stream);
 }
 
-// What mcq4_matmul_q4_0_f16 cannot do without.
+// What mcq4_matmul_q4_0_f16 cannot do without: an upper bound over the kernels that a shape
+// can reach, whatever the pointers' alignment.  The wx kernels need none, nor does
+// q4_gemm at the K it is chosen for.
 static size_t required_ws_bytes(int64_t M, int64_t K, int64_t N) {
     if (M <= 0 || K <= 0 || N <= 0 || K % 32) return 0;
-    if (M <= 32) return mcq4::skinny_workspace_bytes(M, K, N);
-    // The largest of the split-K kernels' needs: an upper bound for any prefill kernel.
-    const size_t pre = std::max(mcq4::gemm_workspace_bytes(M, K, N), prefill_ws_bytes(M, K, N));
-    // 33..64 rows run either family, depending on the pointers' alignment.
-    return M <= 64 ? std::max(pre, mcq4::skinny_workspace_bytes(M, K, N)) : pre;
+    size_t need = M <= 64 ? mcq4::skinny_workspace_bytes(M, K, N) : 0;
+    if (M > 64 || (M > 32 && (N > 16384 || decode_switch()))) {
+        if (N % 8 == 0) need = std::max(need, prefill_ws_bytes(M, K, N));
+        const char *path = mcq4::opt("MCQ4_GEMM_PATH");
+        if (path && path[0] == 's') need = std::max(need, mcq4::gemm_workspace_bytes(M, K, N));
+    }
+    return need;
 }
 
 size_t mcq4_matmul_workspace_bytes(int64_t M, int64_t K, int64_t N) {

@@ -72,6 +72,15 @@ def test_workspace_query_and_check():
     assert rc == _lib.MCQ4_ERR_WORKSPACE
 
 
+def test_workspace_of_shapes_without_split_kernels():
+    """Odd widths in prefill, and 33..64 rows that run wx_mid or the strips, require nothing of the kernels
+    that they do not reach: the query fits the allocation-free entry's array."""
+    L = _lib.lib
+    cap = L.mcq4_matmul_noalloc_max_workspace_bytes()
+    for M, K, N in ((100, 4096, 4097), (300, 11008, 4101), (2048, 14336, 4097), (48, 4096, 8192), (64, 14336, 4096)):
+        assert L.mcq4_matmul_workspace_bytes(M, K, N) <= cap
+
+
 def test_quantize_dequant_validation_codes():
     L = _lib.lib
     assert L.mcq4_quantize_q4_0(None, 8, 32, 8, 0x20000, None) == _lib.MCQ4_ERR_INVALID_ARG
