@@ -346,15 +346,14 @@ int mcq4_matmul_int4_gelu(const void *X, int x_dtype, int64_t ldx, const uint8_t
 // max(matmul workspace, 256 KiB) on, so the counter area is never written with
 // activations and one zero-filled buffer keeps serving every entry point.
 constexpr size_t kCounterArea = (size_t)65536 * 4;
-static size_t norm_offset(int64_t M, int64_t K, int64_t N, int64_t gs) {
-    const size_t w = std::max(query_ws_bytes(M, K, N, gs, MCQ4_DTYPE_F16), kCounterArea);
-    return (w + 255) / 256 * 256;
+static size_t norm_offset(size_t matmul_bytes) {
+    return (std::max(matmul_bytes, kCounterArea) + 255) / 256 * 256;
 }
 
 size_t mcq4_fused_rmsnorm_linear_int4_workspace_bytes(int64_t M, int64_t K, int64_t N,
                                                       int64_t group_size) {
     if (M <= 0 || K <= 0 || N <= 0 || group_size <= 0) return 0;
-    return norm_offset(M, K, N, group_size) + (size_t)M * K * 2;
+    return norm_offset(query_ws_bytes(M, K, N, group_size, MCQ4_DTYPE_F16)) + (size_t)M * K * 2;
 }
 
 int mcq4_fused_rmsnorm_linear_int4(const void *X, int64_t ldx, const void *w_norm, float eps,
@@ -371,7 +370,12 @@ int mcq4_fused_rmsnorm_linear_int4(const void *X, int64_t ldx, const void *w_nor
     if (ldx < K) return fail(MCQ4_ERR_SHAPE, "ldx (%lld) < K (%lld)", (long long)ldx, (long long)K);
     if (!aligned(X, 2) || !aligned(w_norm, 2))
         return fail(MCQ4_ERR_ALIGNMENT, "X and w_norm must be 2-byte aligned (fp16)");
-    const size_t need = mcq4_fused_rmsnorm_linear_int4_workspace_bytes(M, K, N, group_size);
+    // Less than the query's size will do, down to what the matmul requires: its optional
+    // part, which only splits K, is then left out.
+    const size_t xn_bytes = (size_t)M * K * 2;
+    size_t offset = norm_offset(query_ws_bytes(M, K, N, group_size, MCQ4_DTYPE_F16));
+    if (workspace_bytes < offset + xn_bytes) offset = norm_offset(ws_bytes(M, K, N, group_size, MCQ4_DTYPE_F16));
+    const size_t need = offset + xn_bytes;
     if (!workspace || workspace_bytes < need)
         return fail(MCQ4_ERR_WORKSPACE, "workspace of %zu bytes required, %zu given", need,
                     workspace ? workspace_bytes : (size_t)0);
@@ -390,7 +394,7 @@ int mcq4_fused_rmsnorm_linear_int4(const void *X, int64_t ldx, const void *w_nor
                                                      (hipStream_t)stream),
                           "fused rmsnorm + int4 launch");
     }
-    _Float16 *xn = (_Float16 *)((char *)workspace + norm_offset(M, K, N, group_size));
+    _Float16 *xn = (_Float16 *)((char *)workspace + offset);
     if (int st = hip_status(mcq4::launch_i4_rmsnorm((const _Float16 *)X, ldx,
                                                     (const _Float16 *)w_norm, eps, (int)M, (int)K,
                                                     xn, K, (hipStream_t)stream),
@@ -398,7 +402,7 @@ int mcq4_fused_rmsnorm_linear_int4(const void *X, int64_t ldx, const void *w_nor
         return st;
     // The matmul validates the rest (scales/zeros, Y, its own workspace share).
     return matmul_common(0, xn, MCQ4_DTYPE_F16, K, packed, scales, zeros, sz_dtype, Y, ldy, M, K,
-                         N, group_size, workspace, norm_offset(M, K, N, group_size), stream);
+                         N, group_size, workspace, offset, stream);
 }
 
 }  // extern "C"

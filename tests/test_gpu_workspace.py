@@ -57,3 +57,43 @@ def test_noalloc_takes_what_needs_no_workspace(dev, M, K, N):
     assert L.mcq4_matmul_q4_0_f16_noalloc(X.data_ptr(), K, b.data_ptr(), Y[1].data_ptr(), N, M, K, N, stream) == _lib.MCQ4_OK
     torch.cuda.synchronize(dev)
     assert torch.equal(Y[0].view(torch.int16), Y[1].view(torch.int16)) and not bool(Y[0].isnan().any())
+
+
+@pytest.mark.parametrize("M,K,N", [(33, 4100, 4096), (1, 4100, 4096), (40, 1030, 1000)])
+def test_fused_rmsnorm_with_the_required_workspace(dev, M, K, N):
+    """The fused RMSNorm + INT4 linear in a buffer that holds the counters and the normalised rows only:
+    the product's optional K split is left out, not the call refused.  fp32 sums in another order: each
+    output within 2^-10 of itself (two fp16 roundings) and 2 K 2^-24 sum|x w|."""
+    from metalops_amd import _lib
+    L = _lib.lib
+    print(f"fused rmsnorm, smaller workspace M={M} K={K} N={N}", flush=True)
+    gs = 128
+    g = torch.Generator().manual_seed(M + N)
+    X, wn = torch.randn(M, K, generator=g).half(), (1 + 0.1 * torch.randn(K, generator=g)).half()
+    P = torch.randint(0, 256, (K // 2, N), dtype=torch.uint8, generator=g)
+    S = (0.002 * torch.rand(-(-K // gs), N, generator=g)).half()
+    Z = (7 + torch.rand(-(-K // gs), N, generator=g)).half()
+    d = [t.to(dev) for t in (X, wn, P, S, Z)]
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    best = int(L.mcq4_fused_rmsnorm_linear_int4_workspace_bytes(M, K, N, gs))
+    least = 256 * 1024 + M * K * 2
+    assert int(L.mcq4_matmul_int4_workspace_bytes(M, K, N, gs, _lib.MCQ4_DTYPE_F16)) == 0 and least < best
+
+    def call(size):
+        ws = torch.zeros(size + 512, dtype=torch.uint8, device=dev)
+        base = -(-ws.data_ptr() // 256) * 256
+        ws[base - ws.data_ptr() + size:] = 0x5A
+        Y = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
+        st = L.mcq4_fused_rmsnorm_linear_int4(d[0].data_ptr(), K, d[1].data_ptr(), 1e-5, d[2].data_ptr(), d[3].data_ptr(), d[4].data_ptr(),
+                                              _lib.MCQ4_DTYPE_F16, Y.data_ptr(), N, M, K, N, gs, base, size, stream)
+        torch.cuda.synchronize(dev)
+        assert bool((ws[base - ws.data_ptr() + size:] == 0x5A).all())
+        return st, Y.double().cpu()
+
+    assert call(least - 16)[0] == _lib.MCQ4_ERR_WORKSPACE
+    (s0, y0), (s1, y1) = call(best), call(least)
+    assert s0 == s1 == _lib.MCQ4_OK
+    xn = (X.float() * torch.rsqrt((X.float() ** 2).mean(1, keepdim=True) + 1e-5) * wn.float()).double().abs()
+    q = torch.stack([P & 15, P >> 4], 1).reshape(K, N).double()
+    w = ((q - Z.double().repeat_interleave(gs, 0)[:K]) * S.double().repeat_interleave(gs, 0)[:K]).abs()
+    assert bool(((y0 - y1).abs() <= 2.0 ** -10 * y0.abs() + 2 * K * 2.0 ** -24 * (xn @ w)).all())
