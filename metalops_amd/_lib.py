@@ -10,6 +10,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "_lib", "libmcq4.so")
+TORCH_EXT_PATH = os.path.join(_HERE, "_lib", "torch_ext_build", "mcq4_torch.so")   # torch_ext.py
 
 MCQ4_OK = 0
 MCQ4_ERR_INVALID_ARG = 1

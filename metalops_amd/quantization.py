@@ -18,7 +18,9 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import os
 import threading
+import warnings
 from typing import List, Optional, Sequence
 
 import torch
@@ -27,11 +29,14 @@ from . import _lib
 
 # The native call path (csrc/torch_ext/mcq4_torch.cpp): checks, output, workspace and
 # launch of a call whose tensors need no conversion, None for any other.  Without the
-# extension every call goes through ctypes to the same kernels.
-try:
+# extension every call goes through ctypes to the same kernels, at twice the host time of a
+# small call, so a missing one is said and one that does not load is an error.
+if os.path.exists(_lib.TORCH_EXT_PATH):
     from .torch_ext import backend as _native
-except ImportError:
+else:
     _native = None
+    warnings.warn(f"metalops_amd: {_lib.TORCH_EXT_PATH} is not built; small calls take twice the host time",
+                  RuntimeWarning)
 
 QK4_0 = 32                         # quantization.py:303
 BLOCK_Q4_0_SIZE = 2 + QK4_0 // 2   # quantization.py:304 (18 bytes)

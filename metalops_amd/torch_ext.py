@@ -17,7 +17,7 @@ import os
 from . import _lib  # loads libmcq4.so first: the extension links against its soname
 
 EXT_NAME = "mcq4_torch"
-EXT_PATH = os.path.join(os.path.dirname(_lib.LIB_PATH), "torch_ext_build", EXT_NAME + ".so")
+EXT_PATH = _lib.TORCH_EXT_PATH
 
 
 def _load():
