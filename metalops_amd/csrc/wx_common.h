@@ -179,6 +179,14 @@ __device__ __forceinline__ void wx_load(WxFly<WT, TN> &r, const WxArgs &a, const
     }
 }
 
+// Orders a wave's LDS accesses before and after it, which other lanes of the wave make to the
+// same bytes: without it only the lane's own addresses keep the compiler from moving one over
+// the other.  The LDS runs a wave's accesses in order, so this is no instruction.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // A step's weights from flight to the lanes of their columns.
 template <int WT, int TN>
 __device__ __forceinline__ WxRaw<WT, TN> wx_ready(const WxFly<WT, TN> &f, uint8_t *scratch, int lane) {
@@ -189,14 +197,17 @@ __device__ __forceinline__ WxRaw<WT, TN> wx_ready(const WxFly<WT, TN> &f, uint8_
         const int lrow = lane & 31, hi = lane >> 5;
         if constexpr (WT == WX_I4) {
             *(uint4_t *)(scratch + 16 * lane + 64 * hi) = f.v[0];
+            wave_lds_order();
 #pragma unroll
             for (int i = 0; i < 8; ++i) r.q[i] = *(const uint16_t *)(scratch + hi * (512 + 64) + 64 * i + 2 * lrow);
         } else {
             *(uint4_t *)(scratch + 16 * lane) = f.v[0];
             *(uint4_t *)(scratch + 1024 + 64 + 16 * lane) = f.v[1];
+            wave_lds_order();
 #pragma unroll
             for (int i = 0; i < 16; ++i) r.q[i] = *(const uint16_t *)(scratch + hi * (1024 + 64) + 64 * i + 2 * lrow);
         }
+        wave_lds_order();                    // the next step stores to the same scratch
 #pragma unroll
         for (int j = 0; j < TN; ++j) { r.s[j] = f.s[j]; r.z[j] = f.z[j]; }
         return r;
