@@ -26,14 +26,20 @@ def _rows_close(Y, Yref, tol=1e-2):
     assert (err <= tol * np.abs(Yref).max(axis=1)).all(), f"max err {err.max()}"
 
 
-def _q4_case(dev, M, K, N):
+def _q4_case(dev, M, K, N, dtype=torch.float16):
     import metalops_amd as mo
     g = torch.Generator().manual_seed(M + K + N)
     W = torch.randn(K, N, generator=g) * 0.02
-    X = torch.randn(M, K, generator=g).half()
+    X = torch.randn(M, K, generator=g).to(dtype)
     blocks = R.quantize_llama_rule(W.numpy())
     b = torch.from_numpy(blocks).to(dev)
-    return (lambda: mo.matmul_ggml_q4_0(X.to(dev), b)), R.matmul_f32(X.numpy(), blocks)
+    if dtype == torch.float16:
+        return (lambda: mo.matmul_ggml_q4_0(X.to(dev), b)), R.matmul_f32(X.numpy(), blocks)
+    return (lambda: mo.matmul_ggml_q4_0(X.to(dev), b)), X.double().numpy() @ R.dequantize(blocks, np.float32).astype(np.float64)
+
+
+def _q4_bf16_case(dev, M, K, N):
+    return _q4_case(dev, M, K, N, torch.bfloat16)
 
 
 def _i4_case(dev, M, K, N, gs, wb):
@@ -78,6 +84,16 @@ CASES = [
     ("q4_gemvm_rows8_s2", {"MCQ4_GEMVM_SPLIT": "2"}, ("q4", 7, 11008, 512)),
     ("q4_gemm6_s2", {"MCQ4_GEMM_PATH": "6", "MCQ4_GEMM6_SPLIT": "2"}, ("q4", 300, 4096, 640)),
     ("q4_gemm8_s2", {"MCQ4_GEMM_PATH": "8"}, ("q4", 300, 4096, 640)),
+    # 17..32 rows (wx_mid.hip), two and eight splits, and the two-row-block strips that its switch keeps.
+    ("q4_mid_s2", {}, ("q4", 24, 4096, 4096)),
+    ("q4_mid_s8", {}, ("q4", 32, 14336, 1024)),
+    ("q4_gemvm_rb2_s2", {"MCQ4_GEMVM_SPLIT": "2"}, ("q4", 32, 14336, 4096)),
+    # bf16: the recompute rounds its weights to bf16 as the kernels do.
+    ("q4_bf16_span_split_s4", {}, ("q4_bf16", 16, 14336, 4096)),
+    ("q4_bf16_span_split_rows8", {}, ("q4_bf16", 6, 11008, 4096)),
+    ("q4_bf16_mid", {}, ("q4_bf16", 24, 4096, 4096)),
+    ("q4_bf16_gemm6_s2", {"MCQ4_GEMM_PATH": "6", "MCQ4_GEMM6_SPLIT": "2"}, ("q4_bf16", 300, 4096, 640)),
+    ("q4_bf16_gemm8_s2", {"MCQ4_GEMM_PATH": "8"}, ("q4_bf16", 300, 4096, 640)),
     # 64-column spans over K splits (q4_gemv_span.hip): 4, 5 and 4 splits, 16, 4 and 8 rows.
     ("q4_span_split_s4", {}, ("q4", 16, 14336, 4096)),
     ("q4_span_split_rows4_s5", {"MCQ4_GEMV_SPAN": "1"}, ("q4", 3, 2080, 2048)),
@@ -101,7 +117,7 @@ def test_split_recompute_path(dev, monkeypatch, name, env, case):
         monkeypatch.delenv(k, raising=False)
     for k, v in env.items():
         monkeypatch.setenv(k, v)
-    build = {"q4": _q4_case, "i4": _i4_case, "rms": _rms_case}[case[0]]
+    build = {"q4": _q4_case, "q4_bf16": _q4_bf16_case, "i4": _i4_case, "rms": _rms_case}[case[0]]
     fn, Yref = build(dev, *case[1:])
     Y = fn()
     torch.cuda.synchronize()
@@ -128,7 +144,10 @@ FLAG_CASES = [
     ("i8_gemv1", ("i4", 4, 4096, 4096, 128, 8)),
     ("q4_span_split_s4", ("q4", 16, 14336, 4096)),
     ("q4_span_split_rows8", ("q4", 6, 11008, 4096)),
-    ("q4_gemvm_rb2_s2", ("q4", 32, 14336, 4096)),
+    ("q4_mid_s4", ("q4", 32, 14336, 4096)),
+    ("q4_bf16_mid", ("q4_bf16", 24, 4096, 4096)),
+    ("q4_bf16_span_split_s4", ("q4_bf16", 16, 14336, 4096)),
+    ("q4_gemvm_rb2_s2", ("q4", 32, 14336, 4096), {"MCQ4_GEMVM_SPLIT": "2"}),
     ("q4_gemvm_s8", ("q4", 12, 2048, 1032), {"MCQ4_GEMVM_SPLIT": "8"}),
 ]
 
@@ -147,7 +166,7 @@ def test_split_flag_timeout_recomputes(dev, monkeypatch, name, case, env):
         monkeypatch.delenv(k, raising=False)
     for k, v in env.items():
         monkeypatch.setenv(k, v)
-    build = {"q4": _q4_case, "i4": _i4_case, "rms": _rms_case}[case[0]]
+    build = {"q4": _q4_case, "q4_bf16": _q4_bf16_case, "i4": _i4_case, "rms": _rms_case}[case[0]]
     fn, Yref = build(dev, *case[1:])
     Y = fn()
     torch.cuda.synchronize()
