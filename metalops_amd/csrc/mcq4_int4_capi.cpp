@@ -125,9 +125,9 @@ bool bf16_prefill(int64_t M, int64_t K, int wb, int x_dt) {
 //     the 256-row one (i4_gemm7).  INT8 M=32 128x32000 8.0 / 8.8, 4096x32000 54.3 / 49.4,
 //     14336x20480 150 / 174; M=33 4096x65536 158 / 111; M=64 4096x32000 54.3 / 61.9, 4096x65536
 //     163 / 137.
-//   * above 56 rows, long K times wide N: INT4 M=64 8192x16384 49.9 / 43.5, 11008x8192 37.5 /
-//     37.9, 11008x11008 53.2 / 57.5, 14336x14336 67.9 / 75.4; INT8 8192x4096 27.6 / 25.1,
-//     4096x16384 35.7 / 34.3, 8192x8192 35.8 / 37.2, 14336x14336 82.1 / 93.6.
+//   * above 56 rows, long K times wide N: INT4 M=64 8192x8192 32.7 / 31.4, 8192x10240 41.4 /
+//     45.0, 11008x11008 53.2 / 57.5, 14336x14336 67.9 / 75.4 (8192x16384 49.9 / 43.5); INT8
+//     14336x4096 34.4 / 34.7, 8192x8192 35.8 / 37.2, 14336x14336 82.1 / 93.6, 28672x5120 83.3 / 99.4.
 // Not where a test switch names a GEMM.
 bool f16_mid(int64_t M, int64_t K, int64_t N, int wb, int x_dt) {
     if (x_dt != MCQ4_DTYPE_F16 || M > 64 || M <= (wb == 4 ? 32 : 16) || mcq4::opt("MCQ4_I4_GEMM6") || mcq4::opt("MCQ4_I4_GEMM7"))
@@ -138,7 +138,7 @@ bool f16_mid(int64_t M, int64_t K, int64_t N, int wb, int x_dt) {
         return K <= 8192 && (M <= 40 ? K >= 1024 : N >= 65536 && K >= 2048);
     }
     if (M <= 56) return true;
-    return wb == 4 ? K <= 8192 || K * N < 96 << 20 : K < 8192 || N < 8192;
+    return K * N < (wb == 4 ? 80 : 64) << 20;
 }
 
 // Upper bound over the kernels a shape can take (the general kernel needs none).
