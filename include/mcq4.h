@@ -85,8 +85,10 @@ int mcq4_dequantize_q4_0_bf16(const uint8_t *blocks, int64_t K, int64_t N, void 
                               void *stream);
 
 /*
- * Workspace bytes mcq4_matmul_q4_0_f16 needs for this shape (0 = none).  The
- * workspace starts with a fixed 256 KiB area of per-tile arrival counters,
+ * Workspace bytes mcq4_matmul_q4_0_f16 makes use of for this shape (0 = none).  A
+ * part of them may be optional (a K split of the kernels for 17..64 rows and for
+ * odd widths): a smaller buffer is refused only where it does not cover what the
+ * shape's kernels require.  The workspace starts with a fixed 256 KiB area of per-tile arrival counters,
  * followed by fp32 split-K partials and, for the kernels whose splits signal
  * each other with per-split flag words, those words (any starting value: each
  * call reads them as it starts and moves each by a fixed step).  The counter
@@ -116,8 +118,8 @@ int mcq4_matmul_q4_0_f16(const void *X, int64_t ldx, const uint8_t *W, void *Y,
  * arguments minus the workspace: the split-K workspace is the library's own
  * device array (one per GPU, held until the process ends) of
  * mcq4_matmul_noalloc_max_workspace_bytes() bytes (256 KiB of counters +
- * 16 MiB: every decode plan, prefill split-K plans up to M = 64 at
- * K = 14336); a shape whose mcq4_matmul_workspace_bytes exceeds it returns
+ * 16 MiB: every plan up to 64 rows and 16384 columns, and for odd widths; the
+ * smaller split-K plans of aligned prefill); a shape that requires more returns
  * MCQ4_ERR_WORKSPACE.  Calls allocate nothing (no hipMalloc / hipFree, no
  * allocating library routine).  Every call on a GPU shares that GPU's array:
  * calls that overlap on one GPU (two streams, two threads) race and give wrong
@@ -232,12 +234,12 @@ size_t mcq4_matmul_int4_best_workspace_bytes(int64_t M, int64_t K, int64_t N, in
  * matmul_int4 (quantization.py:156-239; Metal binding matmul_int4_metal,
  * native/core_mps.mm:5612-5776): Y[M][ldy] = X[M][ldx] @ dequant(W) with
  * fp32 accumulation; X and Y in x_dtype (F16, BF16 or F32).  fp16 activations
- * with group_size % 32 == 0, K % 32 == 0 and N % 8 == 0 run the MFMA kernels
+ * with group_size % 32 == 0, K % 32 == 0 and N % 8 == 0 run the fp16 kernels
  * (decode GEMV for M <= 16, and for M <= 32 with N % 128 == 0 and 16-byte
- * aligned operands; prefill GEMM above); every other case runs a
- * general fp32 kernel.  X needs x_dtype alignment (16 bytes and ldx % 8 == 0
- * for the MFMA kernels; the general kernel is used otherwise), Y x_dtype
- * alignment; ldx >= K, ldy >= N.
+ * aligned operands; prefill GEMM above); other dtypes, widths and alignments with
+ * group_size % 32 == 0 and N >= 16 run MFMA kernels of x_dtype, the weight rounded
+ * to it; everything else a general fp32 kernel.  X and Y need x_dtype alignment;
+ * ldx >= K, ldy >= N.
  */
 int mcq4_matmul_int4(const void *X, int x_dtype, int64_t ldx, const uint8_t *packed,
                      const void *scales, const void *zeros, int sz_dtype, void *Y, int64_t ldy,
@@ -303,7 +305,9 @@ size_t mcq4_fused_rmsnorm_linear_int4_workspace_bytes(int64_t M, int64_t K, int6
  * GEMV takes: one launch that normalises inside the GEMV.  Otherwise X_norm is
  * written to the workspace behind the matmul's share (workspace 256-byte
  * aligned), then the INT4 matmul runs on the same stream.  Both forms give the
- * same bits.
+ * same bits.  A workspace smaller than the query's size is taken down to what the
+ * matmul requires (mcq4_matmul_int4_workspace_bytes for fp16, at least 256 KiB) plus
+ * 2 M K bytes; the matmul's optional K split is then left out.
  */
 int mcq4_fused_rmsnorm_linear_int4(const void *X, int64_t ldx, const void *w_norm, float eps,
                                    const uint8_t *packed, const void *scales, const void *zeros,

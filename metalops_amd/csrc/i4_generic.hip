@@ -1,6 +1,7 @@
 // General per-group INT4 / INT8 matmul: any activation dtype (fp32 / fp16 /
 // bf16), any group size, any N, even K (INT4).  This is the path for what the
-// MFMA kernels do not take: group sizes that are no multiple of 32, N = 1.
+// MFMA kernels do not take: group sizes that are no multiple of 32, N < 16,
+// fused activations outside INT4 x fp16.
 //
 // Semantics follow quantization.py:207-239 (INT4) and :268-286 (INT8): the
 // weight is dequantized as ((float)q - zero) * scale in fp32 and rounded to X's

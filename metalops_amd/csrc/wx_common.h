@@ -1,7 +1,7 @@
 // Shared parts of the any-activation matmul kernels (wx_gemm, wx_skinny):
 // quantized weights (block_q4_0, per-group INT4, per-group INT8) times fp16, bf16
-// or fp32 activations, any column count, any 2-byte (q4_0) or byte (INT4, INT8)
-// alignment of the weights.
+// or fp32 activations, any column count (INT4, INT8: 16 or more, groups of whole K
+// steps), any 2-byte (q4_0) or byte (INT4, INT8) alignment of the weights.
 //
 // Semantics (quantization.py:207-239, :268-286, :452-454): the weight is
 // dequantized in fp32 and rounded once to the activations' dtype, then

@@ -26,7 +26,7 @@
 //
 // Measured: INT4 x bf16 M = 256 4096x11008 60.9 us (one thread per column: 8165), INT4 x
 // fp32 243.2, q4_0 x fp16 M = 300 11008x4101 83.9.  INT4 in 16 bits is bound by waits
-// (counters: MFMA busy 15 %, 43 % of the wave cycles waiting, LDS conflicts 28 % of the
+// (counters: MFMA busy 15 %, 44 % of the wave cycles waiting, LDS conflicts 28 % of the
 // LDS cycles); fp32 by the fp32 MFMA, whose library rate is 153 TFLOP/s here (95 at M =
 // 256, 108 at 512x4096x4096).  Operands prepared one step ahead of their MFMAs: 61.5 us.
 #include <algorithm>

@@ -62,15 +62,11 @@ DT = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
 
 
 # Every entry; rows of decode, the kernels between and prefill; shapes with and without a K split.
-@pytest.mark.parametrize("op", ["q4", "group", "i4", "i4_3d", "silu", "gelu", "i8", "rms"])
-@pytest.mark.parametrize("x", ["f16", "bf16", "f32"])
-@pytest.mark.parametrize("M", [1, 7, 40, 130])
+# (silu, gelu and rms are fp16 entries, group takes one fp16 row.)
+@pytest.mark.parametrize("op,x,M", [(op, x, M) for op in ("q4", "i4", "i4_3d", "i8") for x in ("f16", "bf16", "f32") for M in (1, 7, 40, 130)]
+                         + [(op, "f16", M) for op in ("silu", "gelu", "rms") for M in (1, 7, 40, 130)] + [("group", "f16", 1)])
 def test_equals_ctypes_path(dev, monkeypatch, op, x, M):
     import metalops_amd as mo
-    if x != "f16" and op in ("group", "silu", "gelu", "rms"):
-        pytest.skip("fp16 entries")
-    if op == "group" and M > 1:
-        pytest.skip("one row")
     print(f"native {op} {x} M={M}", flush=True)
     g = torch.Generator(device=dev).manual_seed(M)
     K, N = 4096, 1040
