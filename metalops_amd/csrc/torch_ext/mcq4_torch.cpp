@@ -11,7 +11,9 @@
 // int4_matmul, int8_matmul, int4_rmsnorm below): the checks, the output, the
 // workspace and the launch of a call whose tensors need no conversion.  Anything
 // else -- other types, strides, alignments, empty shapes, an error -- returns None,
-// and the Python function goes its own way (and raises what it raises).  A
+// and the Python function goes its own way: it raises what it raises, or converts the
+// tensors and calls again (through ctypes from there, 1024x1024 INT4 with strided
+// activations took 24.9 us a call, 16.8 so).  A
 // decode call of a 4.3 us kernel took 11.5 us of host time through ctypes.
 #include <string>
 #include <torch/extension.h>

@@ -218,24 +218,27 @@ def _matmul(X, W_packed, scales, zeros, group_size, act):
     M = x.shape[0]
     s, z = _sz_pair(scales, zeros)
     p = _dense(W_packed, 16)
-    Y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    if M and N:
-        if K == 0:
-            Y.zero_()
-        else:
-            xdt = _DT[x.dtype]
-            need = int(_lib.lib.mcq4_matmul_int4_best_workspace_bytes(M, K, N, group_size, xdt))
-            stream = _stream(x.device)
-            ws, ws_ptr, ws_bytes = None, None, 0
-            if need:
-                ws = _workspace.get(x.device, stream, need)
-                ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
-            fn = getattr(_lib.lib, _FN[act])
-            with torch.cuda.device(x.device), _workspace.guard(ws, stream):
-                _lib.check(fn(x.data_ptr(), xdt, x.stride(0), p.data_ptr(), s.data_ptr(),
-                              z.data_ptr(), _DT[s.dtype], Y.data_ptr(), N, M, K, N, group_size,
-                              ws_ptr, ws_bytes, stream),
-                           _FN[act])
+    # Converted, the tensors are what the native path takes.
+    Y = _native.int4_matmul(x, p, s, z, group_size, act) if _native is not None else None
+    if Y is None:
+        Y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        if M and N:
+            if K == 0:
+                Y.zero_()
+            else:
+                xdt = _DT[x.dtype]
+                need = int(_lib.lib.mcq4_matmul_int4_best_workspace_bytes(M, K, N, group_size, xdt))
+                stream = _stream(x.device)
+                ws, ws_ptr, ws_bytes = None, None, 0
+                if need:
+                    ws = _workspace.get(x.device, stream, need)
+                    ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+                fn = getattr(_lib.lib, _FN[act])
+                with torch.cuda.device(x.device), _workspace.guard(ws, stream):
+                    _lib.check(fn(x.data_ptr(), xdt, x.stride(0), p.data_ptr(), s.data_ptr(),
+                                  z.data_ptr(), _DT[s.dtype], Y.data_ptr(), N, M, K, N, group_size,
+                                  ws_ptr, ws_bytes, stream),
+                               _FN[act])
     Y = Y if Y.dtype == out_dtype else Y.to(out_dtype)
     return Y.reshape(*lead, N) if batched else Y
 
@@ -356,24 +359,26 @@ def matmul_int8(
     M = x.shape[0]
     s, z = _sz_pair(scales, zeros)
     w = _dense(W_packed.view(torch.int8), 16)
-    Y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    if M and N:
-        if K == 0:
-            Y.zero_()
-        else:
-            xdt = _DT[x.dtype]
-            need = int(_lib.lib.mcq4_matmul_int8_best_workspace_bytes(M, K, N, group_size, xdt))
-            stream = _stream(x.device)
-            ws, ws_ptr, ws_bytes = None, None, 0
-            if need:
-                ws = _workspace.get(x.device, stream, need)
-                ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
-            with torch.cuda.device(x.device), _workspace.guard(ws, stream):
-                _lib.check(_lib.lib.mcq4_matmul_int8(x.data_ptr(), xdt, x.stride(0), w.data_ptr(),
-                                                     s.data_ptr(), z.data_ptr(), _DT[s.dtype],
-                                                     Y.data_ptr(), N, M, K, N, group_size, ws_ptr,
-                                                     ws_bytes, stream),
-                           "mcq4_matmul_int8")
+    Y = _native.int8_matmul(x, w, s, z, group_size, 0) if _native is not None else None   # converted
+    if Y is None:
+        Y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        if M and N:
+            if K == 0:
+                Y.zero_()
+            else:
+                xdt = _DT[x.dtype]
+                need = int(_lib.lib.mcq4_matmul_int8_best_workspace_bytes(M, K, N, group_size, xdt))
+                stream = _stream(x.device)
+                ws, ws_ptr, ws_bytes = None, None, 0
+                if need:
+                    ws = _workspace.get(x.device, stream, need)
+                    ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+                with torch.cuda.device(x.device), _workspace.guard(ws, stream):
+                    _lib.check(_lib.lib.mcq4_matmul_int8(x.data_ptr(), xdt, x.stride(0), w.data_ptr(),
+                                                         s.data_ptr(), z.data_ptr(), _DT[s.dtype],
+                                                         Y.data_ptr(), N, M, K, N, group_size, ws_ptr,
+                                                         ws_bytes, stream),
+                               "mcq4_matmul_int8")
     return Y if Y.dtype == out_dtype else Y.to(out_dtype)
 
 

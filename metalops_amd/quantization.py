@@ -233,40 +233,30 @@ def matmul_ggml_q4_0(X: torch.Tensor, W_blocks: torch.Tensor) -> torch.Tensor:
     w = W_blocks if W_blocks.is_contiguous() else W_blocks.contiguous()
     if w.data_ptr() % 2:
         w = w.clone()
-    Y = torch.empty((M, N), dtype=X.dtype, device=X.device)
-    if M == 0 or N == 0:
-        return Y
-    if K == 0:
-        return Y.zero_()
-    stream = _stream(X.device)
-    if X.dtype != torch.float16:
-        x = X if (X.stride(1) == 1 and X.stride(0) >= K) else X.contiguous()
-        code = _DTYPE_CODES[x.dtype]
-        need = int(_lib.lib.mcq4_matmul_q4_0_workspace_bytes(M, K, N, code))
-        ws, ws_ptr, ws_bytes = None, None, 0
-        if need:
-            ws = _workspace.get(x.device, stream, need)
-            ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
-        with torch.cuda.device(x.device), _workspace.guard(ws, stream):
-            _lib.check(_lib.lib.mcq4_matmul_q4_0(x.data_ptr(), code, x.stride(0), w.data_ptr(), Y.data_ptr(), N, M, K,
-                                                 N, ws_ptr, ws_bytes, stream),
-                       "mcq4_matmul_q4_0")
-        return Y
+    if M == 0 or N == 0 or K == 0:
+        return torch.zeros((M, N), dtype=X.dtype, device=X.device)
     x = X
-    if x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < K or x.data_ptr() % 16:
+    f16 = X.dtype == torch.float16
+    if x.stride(1) != 1 or x.stride(0) < K or (f16 and (x.stride(0) % 8 or x.data_ptr() % 16)):
         x = x.contiguous()
-        if x.data_ptr() % 16:
+        if f16 and x.data_ptr() % 16:
             x = x.clone()
-    need = int(_lib.lib.mcq4_matmul_workspace_bytes(M, K, N))
+    if _native is not None and (x is not X or w is not W_blocks):   # converted: what the native path takes
+        Y = _native.q4_matmul(x, w)
+        if Y is not None:
+            return Y
+    Y = torch.empty((M, N), dtype=X.dtype, device=X.device)
+    stream = _stream(X.device)
+    code = _DTYPE_CODES[x.dtype]
+    need = int(_lib.lib.mcq4_matmul_q4_0_workspace_bytes(M, K, N, code))
     ws, ws_ptr, ws_bytes = None, None, 0
     if need:
         ws = _workspace.get(x.device, stream, need)
         ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
     with torch.cuda.device(x.device), _workspace.guard(ws, stream):
-        _lib.check(_lib.lib.mcq4_matmul_q4_0_f16(x.data_ptr(), x.stride(0), w.data_ptr(),
-                                                 Y.data_ptr(), N, M, K, N, ws_ptr, ws_bytes,
-                                                 stream),
-                   "mcq4_matmul_q4_0_f16")
+        _lib.check(_lib.lib.mcq4_matmul_q4_0(x.data_ptr(), code, x.stride(0), w.data_ptr(), Y.data_ptr(), N, M, K, N,
+                                             ws_ptr, ws_bytes, stream),
+                   "mcq4_matmul_q4_0_f16" if f16 else "mcq4_matmul_q4_0")
     return Y
 
 
