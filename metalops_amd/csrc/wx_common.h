@@ -187,27 +187,35 @@ __device__ __forceinline__ void wave_lds_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// A step's weights from flight to the lanes of their columns.
-template <int WT, int TN>
+// A step's weights from flight to the lanes of their columns.  What keeps the compiler from
+// moving the loads over the stores of their step or the next: the fence (FENCE), or a load
+// address that it can't see through, so that each load may be to the bytes of any store.
+// Against code with neither: the fence costs wx_skinny nothing (class means within 0.1 %)
+// and wx_gemm up to 2.5 % (INT4 bf16 1755x1632x5248 74.3 -> 76.2 us), since it holds back the
+// kernel's other LDS work too; the address leaves wx_gemm's class means at 0.992 to 1.001
+// (that call 73.1 -> 73.3, most INT8 fp16 calls up to 3 % faster, the worst 300x4100x1025
+// 44.1 -> 45.0) and costs wx_skinny up to 3.4 % (INT4 fp16 2x4100x14336 46.4 -> 48.0).
+template <int WT, int TN, bool FENCE>
 __device__ __forceinline__ WxRaw<WT, TN> wx_ready(const WxFly<WT, TN> &f, uint8_t *scratch, int lane) {
     if constexpr (WT == WX_Q4) {
         return f;
     } else {
         WxRaw<WT, TN> r;
         const int lrow = lane & 31, hi = lane >> 5;
+        constexpr int HALF = WT == WX_I4 ? 512 + 64 : 1024 + 64, ROWS = WT == WX_I4 ? 8 : 16;
+        uint32_t in_addr = lds_addr(scratch) + (uint32_t)(hi * HALF + 2 * lrow);
+        if constexpr (!FENCE) asm("" : "+v"(in_addr));   // not volatile: one value for all steps
+        const lds_u8 *const in = lds_ptr(in_addr);
         if constexpr (WT == WX_I4) {
             *(uint4_t *)(scratch + 16 * lane + 64 * hi) = f.v[0];
-            wave_lds_order();
-#pragma unroll
-            for (int i = 0; i < 8; ++i) r.q[i] = *(const uint16_t *)(scratch + hi * (512 + 64) + 64 * i + 2 * lrow);
         } else {
             *(uint4_t *)(scratch + 16 * lane) = f.v[0];
             *(uint4_t *)(scratch + 1024 + 64 + 16 * lane) = f.v[1];
-            wave_lds_order();
-#pragma unroll
-            for (int i = 0; i < 16; ++i) r.q[i] = *(const uint16_t *)(scratch + hi * (1024 + 64) + 64 * i + 2 * lrow);
         }
-        wave_lds_order();                    // the next step stores to the same scratch
+        if constexpr (FENCE) wave_lds_order();
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) r.q[i] = *(const lds_u16 *)(in + 64 * i);
+        if constexpr (FENCE) wave_lds_order();           // the next step stores to the same scratch
 #pragma unroll
         for (int j = 0; j < TN; ++j) { r.s[j] = f.s[j]; r.z[j] = f.z[j]; }
         return r;

@@ -109,7 +109,7 @@ __global__ void __launch_bounds__(512, 2) wx_gemm_kernel(WxArgs a) {
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
     auto step = [&](int slot, int t, int u, const WxFly<WT, WG_TN> &f) {
-        const WxRaw<WT, WG_TN> r = wx_ready<WT, WG_TN>(f, scratch, lane);
+        const WxRaw<WT, WG_TN> r = wx_ready<WT, WG_TN, false>(f, scratch, lane);
         const int valid = a.K - (k_lo + kstep(u)) * 32 - 16 * lhi;
         const uint16_t *d = nullptr;
         if constexpr (WT == WX_Q4) d = r.d;

@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(WS_NW * 64) wx_skinny_kernel(WxArgs a) {
 #pragma unroll
                 for (int ks = 0; ks < 2; ++ks) p.x[i][ks] = wx_order<WT>(p.x[i][ks]);
         }
-        const WxRaw<WT, TN> raw = wx_ready<WT, TN>(p.r, scratch, lane);
+        const WxRaw<WT, TN> raw = wx_ready<WT, TN, true>(p.r, scratch, lane);
         const uint16_t *d = nullptr;
         if constexpr (WT == WX_Q4) d = raw.d;
         wx_if_finite<WT, XT, TN>(d, [&](auto fin) {
