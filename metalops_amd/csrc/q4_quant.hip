@@ -221,12 +221,19 @@ hipError_t launch_quantize(bool llama_rule, const float *W, int64_t ldw, int nb,
     return hipGetLastError();
 }
 
-// fp32 out: four columns per thread above 8 M weights, unless more than a sixteenth of
-// the last workgroup's threads in a row would be idle; one column otherwise.  us on fresh
-// blocks, one / four: 4096x4096 17.0 / 13.4, 2048x8192 16.2 / 13.0, 14336x14336 180 / 180,
-// 4096x2048 8.1 / 8.0; 1024x1024 2.9 / 3.8, 8192x1536 10.2 / 11.5.
+// fp32 out: four columns per thread above 8 M weights if the threads that a row leaves idle
+// are at most a sixteenth of N, above 11 M if they are at most a third of those launched; one
+// column otherwise.  us on fresh blocks, one / four, none idle: 4096x4096 17.0 / 13.4,
+// 2048x8192 16.2 / 13.0, 14336x14336 180 / 180, 4096x2048 8.1 / 8.0, 1024x1024 2.9 / 3.8.
+// A third and less: 6816x2312 18.8 / 13.0, 6816x4104 29.4 / 23.5, 14336x2056 30.9 / 24.1,
+// 3200x6400 19.3 / 15.7, 14336x2304 29.0 / 28.6, the worst 4096x3088 10.9 / 12.5; below 11 M
+// 3200x3336 9.7 / 10.4, 1600x5376 8.2 / 8.9, the worst 1600x4104 7.5 / 6.7.  More:
+// 14336x1064 16.1 / 19.2.  Over 172 shapes of 4 M to 57 M weights the line's mean time is
+// 0.5 % above the better kernel's; that of one column alone 7.2 %, of four alone 3.3 %.
+// On blocks that the last-level cache still holds: 2.5, 1.2 and 5.1 % (8192x1536 10.0 / 11.4).
 static bool dequant_wide_f32(int nb, int N) {
-    return (int64_t)nb * QK * N > ((int64_t)1 << 23) && (N + 1023) / 1024 * 1024 - N <= N / 16;
+    const int64_t weights = (int64_t)nb * QK * N, launched = ((int64_t)N + 1023) / 1024 * 1024, idle = launched - N;
+    return (weights > (int64_t)8 << 20 && 16 * idle <= N) || (weights > (int64_t)11 << 20 && 3 * idle <= launched);
 }
 
 template <int DT>

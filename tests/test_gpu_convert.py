@@ -102,9 +102,11 @@ def test_q4_rule_on_specials(dev, dtype, std, N):
 
 
 # Widths around two and four columns per thread, row strides and addresses that leave them, and the
-# fp32 sizes (above 8 M weights) on both sides of the idle-thread line.
+# fp32 sizes (above 8 M and 11 M weights) on both sides of the idle-thread lines.
 @pytest.mark.parametrize("K,N,pad,off", [(64, 2, 0, 0), (64, 510, 1, 0), (96, 514, 2, 1), (32, 1023, 0, 0), (64, 1026, 0, 2),
-                                         (64, 260, 4, 0), (8224, 1024, 0, 0), (5504, 1536, 0, 0), (8224, 1024, 0, 1)])
+                                         (64, 260, 4, 0), (8224, 1024, 0, 0), (5504, 1536, 0, 0), (8224, 1024, 0, 1),
+                                         (4704, 1792, 0, 0), (5664, 2056, 0, 0), (5664, 2044, 0, 0), (8480, 1364, 0, 0),
+                                         (8480, 1368, 0, 0)])
 def test_q4_dequantize_layouts(dev, K, N, pad, off):
     """dequantize through the C entry: padded rows and an `out` at an odd element."""
     from metalops_amd import _lib
